@@ -200,7 +200,8 @@ __global__ __launch_bounds__(kBatchBlock) __attribute__((amdgpu_waves_per_eu(
                 // the choice is uniform over the wave, so the segment loop does not diverge)
                 const bool stored = ds != nullptr && __all(n <= B.dsCap);
                 march_reverse<FILTER, TFM, BLEND, K, GM, SinkTiled<TFM>, true, VS>(VV, T, r, n, adj_acc, ck,
-                                                                                   kBatchBlock, B.ckCap, B.ckEvery,
+                                                                                   kBatchBlock, B.ckCap,
+                                                                                   __builtin_ctz(K * B.ckEvery),
                                                                                    sink, curWantTf,
                                                          wantVol, wantCam, vs,
                                                          adj_start, adj_dir, adj_step, stored ? ds : nullptr,

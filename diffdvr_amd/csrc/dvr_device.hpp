@@ -674,6 +674,18 @@ __device__ __forceinline__ void blend_adjoint_ak(float t_in, const f4& s, float 
     adj_acc.w = adj_acc.w * keep - alpha * dotc;
 }
 
+// The adjoint's (alpha, keep) of a sample from those of alpha_keep: the same for
+// Beer-Lambert, clamped below one for alpha blending.
+template <int BLEND>
+__device__ __forceinline__ void adjoint_alpha_keep(float absorption, float step, float& alpha, float keep, float& keepA)
+{
+    keepA = keep;
+    if constexpr (BLEND != 0) {
+        alpha = tmin_(1.0f - 1e-5f, absorption * step);
+        keepA = 1.0f - alpha;
+    }
+}
+
 template <int BLEND>
 __device__ __forceinline__ void blend_adjoint_t(float t_in, const f4& s, float step, f4& adj_acc, f4& adj_s,
                                                 float& adj_step)

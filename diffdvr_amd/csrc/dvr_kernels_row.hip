@@ -1,0 +1,124 @@
+// Row kernels (16 lanes a ray, dvr_row_impl.hpp): launchers.
+#include "dvr_row_impl.hpp"
+
+namespace dvr {
+
+// At most 2^20 tiles of 1024 threads: a launch holds less than 2^32 threads.
+constexpr int kMaxRowTiles = 1 << 20;
+
+// samples per voxel edge and voxel edges per pixel, both averaged over the axes;
+// a per-ray step or a box in device memory counts as the usual half voxel / unit box
+static float step_voxels(const RenderParams& P)
+{
+    if (P.st || P.bsize) return 0.5f;
+    const float n[3] = {float(P.X - 1), float(P.Y - 1), float(P.Z - 1)};
+    float v = 0.0f;
+    for (int a = 0; a < 3; ++a) v += P.stU * n[a] / (3.0f * P.bsizeU[a]);
+    return v;
+}
+static float pixel_voxels(const RenderParams& P)
+{
+    return float(P.X + P.Y + P.Z) / (3.0f * float(P.W < P.H ? P.W : P.H));
+}
+
+// Few rays leave the tiled kernel's chain of samples exposed: up to 768 tiles the row kernel wins
+// at every size measured (576 tiles: 35 against 84 us through 64^3, 142 against 221 us through
+// 128^3 at quarter-voxel steps).  Beyond, it pays by what the gathers touch: with
+// g = (voxels per pixel) x (voxels per step), 64 neighbouring rays reach further apart than 16
+// consecutive samples where g is large.  Measured, row against tiled, in us: g = 0.125, 64^3,
+// 2048 tiles 101 / 127, 4096 tiles 136 / 124; g = 0.25, 128^3, 4096 tiles 218 / 270, 8192 tiles
+// 411 / 307; g = 0.5, 256^3, 8192 tiles 785 / 1313, 32768 tiles 2824 / 3341; g = 0.44 and 0.6
+// with 160^3 (nearer the 4 MiB L2s), 16384 and 32768 tiles 715 / 669, 1031 / 940; g = 0.35,
+// 256^3, 32768 tiles 2150 / 1896.  A nearest-neighbour sample gathers one voxel, not eight, and
+// has nothing to gain from the last two rules.
+bool use_row_forward(const RenderParams& P, int filter)
+{
+    const int tiles = tiled_num_tiles(P);
+    if (tiles <= 768) return true;
+    if (filter != 1 || tiles > kMaxRowTiles) return false;
+    const float g = step_voxels(P) * pixel_voxels(P);
+    if (g >= 0.45f && size_t(P.X) * P.Y * P.Z >= (size_t(6) << 20)) return true;
+    return tiles <= (g >= 0.22f ? 4096 : (g >= 0.11f ? 2048 : 0));
+}
+
+// Position gradients alone (row_reverse): 583 against 931 us at 8192 tiles (Gaussian TF, 4 rows),
+// 903 / 925 at 16384 (identity TF), 1899 / 1594 at 32768; with steps below 0.4 voxel 4290 / 5011 at
+// 32768.  Volume gradients (split_reverse): 347 / 917 us at 1024 tiles, 634 / 1038 at 2048,
+// 2707 / 2684 at 4096.  TF gradients: 161 / 279 and 141 / 199 us at 1024 tiles, 265 / 247 at 2048;
+// the identity TF's walk is short, 53 / 65 at 576 and 83 / 67 at 1024.
+bool use_row_adjoint(const RenderParams& P, const AdjointParams& A, int tfm)
+{
+    const int tiles = tiled_num_tiles(P);
+    if (tiles > kMaxRowTiles) return false;
+    if (A.avol) return tiles <= 2048;
+    if (A.atf) return tiles <= (tfm == 0 && !A.ars && !A.ast ? 768 : 1024);
+    return tiles <= 16384 || step_voxels(P) < 0.4f;
+}
+
+template <int FILTER, int TFM, int BLEND>
+static hipError_t fwd_row_t(const RenderParams& P, const CkptParams& CK, hipStream_t s)
+{
+    const int tilesX = (P.W + kTileW - 1) / kTileW, tilesY = (P.H + kTileH - 1) / kTileH;
+    const int nTiles = tilesX * tilesY * P.B;
+    if (nTiles == 0) return hipSuccess;
+    const size_t lds = sizeof(float) * size_t(P.R) * P.C;
+    hipLaunchKernelGGL((k_forward_row<FILTER, TFM, BLEND>), dim3(nTiles * row_blocks_per_tile(kRowBlock)),
+                       dim3(kRowBlock), lds, s, P, CK, tilesX, tilesX * tilesY, nTiles);
+    return hipGetLastError();
+}
+
+hipError_t launch_forward_row(const RenderParams& P, const CkptParams& CK, int filter, int tfm, int blend, hipStream_t s)
+{
+    DVR_DISPATCH3(filter, tfm, blend, return fwd_row_t, (P, CK, s));
+    return hipErrorInvalidValue;
+}
+
+template <int FILTER, int TFM, int BLEND, int GM>
+static hipError_t adj_row_g(const RenderParams& P, const AdjointParams& A, const CkptParams& CK, const LossParams& L,
+                            bool fused, bool ckFromFwd, hipStream_t s)
+{
+    const int tilesX = (P.W + kTileW - 1) / kTileW, tilesY = (P.H + kTileH - 1) / kTileH;
+    const int nTiles = tilesX * tilesY * P.B;
+    if (nTiles == 0) return hipSuccess;
+    const int RC = P.R * P.C;
+    constexpr int kThreads = kRowAdjBlock;
+    const bool usePriv = TFM == 3 && A.atf && RC <= 48;  // private slices <= 48 KiB of LDS
+    const int stride = RC | 1;                           // odd: the copies start in different LDS banks
+    const int copyStride = size_t(kTfCopies) * stride * sizeof(float) <= 16384 ? stride : 0;
+    const int ng = A.atf ? (usePriv ? RC * kThreads : (copyStride > 0 ? kTfCopies * copyStride : RC)) : 0;
+    int aggLog2 = kAggLog2;
+    size_t lds = sizeof(float) * (size_t(RC) + size_t(ng));
+    if ((GM & 2) && A.avol) {
+        // the largest chunk table per wave beside the TF tables that leaves room for sixteen waves per CU
+        const size_t base = sizeof(float) * size_t(agg_offset(RC, ng));
+        constexpr size_t kWaves = kThreads / 64;
+        while (aggLog2 > kAggMinLog2 && base + kWaves * agg_bytes(aggLog2) > size_t(kLdsPerCu) * kWaves / kTiledVolWgPerCu)
+            --aggLog2;
+        lds = base + kWaves * agg_bytes(aggLog2);
+    }
+    hipLaunchKernelGGL((k_adjoint_row<FILTER, TFM, BLEND, GM>), dim3(nTiles * row_blocks_per_tile(kThreads)),
+                       dim3(kThreads), lds, s, P, A, CK, L, fused ? 1 : 0, ckFromFwd ? 1 : 0, usePriv ? 1 : 0, copyStride,
+                       tilesX, tilesX * tilesY, nTiles, aggLog2);
+    return hipGetLastError();
+}
+
+template <int FILTER, int TFM, int BLEND>
+static hipError_t adj_row_t(const RenderParams& P, const AdjointParams& A, const CkptParams& CK, const LossParams& L,
+                            bool fused, bool ckFromFwd, hipStream_t s)
+{
+    const bool pos = A.ars || A.ast;
+    if (pos && A.avol) return adj_row_g<FILTER, TFM, BLEND, 7>(P, A, CK, L, fused, ckFromFwd, s);
+    if (pos && A.atf) return adj_row_g<FILTER, TFM, BLEND, 5>(P, A, CK, L, fused, ckFromFwd, s);
+    if (pos) return adj_row_g<FILTER, TFM, BLEND, 4>(P, A, CK, L, fused, ckFromFwd, s);
+    if (A.avol) return adj_row_g<FILTER, TFM, BLEND, 3>(P, A, CK, L, fused, ckFromFwd, s);
+    return adj_row_g<FILTER, TFM, BLEND, 1>(P, A, CK, L, fused, ckFromFwd, s);
+}
+
+hipError_t launch_adjoint_row(const RenderParams& P, const AdjointParams& A, const CkptParams& CK, const LossParams& L,
+                              bool fused, bool ckFromFwd, int filter, int tfm, int blend, hipStream_t s)
+{
+    DVR_DISPATCH3(filter, tfm, blend, return adj_row_t, (P, A, CK, L, fused, ckFromFwd, s));
+    return hipErrorInvalidValue;
+}
+
+}  // namespace dvr

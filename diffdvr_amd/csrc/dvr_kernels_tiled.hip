@@ -43,6 +43,7 @@ static hipError_t fwd_tiled_t(const RenderParams& P, const CkptParams& CK, hipSt
 hipError_t launch_forward_tiled(const RenderParams& P, const CkptParams& CK, int filter, int tfm, int blend,
                                 hipStream_t s)
 {
+    if (use_row_forward(P, filter)) return launch_forward_row(P, CK, filter, tfm, blend, s);
     DVR_DISPATCH3(filter, tfm, blend, return fwd_tiled_t, (P, CK, s));
     return hipErrorInvalidValue;
 }
@@ -52,6 +53,8 @@ hipError_t launch_adjoint_tiled(const RenderParams& P, const AdjointParams& A, c
                                 hipStream_t s)
 {
     if (filter < 0 || filter > 1 || blend < 0 || blend > 1) return hipErrorInvalidValue;
+    if (use_row_adjoint(P, A, tfm))
+        return launch_adjoint_row(P, A, CK, L, fused, ckFromFwd, filter, tfm, blend, s);
 #define DVR_CALL(F, B, K) return adj_tiled_inst_##F##_##B##_##K(P, A, CK, L, fused, ckFromFwd, tfm, s)
 #define DVR_SEL_K(F, B)                      \
     switch (CK.K) {                          \

@@ -49,7 +49,7 @@ hipError_t launch_adjoint_plain(const RenderParams& P, const AdjointParams& A, i
                                 hipStream_t s);
 
 // dvr_kernels_tiled.hip
-// Number of 16x16 tiles of the B x H x W image batch.
+// Number of 8x8 tiles of the B x H x W image batch.
 int tiled_num_tiles(const RenderParams& P);
 hipError_t launch_forward_tiled(const RenderParams& P, const CkptParams& CK, int filter, int tfm, int blend,
                                 hipStream_t s);
@@ -61,6 +61,14 @@ hipError_t launch_forward_tiled(const RenderParams& P, const CkptParams& CK, int
 hipError_t launch_adjoint_tiled(const RenderParams& P, const AdjointParams& A, const CkptParams& CK,
                                 const LossParams& L, bool fused, bool ckptFromForward, int filter, int tfm,
                                 int blend, hipStream_t s);
+
+// dvr_kernels_row.hip: the same, 16 lanes a ray, and the sizes at which they are faster
+bool use_row_forward(const RenderParams& P, int filter);
+bool use_row_adjoint(const RenderParams& P, const AdjointParams& A, int tfm);
+hipError_t launch_forward_row(const RenderParams& P, const CkptParams& CK, int filter, int tfm, int blend,
+                              hipStream_t s);
+hipError_t launch_adjoint_row(const RenderParams& P, const AdjointParams& A, const CkptParams& CK, const LossParams& L,
+                              bool fused, bool ckptFromForward, int filter, int tfm, int blend, hipStream_t s);
 
 // dvr_kernels_aux.hip
 hipError_t launch_generate_rays(const float* viewport, int vSb, int vSr, int vSc, int B, int H, int W, float fovY,

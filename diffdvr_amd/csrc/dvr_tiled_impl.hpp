@@ -330,16 +330,17 @@ struct VolAgg {
     unsigned boff;    // floats from abase to the gradient base
 
     __device__ __forceinline__ unsigned slots() const { return 1u << lg; }
-    // every thread of the (one-wave) workgroup; lds is 16-byte aligned, agg_bytes(log2) long
+    // every lane of the wave that owns the table; lds is 16-byte aligned, agg_bytes(log2) long
     __device__ __forceinline__ void init(void* lds, int log2)
     {
+        const unsigned lane = threadIdx.x & 63u;
         lg = unsigned(log2);
         const unsigned kSlots = slots();
         tags = (unsigned*)lds;
         list = tags + kSlots;
         vals = (float*)(list + kSlots + 4);  // 16 bytes of padding after the list
-        for (int e = threadIdx.x; e < kSlots; e += blockDim.x) tags[e] = kAggEmpty;
-        for (int e = threadIdx.x; e < kSlots * 16; e += blockDim.x) vals[e] = 0.f;
+        for (unsigned e = lane; e < kSlots; e += 64u) tags[e] = kAggEmpty;
+        for (unsigned e = lane; e < kSlots * 16; e += 64u) vals[e] = 0.f;
     }
     // the table must be empty (flushed) when the base changes
     __device__ __forceinline__ void bind(float* g)
@@ -556,18 +557,19 @@ __device__ __forceinline__ void corner_move(CornerCache& c, const Vol& V, VS& vs
 }
 
 // ---------------------------------------------------------------------------
-// Reverse march of one ray with transmittance checkpoints every K*ckEvery
-// samples, walked back in register segments of K samples.  GM is the set of gradient
+// Reverse march of one ray with transmittance checkpoints every 2^ckShift
+// samples, walked back in register segments of K samples, from the one that
+// holds sample n - 1 down to segment segLo.  GM is the set of gradient
 // kinds compiled in: bit0 TF, bit1 volume, bit2 position (camera / step);
 // the runtime flags select among them.
 // ---------------------------------------------------------------------------
 template <int FILTER, int TFM, int BLEND, int K, int GM, class Sink, bool SPLIT = false, class VS = VolDirect>
 __device__ __forceinline__ void march_reverse(const Vol& V, const Tf& T, const Ray& r, int n, f4 adj_acc,
-                                              const float* ck, int ckS, int cap, int ckEvery, Sink& sink,
+                                              const float* ck, int ckS, int cap, int ckShift, Sink& sink,
                                               bool wantTf,
                                               bool wantVol, bool wantPos, VS& vs,
                                               f3& adj_start, f3& adj_dir, float& adj_step,
-                                              const float* dsr = nullptr, int dsS = 0)
+                                              const float* dsr = nullptr, int dsS = 0, int segLo = 0)
 {
     constexpr bool CT_TF = (GM & 1) != 0, CT_VOL = (GM & 2) != 0, CT_POS = (GM & 4) != 0;
     wantTf = CT_TF && wantTf;
@@ -596,19 +598,19 @@ __device__ __forceinline__ void march_reverse(const Vol& V, const Tf& T, const R
     float nAcc = 0.0f;
 
     const int nseg = (n + K - 1) / K;
-    for (int seg = nseg - 1; seg >= 0; --seg) {
+    for (int seg = nseg - 1; seg >= segLo; --seg) {
         const int i0 = seg * K;
         const int cnt = min(K, n - i0);
         // transmittance before sample i0
         float Tr = 1.0f;
         {
-            // checkpoints hold T after every K*ckEvery samples; recompute from the
-            // last one before i0 (ckEvery > 1, or a ray longer than the capacity)
-            const int c = min(seg / ckEvery, cap);
+            // recompute from the last checkpoint in front of i0 (an interval above K, or a ray
+            // longer than the capacity)
+            const int c = min(i0 >> ckShift, cap);
             if (c > 0) Tr = ck[(c - 1) * ckS];
             Cell cc;
             cell_invalidate(cc);
-            for (int i = c * K * ckEvery; i < i0; ++i) {
+            for (int i = c << ckShift; i < i0; ++i) {
                 const float t = r.t0 + float(i) * r.step;
                 const float d = dsr ? *(const gfloat*)(dsr + i * dsS) : fetch<FILTER>(V, sample_pos(r, t), cc);
                 float alpha, keep;
@@ -878,7 +880,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(GM == 3 
         // except for the arithmetic-bound Gaussian TF
         if constexpr (!kVolInst) vs.p = nullptr;
         march_reverse<FILTER, TFM, BLEND, K, GM, SinkTiled<TFM>, TFM != 3, VS>(V, T, r, n, adj_acc, ck, kBlock, CK.cap,
-                                                                               CK.every, sink, wantTf, wantVol,
+                                                                               __builtin_ctz(K * CK.every), sink, wantTf, wantVol,
                                                  wantPos, vs, adj_start, adj_dir, adj_step, stored ? ds : nullptr,
                                                  kBlock);
         if (A.ast) {
