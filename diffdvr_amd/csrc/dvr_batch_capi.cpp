@@ -57,6 +57,12 @@ int wave_shift_of(int ww)
     }
 }
 
+// Volume gradients in two passes: bytes of density adjoints a plan may hold at a time (C5's tiles of
+// 900-sample rays then run in groups of 37 000), and groups a run may be cut into.
+constexpr long long kMaxAdjointStore = 8LL << 30;
+constexpr int kMaxGroups = 64;
+constexpr double kMaxSampleDensity = 16.0;
+
 int tf_cols(int tfm)
 {
     switch (tfm) {
@@ -81,12 +87,12 @@ struct dvr_batch_plan {
     std::vector<dvr::BTf> tfs;
     int maxRC = 0;
     bool usePriv = false;
+    double sampleDensity = 0;  // samples per voxel of a view, averaged over the samples of the volume gradients
     double maxSamples = 0;  // upper bound of samples per ray over the views
     // layout
     int K = 16, waveWidth = 8, gridReq = 0, grid = 0, nTiles = 0, cap = 1;
     bool reinterpolate = false;  // no density store
     int cus = 0, resident = 0;  // compute units, resident workgroups of the current instance
-    int qBegin[dvr::kNumXcd + 1] = {};
     size_t lds = 0;
     int aggOffset = 0;  // float offset of the volume-gradient chunk table in LDS (0: none)
     int aggLog2 = dvr::kAggLog2;  // log2 of the chunk table's slots
@@ -99,7 +105,7 @@ struct dvr_batch_plan {
     int nSegsAll = 0;
     long long maxSegAll = 0;
     int nSegsAlways = 1;                // cleared by every run: queues and bricked scratch
-    long long maxSegAlways = dvr::kNumXcd;
+    long long maxSegAlways = kMaxGroups * dvr::kNumXcd;
     float* dBricks = nullptr;           // bricked volume-gradient scratch of every gradient volume
     size_t brickFloats = 0;
     dvr::DebrickSeg* dDebrick = nullptr;
@@ -110,45 +116,53 @@ struct dvr_batch_plan {
     float* dDs = nullptr;   // density store of the forward march (adjoint plans), or NULL
     size_t dsFloats = 0;
     int dsCap = 0;
+    // volume gradients in two passes (dvr_kernels_scatter.hip): density adjoints and rays of a group of tiles
+    float* dAs = nullptr;
+    size_t asFloats = 0;
+    int asCap = 0, groupTiles = 0;  // 0: the chunk tables of the one-pass instances
     std::string signature;  // autotune cache key
     bool frozen = false;    // captured graphs hold the scratch pointers: no re-layout
 
     ~dvr_batch_plan()
     {
         dev_free(dViews); dev_free(dVols); dev_free(dTfs); dev_free(dQueues); dev_free(dSegsAll); dev_free(dCk);
-        dev_free(dDs); dev_free(dBricks); dev_free(dDebrick);
+        dev_free(dDs); dev_free(dAs); dev_free(dBricks); dev_free(dDebrick);
     }
 
-    // floats between the TF-gradient table copies (odd: the copies start in different LDS banks);
-    // 0 (one table) when the copies would take more than 16 KiB of LDS per workgroup, which keeps
-    // eight one-wave workgroups resident per CU
-    int copy_stride() const
-    {
-        const int st = maxRC | 1;
-        return size_t(dvr::kTfCopies) * st * sizeof(float) <= 16384 ? st : 0;
-    }
+    // doubles between the TF-gradient table copies; 0 (one table) when the copies would take more than
+    // 16 KiB of LDS per workgroup, which keeps eight one-wave workgroups resident per CU
+    int copy_stride() const { return dvr::tf_grad_copy_stride(maxRC); }
 
-    // floats of the LDS TF table (the kernel pads linear-TF rows to 8 floats, dvr::tf_lds_stride)
-    int tf_lds() const { return tfm == 2 ? (maxRC / 5) * 8 : maxRC; }
+    // floats of the LDS TF table (the kernel pads linear-TF rows to 8 floats, dvr::tf_lds_stride), even
+    int tf_lds() const { return dvr::tf_grad_offset(tfm == 2 ? (maxRC / 5) * 8 : maxRC); }
 
     // register segment length of checkpoint interval K (64 = two 32-sample segments)
     int segK() const { return K > 32 ? 32 : K; }
 
-    dvr::BatchParams params() const
+    bool twoPass() const { return groupTiles > 0; }
+    int gmRun() const { return twoPass() ? (gm & 4 ? 13 : 9) : gm; }
+    int groups() const { return twoPass() ? (nTiles + groupTiles - 1) / groupTiles : 1; }
+
+    dvr::BatchParams params(int group = 0) const
     {
         dvr::BatchParams P{};
-        P.views = dViews; P.vols = dVols; P.tfs = dTfs; P.queues = dQueues; P.ck = dCk; P.lossOut = lossOut;
+        P.views = dViews; P.vols = dVols; P.tfs = dTfs; P.ck = dCk; P.lossOut = lossOut;
         P.ds = dsCap > 0 ? dDs : nullptr; P.dsCap = dsCap;
         P.nViews = (int)views.size(); P.nTiles = nTiles; P.ckCap = cap;
         P.ckEvery = K > 32 ? K / 32 : 1;
-        for (int i = 0; i <= dvr::kNumXcd; ++i) P.qBegin[i] = qBegin[i];
+        // the group's tiles, one range per XCD
+        const int t0 = twoPass() ? group * groupTiles : 0, t1 = twoPass() ? std::min(nTiles, t0 + groupTiles) : nTiles;
+        for (int q = 0; q <= dvr::kNumXcd; ++q) P.qBegin[q] = t0 + (int)((long long)(t1 - t0) * q / dvr::kNumXcd);
+        P.queues = dQueues + group * dvr::kNumXcd;
+        P.tile0 = t0;
+        if (twoPass()) P.as = dvr::AdjStore{dAs + size_t(groupTiles) * dvr::kRayRecord * dvr::kBlock, dAs, asCap};
         P.earlyOut = earlyOut; P.lossKind = lossKind;
         P.wantTf = (gm & 1) ? 1 : 0; P.wantVol = (gm & 2) ? 1 : 0; P.wantCam = (gm & 4) ? 1 : 0;
         P.waveShift = wave_shift_of(waveWidth);
         P.tileW = waveWidth; P.tileH = 64 / waveWidth;
         P.ldsTf = tf_lds(); P.usePriv = usePriv ? 1 : 0;
         P.tfCopyStride = (gm && !usePriv) ? copy_stride() : 0;
-        P.ldsAgg = aggOffset;
+        P.ldsAgg = twoPass() ? 0 : aggOffset;
         P.aggLog2 = aggLog2;
         return P;
     }
@@ -166,16 +180,13 @@ struct dvr_batch_plan {
         }
         if (t >= (1LL << 31)) fail(DVR_ERR_INVALID_ARGUMENT, "batch has too many tiles");
         nTiles = (int)t;
-        for (int q = 0; q <= dvr::kNumXcd; ++q) qBegin[q] = (int)((long long)nTiles * q / dvr::kNumXcd);
-        const size_t ldsG =
-            gm ? (usePriv ? size_t(maxRC) * dvr::kBatchBlock
-                          : (copy_stride() > 0 ? size_t(dvr::kTfCopies) * copy_stride() : size_t(maxRC)))
-               : 0;
+        const size_t ldsG = gm ? size_t(dvr::tf_grad_floats(maxRC, usePriv, dvr::kBatchBlock, copy_stride())) : 0;
         lds = sizeof(float) * (size_t(tf_lds()) + ldsG);
         // volume gradients: the per-wave table of 64-byte chunks follows the TF tables (not
         // reserved for camera-only plans, which run the same instance without it)
         aggOffset = 0;
         int occ = 0;
+        groupTiles = 0;
         if ((gm & 2) && volGrad) {
             // the largest table that keeps the instance at the waves per SIMD its registers
             // were fitted for (workgroups per CU from the runtime's occupancy calculator)
@@ -183,10 +194,19 @@ struct dvr_batch_plan {
             const int target = 4 * dvr::batched_vol_waves(gm);
             for (int lg = dvr::kAggLog2; lg >= dvr::kAggMinLog2; --lg) {
                 aggLog2 = lg;
-                lds = sizeof(float) * size_t(aggOffset) + dvr::agg_bytes(lg);
+                lds = sizeof(float) * size_t(aggOffset) + dvr::agg_bytes(lg, sizeof(double));
                 check_hip(dvr::launch_batched(params(), filter, tfm, blend, segK(), gm, 0, lds, nullptr, &occ),
                           "occupancy query");
                 if (occ >= target) break;
+            }
+            // Two passes up to kMaxSampleDensity samples a voxel and view: the samples of rays close
+            // together meet in the one-pass walk's registers and small table, those of rays far apart
+            // only in the scatter kernel's.  Measured (one pass / two passes): 0.4 samples a voxel 11.4 /
+            // 5.2 ms, 1.7 12.2 / 5.9, 6.9 5.9 / 4.0, 14 4.9 / 4.4, 28 5.7 / 11.0 (256^3; 2.0 / 1.9 at 128^3).
+            if (sampleDensity <= kMaxSampleDensity && reserve_adjoints()) {
+                lds = sizeof(float) * (size_t(tf_lds()) + ldsG);
+                check_hip(dvr::launch_batched(params(), filter, tfm, blend, segK(), gmRun(), 0, lds, nullptr, &occ),
+                          "occupancy query");
             }
         } else {
             check_hip(dvr::launch_batched(params(), filter, tfm, blend, segK(), gm, 0, lds, nullptr, &occ),
@@ -199,8 +219,9 @@ struct dvr_batch_plan {
         // default: two waves per SIMD (eight one-wave workgroups per CU; measured
         // best for gather-bound tiles on MI355X: fewer concurrent rays per CU keep
         // their cells in L1), within residency; volume-gradient instances are bound
-        // by the latency of their walk and fill the CU (four waves per SIMD)
-        int g = gridReq > 0 ? gridReq : (((gm & 2) && volGrad) ? resident : std::min(resident, 8 * cus));
+        // by the latency of their walk and fill the CU (four waves per SIMD) unless they leave the
+        // corner gradients to k_scatter_volume
+        int g = gridReq > 0 ? gridReq : (((gm & 2) && volGrad && !twoPass()) ? resident : std::min(resident, 8 * cus));
         g = std::max(1, std::min(g, std::max(nTiles, 1)));
         grid = g;
         cap = std::max(1, std::min((int)std::ceil(maxSamples / K), 1 << 14));
@@ -231,6 +252,36 @@ struct dvr_batch_plan {
                   "hipMemcpy views");
     }
 
+    // The density adjoints of as many tiles as kMaxAdjointStore bytes hold (every ray as long as the
+    // longest), at least 4096 (the chip's one-wave workgroups at four waves per SIMD) or all; where
+    // memory is short, half as many and so on.  False: the one-pass instances and their chunk tables.
+    bool reserve_adjoints()
+    {
+        const double want = std::ceil(maxSamples) + 2.0;
+        if (want > double(1 << 20) || nTiles == 0) return false;
+        asCap = dvr::adj_store_cap((int)want);
+        const size_t perTile = dvr::adj_store_floats(asCap);
+        const int least = std::max(std::min(nTiles, 4096), (nTiles + kMaxGroups - 1) / kMaxGroups);
+        long long t = std::min<long long>(nTiles, kMaxAdjointStore / (long long)(perTile * sizeof(float)));
+        for (; t >= least; t = t > least ? std::max<long long>(least, t / 2) : 0) {
+            const size_t need = size_t(t) * perTile;
+            if (need > asFloats) {
+                dev_free(dAs);
+                dAs = nullptr;
+                asFloats = 0;
+                if (hipMalloc((void**)&dAs, need * sizeof(float)) != hipSuccess) {
+                    (void)hipGetLastError();
+                    dAs = nullptr;
+                    continue;
+                }
+                asFloats = need;
+            }
+            groupTiles = (int)t;
+            return true;
+        }
+        return false;
+    }
+
     void zero(bool gradients, hipStream_t s) const
     {
         const int n = gradients ? nSegsAll : nSegsAlways;
@@ -243,9 +294,19 @@ struct dvr_batch_plan {
     {
         zero((flags & DVR_BATCH_ZERO_GRADIENTS) != 0, s);
         if (evBegin) check_hip(hipEventRecord(evBegin, s), "hipEventRecord");
-        if (nTiles > 0)
-            check_hip(dvr::launch_batched(params(), filter, tfm, blend, segK(), gm, grid, lds, s, nullptr),
-                      "batched launch");
+        for (int k = 0; nTiles > 0 && k < groups(); ++k) {
+            const dvr::BatchParams P = params(k);
+            check_hip(dvr::launch_batched(P, filter, tfm, blend, segK(), gmRun(), grid, lds, s, nullptr), "batched launch");
+            if (!twoPass()) continue;
+            dvr::ScatterParams S{};
+            S.S = P.as;
+            S.nTiles = P.qBegin[dvr::kNumXcd] - P.tile0;
+            S.tile0 = P.tile0;
+            S.views = dViews;
+            S.nViews = (int)views.size();
+            S.vols = dVols;
+            check_hip(dvr::launch_scatter_volume(S, filter, s), "scatter launch");
+        }
         if (evEnd) check_hip(hipEventRecord(evEnd, s), "hipEventRecord");
         if (nDebrick > 0) check_hip(dvr::launch_debrick(dDebrick, nDebrick, maxBricks, s), "debrick launch");
     }
@@ -410,6 +471,7 @@ dvr_batch_plan* create(const dvr_batch* b, const dvr_batch_options* o)
         p->tfs.push_back(d);
     }
     long long totalPix = 0;
+    double volSamples = 0, volDensity = 0;
     std::vector<dvr::BView> vs;
     for (int i = 0; i < b->num_views; ++i) {
         const dvr_batch_view& v = b->views[i];
@@ -446,7 +508,13 @@ dvr_batch_plan* create(const dvr_batch* b, const dvr_batch_options* o)
         const dvr::BVol& vol = p->vols[v.volume];
         const double diag = std::sqrt(double(vol.bsize[0]) * vol.bsize[0] + double(vol.bsize[1]) * vol.bsize[1] +
                                       double(vol.bsize[2]) * vol.bsize[2]);
-        p->maxSamples = std::max(p->maxSamples, diag / double(v.step_size) + 2.0);
+        const double rayMax = diag / double(v.step_size) + 2.0;
+        p->maxSamples = std::max(p->maxSamples, rayMax);
+        if (vol.adj) {  // about half the longest ray on average
+            const double samples = 0.5 * rayMax * v.width * v.height;
+            volSamples += samples;
+            volDensity += samples * samples / (double(vol.X) * vol.Y * vol.Z);
+        }
         vs.push_back(d);
     }
     if (!b->forward_only && b->loss != DVR_LOSS_NONE) {
@@ -459,6 +527,7 @@ dvr_batch_plan* create(const dvr_batch* b, const dvr_batch_options* o)
         return a.tf != c.tf ? a.tf < c.tf : a.vol < c.vol;
     });
     p->views = vs;
+    p->sampleDensity = volSamples > 0 ? volDensity / volSamples : 0.0;
     if (b->forward_only) p->gm = 0;
     else {
         if (!anyTfGrad && !anyVolGrad && !anyCamGrad && !p->lossOut)
@@ -472,8 +541,8 @@ dvr_batch_plan* create(const dvr_batch* b, const dvr_batch_options* o)
     DeviceGuard guard(b->device);
     // clear list: queue counters first, then every gradient buffer and the loss
     std::vector<dvr::ZeroSeg> segs;
-    p->dQueues = dev_alloc<unsigned>(dvr::kNumXcd);
-    segs.push_back({reinterpret_cast<float*>(p->dQueues), dvr::kNumXcd});
+    p->dQueues = dev_alloc<unsigned>(kMaxGroups * dvr::kNumXcd);
+    segs.push_back({reinterpret_cast<float*>(p->dQueues), kMaxGroups * dvr::kNumXcd});
     // bricked volume-gradient scratch (2 x 2 x 4 voxels per 64-byte chunk), one range per gradient
     // volume, each 256-byte aligned; cleared by every run, added into the gradient after the kernel
     if (p->gm & 2) {
@@ -482,7 +551,7 @@ dvr_batch_plan* create(const dvr_batch* b, const dvr_batch_options* o)
         for (auto& v : p->vols) {
             off.push_back(total);
             if (!v.adj) continue;
-            const size_t n = size_t((v.X + 1) / 2) * size_t((v.Y + 1) / 2) * size_t((v.Z + 3) / 4) * 16;
+            const size_t n = dvr::brick_floats(v.X, v.Y, v.Z);
             total += (n + 63) / 64 * 64;
         }
         if (total > 0) {
@@ -496,7 +565,7 @@ dvr_batch_plan* create(const dvr_batch* b, const dvr_batch_options* o)
                 const long long nb = (long long)((v.X + 1) / 2) * ((v.Y + 1) / 2) * ((v.Z + 3) / 4);
                 segs.push_back({v.brick, nb * 16});
                 p->maxSegAlways = std::max(p->maxSegAlways, nb * 16);
-                db.push_back({v.brick, v.adj, v.X, v.Y, v.Z, 0});
+                db.push_back({v.brick, v.adj, v.X, v.Y, v.Z, 0, (long long)v.Y * v.Z, v.Z, 1});
                 p->maxBricks = std::max(p->maxBricks, nb);
             }
             p->nDebrick = (int)db.size();
@@ -663,7 +732,7 @@ dvr_status dvr_batch_plan_autotune(dvr_batch_plan* plan, int32_t iterations, dvr
         hipStream_t s = (hipStream_t)stream;
         const int gridReq = plan->gridReq;
         // the leading tag names the kernels' and search's revision: results of older ones are not reused
-        const std::string tuneKey = "r2|" + plan->signature + (plan->reinterpolate ? "|reinterpolate" : "");
+        const std::string tuneKey = "r3|" + plan->signature + (plan->reinterpolate ? "|reinterpolate" : "");
         Tuned best{0, 0, 0};
         {
             std::lock_guard<std::mutex> lk(g_tuneMu);
@@ -754,10 +823,10 @@ int32_t dvr_batch_plan_chunk_slots(const dvr_batch_plan* plan)
 int64_t dvr_batch_plan_workspace_bytes(const dvr_batch_plan* plan)
 {
     if (!plan) return -1;
-    return (int64_t)((plan->ckFloats + plan->dsFloats + plan->brickFloats) * sizeof(float) +
+    return (int64_t)((plan->ckFloats + plan->dsFloats + plan->asFloats + plan->brickFloats) * sizeof(float) +
                      plan->nDebrick * sizeof(dvr::DebrickSeg) + plan->views.size() * sizeof(dvr::BView) +
                      plan->vols.size() * sizeof(dvr::BVol) + plan->tfs.size() * sizeof(dvr::BTf) +
-                     plan->nSegsAll * sizeof(dvr::ZeroSeg) + dvr::kNumXcd * sizeof(unsigned));
+                     plan->nSegsAll * sizeof(dvr::ZeroSeg) + kMaxGroups * dvr::kNumXcd * sizeof(unsigned));
 }
 
 // ---------------------------------------------------------------------------

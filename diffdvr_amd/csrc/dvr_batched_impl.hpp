@@ -32,12 +32,8 @@ __device__ __forceinline__ void batched_flush_tf(const BatchParams& B, int tfi, 
         if (priv) {
             v = 0.0f;
             for (int t = 0; t < kBatchBlock; ++t) v += s_g[e * kBatchBlock + t];
-        } else if (B.tfCopyStride > 0) {
-            v = 0.0f;
-#pragma unroll
-            for (int k = 0; k < kTfCopies; ++k) v += s_g[k * B.tfCopyStride + e];
         } else {
-            v = s_g[e];
+            v = tf_grad_sum(s_g, e, B.tfCopyStride);
         }
         if (v != 0.0f) gatomic_add(g, unsigned(e), v);
     }
@@ -81,7 +77,7 @@ __global__ __launch_bounds__(kBatchBlock) __attribute__((amdgpu_waves_per_eu(
     // into the volume's bricked scratch at the end of every tile (each tile belongs to one view,
     // hence one volume); k_debrick adds the scratch into the caller's gradient after the launch
     constexpr bool kVolInst = (GM & 2) != 0;
-    using VS = std::conditional_t<kVolInst, VolAgg<BrickLayout>, VolDirect>;
+    using VS = std::conditional_t<kVolInst, VolAgg<BrickLayout, double>, VolDirectT<BrickLayout>>;
     VS vs;
     const bool aggOn = kVolInst && B.wantVol && B.ldsAgg > 0;
     if constexpr (kVolInst) {
@@ -122,7 +118,7 @@ __global__ __launch_bounds__(kBatchBlock) __attribute__((amdgpu_waves_per_eu(
             for (int e = threadIdx.x; e < curRC; e += kBatchBlock)
                 s_tf[(e / tf_cols<TFM>()) * tf_lds_stride<TFM>() + (e % tf_cols<TFM>())] = gld(tf.p, unsigned(e));
             if (curWantTf) {
-                const int ng = priv ? curRC * kBatchBlock : (B.tfCopyStride > 0 ? kTfCopies * B.tfCopyStride : curRC);
+                const int ng = tf_grad_floats(curRC, priv, kBatchBlock, B.tfCopyStride);
                 for (int e = threadIdx.x; e < ng; e += kBatchBlock) s_g[e] = 0.0f;
             }
             __syncthreads();
@@ -199,13 +195,22 @@ __global__ __launch_bounds__(kBatchBlock) __attribute__((amdgpu_waves_per_eu(
                 // the store holds every sample of every active ray of the wave (else re-interpolate;
                 // the choice is uniform over the wave, so the segment loop does not diverge)
                 const bool stored = ds != nullptr && __all(n <= B.dsCap);
+                AdjLane<false> as;
+                if constexpr ((GM & 8) != 0) {
+                    if (B.wantVol && vol.adj != nullptr) {
+                        vs.p = vol.brick;
+                        vs.L.set(vol.X, vol.Y, vol.Z);
+                        as = adj_store<false>(B.as, tile - B.tile0, threadIdx.x);
+                        store_ray(B.as, tile - B.tile0, threadIdx.x, r, n);
+                    }
+                }
                 march_reverse<FILTER, TFM, BLEND, K, GM, SinkTiled<TFM>, true, VS>(VV, T, r, n, adj_acc, ck,
                                                                                    kBatchBlock, B.ckCap,
                                                                                    __builtin_ctz(K * B.ckEvery),
                                                                                    sink, curWantTf,
                                                          wantVol, wantCam, vs,
                                                          adj_start, adj_dir, adj_step, stored ? ds : nullptr,
-                                                         kBatchBlock);
+                                                         kBatchBlock, 0, as);
                 if constexpr ((GM & 4) != 0) {
                     if (wantCam) {
                         // ray (eye, normalize(front + fx tanX right + fy tanY up)) -> viewport rows
@@ -227,6 +232,9 @@ __global__ __launch_bounds__(kBatchBlock) __attribute__((amdgpu_waves_per_eu(
                     }
                 }
             }
+        }
+        if constexpr ((GM & 8) != 0) {
+            if (!valid && B.wantVol && vol.adj != nullptr) store_ray(B.as, tile - B.tile0, threadIdx.x, Ray{}, 0);
         }
         if constexpr (ADJ) {
             if constexpr (kVolInst) {
@@ -281,6 +289,8 @@ static hipError_t batched_fbk(const BatchParams& P, int tfm, int gm, int grid, s
     case 3: return batched_k<FILTER, TV, BLEND, K, 3>(P, grid, lds, s, occ);       \
     case 5: return batched_k<FILTER, TV, BLEND, K, 5>(P, grid, lds, s, occ);       \
     case 7: return batched_k<FILTER, TV, BLEND, K, 7>(P, grid, lds, s, occ);       \
+    case 9: return batched_k<FILTER, TV, BLEND, K, 9>(P, grid, lds, s, occ);       \
+    case 13: return batched_k<FILTER, TV, BLEND, K, 13>(P, grid, lds, s, occ);     \
     default: return hipErrorInvalidValue;                                          \
     }
     switch (tfm) {

@@ -610,16 +610,106 @@ void do_forward(const dvr_inputs* inputs, dvr_outputs* outputs, const dvr_forwar
     }
 }
 
+// Device scratch of one call.
+struct Scratch {
+    void* data = nullptr;
+    size_t bytes = 0;
+};
+
+// no two indices of the X x Y x Z (x B) gradient share an element (an expanded tensor takes atomics)
+bool distinct_elements(const Checked& c, const dvr::AdjointParams& A)
+{
+    std::pair<int64_t, int64_t> d[4] = {{A.avSx, c.X}, {A.avSy, c.Y}, {A.avSz, c.Z}, {A.avSb, A.avSb != 0 ? c.B : 1}};
+    std::sort(d, d + 4);
+    int64_t reach = 0;  // largest offset of the dimensions so far
+    for (const auto& [stride, n] : d) {
+        if (n == 1) continue;
+        if (stride <= reach) return false;
+        reach += stride * (n - 1);
+    }
+    return true;
+}
+
+// Volume gradients of the checkpointed adjoint in two passes (dvr_kernels_scatter.hip): the walk stores
+// the density adjoints of a group of tiles and their rays, k_scatter_volume adds them into bricked
+// scratch, and after the last group k_debrick adds that into the caller's gradient.  Scratch layout:
+// [bricks][rays][density adjoints], each 64-byte aligned.
+class TwoPassGradient {
+public:
+    TwoPassGradient(const Checked& c, const dvr::AdjointParams& A) : c_(c), A_(A)
+    {
+        // the store holds the longest ray of a uniform box and step; clearing and adding the bricks
+        // (16 bytes a voxel) pays from a few samples per ten voxels on
+        if (!A.avol || c.preshaded || c.P.st || c.P.bsize || !distinct_elements(c, A)) return;
+        volumes_ = A.avSb != 0 ? c.B : 1;
+        const double voxels = double(c.X) * c.Y * c.Z * volumes_;
+        tiles_ = dvr::tiled_num_tiles(c.P);
+        cap_ = dvr::adj_store_cap(density_cap(c));
+        const double samples = double(c.B) * c.W * c.H * cap_ * 0.5;
+        if (tiles_ == 0 || samples < 0.25 * voxels) return;
+        const size_t perTile = dvr::adj_store_floats(cap_) * sizeof(float);
+        group_ = int(std::min<size_t>(size_t(tiles_), kMaxStore / perTile));
+        if (group_ < std::min(tiles_, 4096)) return;  // groups too small to fill the chip
+        brickFloats_ = dvr::brick_floats(c.X, c.Y, c.Z);
+        if (brickFloats_ >= (size_t(1) << 30)) return;  // 32-bit byte offsets
+        bytes_ = sizeof(float) * brickFloats_ * volumes_ + size_t(group_) * perTile;
+    }
+    size_t bytes() const { return bytes_; }
+
+    // Runs the adjoint: launch(CK) must launch the tiles CK.tile0 .. tile0 + tileN - 1.
+    template <class Launch>
+    void run(dvr::CkptParams CK, const Scratch& scr, hipStream_t s, Launch launch) const
+    {
+        if (bytes_ == 0 || scr.bytes < bytes_) return launch(CK);
+        float* brick = (float*)scr.data;
+        const size_t brickAll = brickFloats_ * volumes_;
+        CK.as.rays = brick + brickAll;
+        CK.as.adj = CK.as.rays + size_t(group_) * dvr::kRayRecord * dvr::kBlock;
+        CK.as.cap = cap_;
+        check_hip(dvr::launch_clear(brick, brickAll, s), "clear launch");
+        for (int t0 = 0; t0 < tiles_; t0 += group_) {
+            CK.tile0 = t0;
+            CK.tileN = std::min(group_, tiles_ - t0);
+            launch(CK);
+            dvr::ScatterParams S;
+            std::memset(&S, 0, sizeof(S));
+            S.S = CK.as;
+            S.nTiles = CK.tileN;
+            S.tile0 = t0;
+            S.brick = brick;
+            S.brickFloats = brickFloats_;
+            S.tilesPerVolume = volumes_ > 1 ? tiles_ / c_.B : tiles_;
+            S.X = c_.X; S.Y = c_.Y; S.Z = c_.Z;
+            check_hip(dvr::launch_scatter_volume(S, c_.filter, s), "scatter launch");
+        }
+        const dvr::DebrickSeg D{brick, A_.avol, c_.X, c_.Y, c_.Z, 0, A_.avSx, A_.avSy, A_.avSz};
+        check_hip(dvr::launch_debrick_call(D, volumes_, A_.avSb, s), "debrick launch");
+    }
+
+private:
+    static constexpr size_t kMaxStore = size_t(2) << 30;
+    const Checked& c_;
+    const dvr::AdjointParams& A_;
+    int volumes_ = 1, tiles_ = 0, cap_ = 0, group_ = 0;
+    size_t brickFloats_ = 0, bytes_ = 0;
+};
+
+int adjoint_method(const Checked& c, const dvr_adjoint_options* opt)
+{
+    const int method = opt ? opt->method : DVR_ADJOINT_AUTO;
+    if (method != DVR_ADJOINT_AUTO) return method;
+    return tiled_ok(c) ? DVR_ADJOINT_CHECKPOINT : DVR_ADJOINT_INVERSION;
+}
+
 void do_adjoint(const dvr_inputs* inputs, const dvr_outputs* fwd, const dvr_tensor* adj_color,
-                dvr_adjoint_outputs* ao, const dvr_adjoint_options* opt, void* stream)
+                dvr_adjoint_outputs* ao, const dvr_adjoint_options* opt, void* stream, const Scratch& scr = {})
 {
     Checked c = check_inputs(inputs);
     dvr::AdjointParams A = check_adjoint(c, fwd, adj_color, ao);
     DeviceGuard g(c.device);
     hipStream_t s = (hipStream_t)stream;
-    int method = opt ? opt->method : DVR_ADJOINT_AUTO;
-    int path = opt ? opt->path : DVR_PATH_AUTO;
-    if (method == DVR_ADJOINT_AUTO) method = tiled_ok(c) ? DVR_ADJOINT_CHECKPOINT : DVR_ADJOINT_INVERSION;
+    const int method = adjoint_method(c, opt);
+    const int path = opt ? opt->path : DVR_PATH_AUTO;
     if (c.preshaded) {
         if (method != DVR_ADJOINT_INVERSION || path == DVR_PATH_TILED)
             fail(DVR_ERR_UNSUPPORTED, "pre-shaded volumes use the inversion adjoint on the plain path");
@@ -667,8 +757,11 @@ void do_adjoint(const dvr_inputs* inputs, const dvr_outputs* fwd, const dvr_tens
     }
     dvr::LossParams L;
     std::memset(&L, 0, sizeof(L));
-    check_hip(dvr::launch_adjoint_tiled(c.P, A, CK, L, false, fromFwd, c.filter, c.tfm, c.blend, s),
-              "adjoint (tiled) launch");
+    const TwoPassGradient vol(c, A);
+    vol.run(CK, scr, s, [&](const dvr::CkptParams& ck) {
+        check_hip(dvr::launch_adjoint_tiled(c.P, A, ck, L, false, fromFwd, c.filter, c.tfm, c.blend, s),
+                  "adjoint (tiled) launch");
+    });
 }
 
 // fixed: the allocation-free variant's scratch (a getter of the device's static array and its
@@ -1073,6 +1166,32 @@ dvr_status dvr_compare_to_image(const dvr_tensor* color, const dvr_tensor* gradi
                                 dvr_tensor* difference_out, dvr_tensor* gradients_out, int32_t reduce, void* stream)
 {
     return guarded([&] { do_compare(color, gradients, reference, difference_out, gradients_out, reduce, stream); });
+}
+
+int64_t dvr_adjoint_scratch_bytes(const dvr_inputs* inputs, const dvr_outputs* outputs_from_forward,
+                                  const dvr_tensor* adj_color, const dvr_adjoint_outputs* adj_outputs,
+                                  const dvr_adjoint_options* options)
+{
+    int64_t r = -1;
+    guarded([&] {
+        Checked c = check_inputs(inputs);
+        const dvr::AdjointParams A = check_adjoint(c, outputs_from_forward, adj_color, adj_outputs);
+        r = adjoint_method(c, options) == DVR_ADJOINT_CHECKPOINT ? int64_t(TwoPassGradient(c, A).bytes()) : 0;
+    });
+    return r;
+}
+
+dvr_status dvr_render_adjoint_scratch(const dvr_inputs* inputs, const dvr_outputs* outputs_from_forward,
+                                      const dvr_tensor* adj_color, dvr_adjoint_outputs* adj_outputs,
+                                      const dvr_adjoint_options* options, void* scratch, int64_t scratch_bytes,
+                                      void* stream)
+{
+    return guarded([&] {
+        if (scratch_bytes > 0 && (reinterpret_cast<uintptr_t>(scratch) & 255u) != 0)
+            fail(DVR_ERR_INVALID_ARGUMENT, "scratch must be 256-byte aligned");
+        do_adjoint(inputs, outputs_from_forward, adj_color, adj_outputs, options, stream,
+                   Scratch{scratch, scratch ? size_t(std::max<int64_t>(scratch_bytes, 0)) : 0});
+    });
 }
 
 int64_t dvr_checkpoint_buffer_elements(const dvr_inputs* inputs, int32_t checkpoint_interval)

@@ -91,6 +91,13 @@ __device__ __forceinline__ float wave_sum(float v)
     return v;
 }
 
+__device__ __forceinline__ int wave_max(int v)
+{
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) v = max(v, __shfl_xor(v, o, 64));
+    return __builtin_amdgcn_readfirstlane(v);
+}
+
 // Workgroup index -> logical tile index so that each XCD (workgroups are
 // dispatched round-robin over the 8 XCDs) owns one contiguous range of tiles:
 // neighbouring tiles then share that XCD's L2.

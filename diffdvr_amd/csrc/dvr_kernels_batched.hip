@@ -36,17 +36,17 @@ hipError_t launch_batched(const BatchParams& P, int filter, int tfm, int blend, 
 #undef DVR_CALL
 }
 
-// Adds each volume's bricked gradient scratch (2 x 2 x 4 voxels per 64-byte
-// chunk, bricks z-fastest) into the caller's contiguous X x Y x Z gradient: a
-// thread per brick, consecutive threads on consecutive z bricks of one (x, y)
-// brick column, so reads and the four 16-byte row segments it updates are
-// contiguous across the wave.  blockIdx.y = volume.
-__global__ __launch_bounds__(256) void k_debrick(const DebrickSeg* segs)
+// Adds a volume's bricked gradient scratch (2 x 2 x 4 voxels per 64-byte chunk,
+// bricks z-fastest) into the caller's X x Y x Z gradient: a thread per brick,
+// consecutive threads on consecutive z bricks of one (x, y) brick column, so
+// reads and, with z innermost, the four 16-byte row segments it updates are
+// contiguous across the wave.
+__device__ __forceinline__ void debrick(const DebrickSeg& S)
 {
-    const DebrickSeg S = segs[blockIdx.y];
     const int BY = (S.Y + 1) >> 1, BZ = (S.Z + 3) >> 2;
     const long long nb = (long long)((S.X + 1) >> 1) * BY * BZ;
-    const bool vec = (S.Z & 3) == 0;
+    const bool vec = S.sz == 1 && (S.Z & 3) == 0 && (S.sx & 3) == 0 && (S.sy & 3) == 0 &&
+                     (reinterpret_cast<uintptr_t>(S.adj) & 15u) == 0;
     for (long long b = (long long)blockIdx.x * 256 + threadIdx.x; b < nb; b += (long long)gridDim.x * 256) {
         const int zb = int(b % BZ);
         const long long r = b / BZ;
@@ -57,17 +57,53 @@ __global__ __launch_bounds__(256) void k_debrick(const DebrickSeg* segs)
             const int x = 2 * xb + (q >> 1), y = 2 * yb + (q & 1);
             if (x >= S.X || y >= S.Y) continue;
             const float4 v = src[q];
-            float* g = S.adj + ((size_t)x * S.Y + y) * S.Z + 4 * zb;
+            float* g = S.adj + x * S.sx + y * S.sy + 4 * zb * S.sz;
             if (vec) {
                 float4 o = *reinterpret_cast<float4*>(g);
                 o.x += v.x; o.y += v.y; o.z += v.z; o.w += v.w;
                 *reinterpret_cast<float4*>(g) = o;
             } else {
                 const float vv[4] = {v.x, v.y, v.z, v.w};
-                for (int k = 0; k < 4 && 4 * zb + k < S.Z; ++k) g[k] += vv[k];
+                for (int k = 0; k < 4 && 4 * zb + k < S.Z; ++k) g[k * S.sz] += vv[k];
             }
         }
     }
+}
+// blockIdx.y = volume of a plan
+__global__ __launch_bounds__(256) void k_debrick(const DebrickSeg* segs)
+{
+    const DebrickSeg S = segs[blockIdx.y];
+    debrick(S);
+}
+// blockIdx.y = batch of one call's gradient
+__global__ __launch_bounds__(256) void k_debrick_call(DebrickSeg S, long long brickFloats, long long sb)
+{
+    S.brick += blockIdx.y * brickFloats;
+    S.adj += blockIdx.y * sb;
+    debrick(S);
+}
+
+__global__ __launch_bounds__(256) void k_clear(float4* p, long long n)
+{
+    for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long long)gridDim.x * 256)
+        p[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+}
+
+hipError_t launch_clear(float* p, size_t n, hipStream_t s)
+{
+    if (n == 0) return hipSuccess;
+    const long long v = (long long)(n / 4);
+    const long long bx = (v + 255) / 256;
+    hipLaunchKernelGGL(k_clear, dim3(unsigned(bx < 4096 ? bx : 4096)), dim3(256), 0, s, reinterpret_cast<float4*>(p), v);
+    return hipGetLastError();
+}
+
+hipError_t launch_debrick_call(const DebrickSeg& S, int batches, long long sb, hipStream_t s)
+{
+    const long long bf = (long long)brick_floats(S.X, S.Y, S.Z);
+    const long long bx = (bf / 16 + 255) / 256;
+    hipLaunchKernelGGL(k_debrick_call, dim3(unsigned(bx < 8192 ? bx : 8192), unsigned(batches)), dim3(256), 0, s, S, bf, sb);
+    return hipGetLastError();
 }
 
 hipError_t launch_debrick(const DebrickSeg* dSegs, int nSegs, long long maxBricks, hipStream_t s)

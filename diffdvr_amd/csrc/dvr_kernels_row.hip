@@ -83,18 +83,17 @@ static hipError_t adj_row_g(const RenderParams& P, const AdjointParams& A, const
     const int RC = P.R * P.C;
     constexpr int kThreads = kRowAdjBlock;
     const bool usePriv = TFM == 3 && A.atf && RC <= 48;  // private slices <= 48 KiB of LDS
-    const int stride = RC | 1;                           // odd: the copies start in different LDS banks
-    const int copyStride = size_t(kTfCopies) * stride * sizeof(float) <= 16384 ? stride : 0;
-    const int ng = A.atf ? (usePriv ? RC * kThreads : (copyStride > 0 ? kTfCopies * copyStride : RC)) : 0;
+    const int copyStride = tf_grad_copy_stride(RC);
+    const int ng = A.atf ? tf_grad_floats(RC, usePriv, kThreads, copyStride) : 0;
     int aggLog2 = kAggLog2;
-    size_t lds = sizeof(float) * (size_t(RC) + size_t(ng));
+    size_t lds = sizeof(float) * size_t(tf_grad_offset(RC) + ng);
     if ((GM & 2) && A.avol) {
         // the largest chunk table per wave beside the TF tables that leaves room for sixteen waves per CU
-        const size_t base = sizeof(float) * size_t(agg_offset(RC, ng));
+        const size_t base = sizeof(float) * size_t(agg_offset(tf_grad_offset(RC), ng));
         constexpr size_t kWaves = kThreads / 64;
-        while (aggLog2 > kAggMinLog2 && base + kWaves * agg_bytes(aggLog2) > size_t(kLdsPerCu) * kWaves / kTiledVolWgPerCu)
+        while (aggLog2 > kAggMinLog2 && base + kWaves * agg_bytes(aggLog2, sizeof(float)) > size_t(kLdsPerCu) * kWaves / kTiledVolWgPerCu)
             --aggLog2;
-        lds = base + kWaves * agg_bytes(aggLog2);
+        lds = base + kWaves * agg_bytes(aggLog2, sizeof(float));
     }
     hipLaunchKernelGGL((k_adjoint_row<FILTER, TFM, BLEND, GM>), dim3(nTiles * row_blocks_per_tile(kThreads)),
                        dim3(kThreads), lds, s, P, A, CK, L, fused ? 1 : 0, ckFromFwd ? 1 : 0, usePriv ? 1 : 0, copyStride,
@@ -107,6 +106,10 @@ static hipError_t adj_row_t(const RenderParams& P, const AdjointParams& A, const
                             bool fused, bool ckFromFwd, hipStream_t s)
 {
     const bool pos = A.ars || A.ast;
+    if (A.avol && CK.as.adj) {  // volume gradients in two passes
+        if (pos) return adj_row_g<FILTER, TFM, BLEND, 13>(P, A, CK, L, fused, ckFromFwd, s);
+        return adj_row_g<FILTER, TFM, BLEND, 9>(P, A, CK, L, fused, ckFromFwd, s);
+    }
     if (pos && A.avol) return adj_row_g<FILTER, TFM, BLEND, 7>(P, A, CK, L, fused, ckFromFwd, s);
     if (pos && A.atf) return adj_row_g<FILTER, TFM, BLEND, 5>(P, A, CK, L, fused, ckFromFwd, s);
     if (pos) return adj_row_g<FILTER, TFM, BLEND, 4>(P, A, CK, L, fused, ckFromFwd, s);

@@ -90,6 +90,12 @@ hipError_t launch_batched(const BatchParams& P, int filter, int tfm, int blend, 
                           hipStream_t s, int* occ);
 // adds every volume's bricked gradient scratch into its gradient (after launch_batched)
 hipError_t launch_debrick(const DebrickSeg* dSegs, int nSegs, long long maxBricks, hipStream_t s);
+// the same for one call's gradient: `batches` scratch volumes of brick_floats() each, batch stride sb of the gradient
+hipError_t launch_debrick_call(const DebrickSeg& S, int batches, long long sb, hipStream_t s);
+// dvr_kernels_scatter.hip: the second pass of the volume gradients (P.parts is chosen here)
+hipError_t launch_scatter_volume(const ScatterParams& P, int filter, hipStream_t s);
+// clears n floats (a multiple of 4, 16-byte aligned) with a kernel
+hipError_t launch_clear(float* p, size_t n, hipStream_t s);
 
 // pre-shaded volumes (dvr_kernels_preshaded.hip): plain structure, inversion adjoint
 hipError_t launch_forward_preshaded(const RenderParams& P, int blend, hipStream_t s);

@@ -11,18 +11,31 @@ constexpr int kTileW = 8;         // pixels per workgroup tile (x)
 constexpr int kTileH = 8;         // pixels per workgroup tile (y)
 constexpr int kBlock = 64;        // threads per workgroup = one wave of 8x8 rays
 constexpr int kBatchBlock = 64;   // batched persistent kernel: one wave per workgroup, one wave tile per pop
-constexpr int kTfCopies = 8;      // batched kernel: copies of the LDS TF-gradient table, lane & 7 selects one
+constexpr int kTfCopies = 4;      // copies of the LDS TF-gradient table, lane & 3 selects one
+// LDS gradient sums are doubles: on MI355X a ds_add_f32 takes 3 clocks a lane (193 a full wave instruction),
+// ds_add_f64 16 to 20 a wave instruction (addresses on distinct banks or random; lanes on one address take
+// 3 to 4 clocks each either way).
+// TF gradients: doubles between the copies (odd: the copies start in different banks), 0 = one table (copies
+// would take more than 16 KiB); 8-byte aligned offset behind the TF table; floats in all
+constexpr int tf_grad_copy_stride(int RC) { return kTfCopies * (RC | 1) * 8 <= 16384 ? (RC | 1) : 0; }
+constexpr int tf_grad_offset(int tfFloats) { return (tfFloats + 1) & ~1; }
+constexpr int tf_grad_floats(int RC, bool priv, int threads, int stride)
+{
+    return priv ? RC * threads : 2 * (stride > 0 ? kTfCopies * stride : RC);
+}
 constexpr int kNumXcd = 8;        // MI355X: 8 XCDs, workgroups dispatched round-robin
 constexpr int kMaxTfLds = 4096;   // max R*C floats of a TF staged in LDS by the tiled kernels
 // LDS table of the volume-gradient aggregation (one per wave): 2^log2 slots of
-// one 64-byte chunk each, plus tags, slot list and 16 bytes of padding.  The per-call tiled
+// one 64-byte chunk (16 sums) each, plus tags, slot list and 16 bytes of padding.  The per-call tiled
 // adjoint uses kAggLog2 where it also carries the position adjoint; its volume +
 // TF instances and a batched plan take the largest table (kAggMinLog2 ..
-// kAggLog2) that keeps its instance at batched_vol_waves waves per SIMD.
+// kAggLog2) that keeps its instance at batched_vol_waves waves per SIMD.  The batched
+// tables sum in doubles (see kTfCopies): 8.05 instead of 8.82 ms for 40 views of five
+// volumes of 64^3 to 192^3, although half as many slots fit; where rays lie far apart
+// and the slots count (16.0 against 10.9 ms, 24 views of 256^3) plans take two passes.
 constexpr int kAggLog2 = 8;
 constexpr int kAggMinLog2 = 5;
-constexpr size_t agg_bytes(int log2) { return (size_t(1) << log2) * (4 + 4 + 16 * 4) + 16; }
-constexpr size_t kAggBytes = agg_bytes(kAggLog2);
+constexpr size_t agg_bytes(int log2, size_t sum) { return (size_t(1) << log2) * (4 + 4 + 16 * sum) + 16; }
 // Batched volume-gradient instances: waves per SIMD the compiler must fit
 // (registers).  Measured on C5 / C3 (linear / identity TF): the walk is bound by
 // latency at two waves per SIMD; four waves ran C5 in 105 ms (64-slot table)
@@ -75,6 +88,16 @@ struct AdjointParams {
     int tfDelayed;
 };
 
+// Density adjoints of every sample and the rays, stored by the reverse walk for k_scatter_volume.
+constexpr int kRayRecord = 9;   // floats of a ray: p0, dp, t0, step, samples (as bits)
+constexpr int kAdjSpill = 32;   // rows behind the samples: one segment past the capacity
+struct AdjStore {
+    float* adj;                 // [tile][cap + kAdjSpill][64] density adjoints, or NULL
+    float* rays;                // [tile][kRayRecord][64]
+    int cap;                    // samples per ray adj holds, a multiple of kAdjSpill
+};
+constexpr int adj_store_cap(int samples) { return (samples + kAdjSpill - 1) / kAdjSpill * kAdjSpill; }
+constexpr size_t adj_store_floats(int cap) { return size_t(cap + kAdjSpill + kRayRecord) * kBlock; }  // a tile
 // Checkpoints: ckpt c (0-based) of a ray holds the transmittance 1 - alpha
 // accumulated after (c+1)*K*every samples.  Layout [tile][c][thread] so one
 // wave stores 256 B.  The reverse march walks K-sample register segments.
@@ -85,6 +108,8 @@ struct CkptParams {
     int every;    // checkpoint interval in segments (1 or 2): interval = K*every
     float* ds;    // density store [tile][dsCap][kBlock] of the forward march, or NULL
     int dsCap;    // samples per ray it holds
+    AdjStore as;  // density adjoints of the launch's tiles (volume gradients in two passes), or NULL
+    int tile0, tileN;  // tiles of the launch (adjoint; tileN 0: all)
 };
 
 // Per-pixel loss whose gradient the fused forward+adjoint kernel forms in
@@ -130,11 +155,32 @@ struct BVol {
     float bmin[3], bsize[3];
 };
 
-// Bricked scratch of one volume gradient, added into the caller's gradient after the batched kernel
+// Bricked scratch of one volume gradient (2x2x4 voxels a 64-byte chunk), added into the caller's
+// gradient after the kernel that filled it
 struct DebrickSeg {
     const float* brick;
     float* adj;
     int X, Y, Z, pad0;
+    long long sx, sy, sz;       // element strides of adj
+};
+constexpr size_t brick_floats(int X, int Y, int Z)
+{
+    return size_t((X + 1) / 2) * size_t((Y + 1) / 2) * size_t((Z + 3) / 4) * 16;
+}
+
+// ---------------------------------------------------------------------------
+// Volume gradients in two passes: the reverse walk stores every sample's density
+// adjoint and the rays, and k_scatter_volume (dvr_kernels_scatter.hip) adds the
+// samples' corner gradients into bricked scratch.
+// ---------------------------------------------------------------------------
+struct ScatterParams {
+    AdjStore S;
+    int nTiles, parts;          // tiles of the store; workgroups that share a tile's samples
+    // the volume of a tile: of a view (views given, tile0 = number of the store's first tile), or of
+    // tile / tilesPerVolume
+    const struct BView* views; int nViews, tile0;
+    const struct BVol* vols;
+    float* brick; size_t brickFloats; int tilesPerVolume, X, Y, Z;
 };
 
 struct BTf {
@@ -151,6 +197,8 @@ struct BatchParams {
     float* ck;                  // checkpoints [workgroup][cap][kBatchBlock]
     float* ds;                  // sample densities [workgroup][dsCap][kBatchBlock] of the forward march, or NULL
     int dsCap;                  // samples per ray the density store holds
+    AdjStore as;                // density adjoints of the launch's tiles (volume gradients), or NULL
+    int tile0;                  // first tile of the launch
     float* lossOut;             // scalar loss accumulator or NULL
     int nViews, nTiles, ckCap;
     int ckEvery;                // checkpoint interval = K * ckEvery samples
@@ -162,7 +210,7 @@ struct BatchParams {
     int tileW, tileH;           // workgroup tile = one wave tile
     int ldsTf;                  // floats of the LDS TF table (max rows x the staged row stride)
     int usePriv;                // Gaussian TF gradient in per-thread LDS slices
-    int tfCopyStride;           // floats between the kTfCopies TF-gradient tables (0: one table)
+    int tfCopyStride;           // doubles between the kTfCopies TF-gradient tables (0: one table)
     int ldsAgg;                 // float offset of the volume-gradient chunk table in LDS (0: none)
     int aggLog2;                // log2 of the chunk table's slots
 };

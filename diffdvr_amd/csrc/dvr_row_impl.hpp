@@ -302,7 +302,7 @@ template <int FILTER, int TFM, int BLEND, int K, int GM, class Sink, class VS>
 __device__ __forceinline__ void split_reverse(const Vol& V, const Tf& T, const Ray& r, int s, int n, f4 adj_acc,
                                               const float* ck, int cap, int ckShift, Sink& sink, bool wantTf,
                                               bool wantVol, bool wantPos, VS& vs, f3& adj_start, f3& adj_dir,
-                                              float& adj_step, const float* dsr)
+                                              float& adj_step, const float* dsr, AdjLane<true> as)
 {
     const int nseg = (n + K - 1) / K;
     const int per = (nseg + kRow - 1) / kRow;
@@ -328,7 +328,7 @@ __device__ __forceinline__ void split_reverse(const Vol& V, const Tf& T, const R
     adj_acc.w = row_compose_behind(s, A, B, adj_acc.w);
     march_reverse<FILTER, TFM, BLEND, K, GM, Sink, false, VS>(V, T, r, end, adj_acc, ck, kBlock, cap, ckShift, sink,
                                                               wantTf, wantVol, wantPos, vs, adj_start, adj_dir,
-                                                              adj_step, dsr, kBlock, lo);
+                                                              adj_step, dsr, kBlock, lo, as);
 }
 
 template <int FILTER, int TFM, int BLEND>
@@ -371,21 +371,21 @@ __global__ __launch_bounds__(kRowAdjBlock) __attribute__((amdgpu_waves_per_eu(GM
     float* xc = s_x + (threadIdx.x / kRow) * kRowXchg;
     const int RC = P.R * P.C;
     float* s_tf = lds;
-    float* s_g = lds + RC;
+    float* s_g = lds + tf_grad_offset(RC);
     const RowXY tc = row_xy<kThreads>(tilesX, tilesPerView, nTiles);
     const bool wantTf = (GM & 1) && A.atf != nullptr;
-    const int ng = wantTf ? (usePriv ? RC * kThreads : (copyStride > 0 ? kTfCopies * copyStride : RC)) : 0;
+    const int ng = wantTf ? tf_grad_floats(RC, usePriv != 0, kThreads, copyStride) : 0;
     stage_tf(P, tc.b, s_tf);
     for (int e = threadIdx.x; e < ng; e += kThreads) s_g[e] = 0.0f;
     constexpr bool kVolInst = (GM & 2) != 0;
-    using VS = std::conditional_t<kVolInst, VolAgg<LinearLayout>, VolDirect>;
+    using VS = std::conditional_t<kVolInst, VolAgg<LinearLayout, float>, VolDirect>;
     VS vs;
     vs.L = LinearLayout{P.X, P.Y, P.Z, A.avSx, A.avSy, A.avSz};
     const bool aggOn = kVolInst && A.avol != nullptr;
     if constexpr (kVolInst) {
         if (aggOn) {
-            char* table = reinterpret_cast<char*>(lds + agg_offset(RC, ng));
-            vs.init(table + (threadIdx.x >> 6) * agg_bytes(aggLog2), aggLog2);
+            char* table = reinterpret_cast<char*>(lds + agg_offset(tf_grad_offset(RC), ng));
+            vs.init(table + (threadIdx.x >> 6) * agg_bytes(aggLog2, sizeof(float)), aggLog2);
             vs.bind(A.avol + tc.b * A.avSb);
         }
     } else {
@@ -452,10 +452,16 @@ __global__ __launch_bounds__(kRowAdjBlock) __attribute__((amdgpu_waves_per_eu(GM
         row_reverse<FILTER, TFM, BLEND>(V, T, r, tc.s, n, adj_acc, ck, CK.cap, ckShift, wantPos, adj_start, adj_dir,
                                         adj_step, dsr);
     } else {
+        AdjLane<true> as;
+        if constexpr ((GM & 8) != 0) {
+            vs.p = A.avol + b * A.avSb;
+            as = adj_store<true>(CK.as, tc.tile, tc.slot);
+            if (tc.s == 0) store_ray(CK.as, tc.tile, tc.slot, r, n);
+        }
         SinkTiled<TFM> sink;
         sink.init(s_g, kC, usePriv != 0, kThreads, usePriv ? 0 : copyStride);
         split_reverse<FILTER, TFM, BLEND, kRow, GM>(V, T, r, tc.s, n, adj_acc, ck, CK.cap, ckShift, sink, wantTf, aggOn,
-                                                    wantPos, vs, adj_start, adj_dir, adj_step, dsr);
+                                                    wantPos, vs, adj_start, adj_dir, adj_step, dsr, as);
         if constexpr (kVolInst) {
             if (aggOn) vs.flush();
         }
@@ -505,11 +511,7 @@ __global__ __launch_bounds__(kRowAdjBlock) __attribute__((amdgpu_waves_per_eu(GM
             }
         } else {
             for (int e = threadIdx.x; e < RC; e += kThreads) {
-                float v = s_g[e];
-                if (copyStride > 0) {
-#pragma unroll
-                    for (int k = 1; k < kTfCopies; ++k) v += s_g[k * copyStride + e];
-                }
+                const float v = tf_grad_sum(s_g, e, copyStride);
                 const int rr = e / P.C, cc = e - rr * P.C;
                 if (v != 0.0f) atomicAdd(g + rr * A.atfSr + cc * A.atfSc, v);
             }

@@ -25,10 +25,10 @@ struct TileXY {
     int tile, b, x, y;
 };
 
-__device__ __forceinline__ TileXY tile_xy(int tilesX, int tilesPerView, int nTiles)
+__device__ __forceinline__ TileXY tile_xy(int tilesX, int tilesPerView, int nTiles, int tile0 = 0)
 {
     TileXY t;
-    t.tile = xcd_remap(blockIdx.x, nTiles);
+    t.tile = tile0 + xcd_remap(blockIdx.x, nTiles);
     t.b = t.tile / tilesPerView;
     const int tl = t.tile - t.b * tilesPerView;
     const int ty = tl / tilesX, tx = tl - ty * tilesX;
@@ -104,15 +104,15 @@ __device__ __forceinline__ void march_forward(const Vol& V, const Tf& T, const R
 //   texture / linear : per-lane cache of the two most recent rows (densities
 //       change slowly along a ray), flushed into a workgroup LDS table with
 //       LDS atomics only when a row leaves (a move by one texel keeps the
-//       shared row); the batched kernel spreads the atomics of a wave over
-//       kTfCopies copies of the table (neighbouring rays hit the same rows)
+//       shared row), spread over kTfCopies copies of the table (neighbouring
+//       rays hit the same rows)
 //   gaussian : every sample touches every entry; per-thread private LDS slices
 //       (entry-major, conflict-free) when they fit, else LDS atomics
 // ---------------------------------------------------------------------------
 template <int TFM>
 struct SinkTiled {
-    float* tab;   // workgroup table (R*C) or private slice base (priv)
-    float* tabc;  // this lane's copy of the table (copies: lanes of one wave spread their LDS atomics)
+    float* tab;   // private slice base (priv)
+    double* tabc; // this lane's copy of the workgroup's table (lanes of one wave spread their LDS atomics)
     int C;
     int nthreads; // threads of the workgroup (slice stride of the private slices)
     bool priv;
@@ -120,11 +120,11 @@ struct SinkTiled {
     float a0[5], a1[5];
     float id0, id1;
 
-    // copyStride > 0: kTfCopies tables copyStride floats apart, lane & (kTfCopies-1) adds to its own
+    // copyStride > 0: kTfCopies tables copyStride doubles apart, lane & (kTfCopies-1) adds to its own
     __device__ __forceinline__ void init(float* table, int C_, bool usePriv, int threads = kBlock, int copyStride = 0)
     {
         tab = table; C = C_; priv = usePriv; nthreads = threads;
-        tabc = table + (copyStride > 0 ? int(threadIdx.x & (kTfCopies - 1)) * copyStride : 0);
+        tabc = reinterpret_cast<double*>(table) + (copyStride > 0 ? int(threadIdx.x & (kTfCopies - 1)) * copyStride : 0);
         r0 = r1 = -1;
 #pragma unroll
         for (int k = 0; k < 5; ++k) { a0[k] = 0.f; a1[k] = 0.f; }
@@ -136,7 +136,7 @@ struct SinkTiled {
             if (c == 0) id0 += v; else id1 += v;
         } else {
             if (priv) tab[(r * C + c) * nthreads + threadIdx.x] += v;
-            else atomicAdd(&tabc[r * C + c], v);
+            else atomicAdd(&tabc[r * C + c], double(v));
         }
     }
     template <int NC>
@@ -144,7 +144,7 @@ struct SinkTiled {
     {
         if (r >= 0) {
 #pragma unroll
-            for (int c = 0; c < NC; ++c) atomicAdd(&tabc[r * C + c], a[c]);
+            for (int c = 0; c < NC; ++c) atomicAdd(&tabc[r * C + c], double(a[c]));
         }
 #pragma unroll
         for (int k = 0; k < 5; ++k) a[k] = 0.f;
@@ -182,8 +182,8 @@ struct SinkTiled {
         if constexpr (TFM == 0) {
             const float s0 = wave_sum(id0), s1 = wave_sum(id1);
             if ((threadIdx.x & 63) == 0) {
-                atomicAdd(&tab[0], s0);
-                atomicAdd(&tab[1], s1);
+                atomicAdd(&tabc[0], double(s0));
+                atomicAdd(&tabc[1], double(s1));
             }
         } else if constexpr (TFM == 1 || TFM == 2) {
             flush_row<NC>(r0, a0);
@@ -191,6 +191,18 @@ struct SinkTiled {
         }
     }
 };
+
+// sum of entry e over the copies of the workgroup's table
+__device__ __forceinline__ float tf_grad_sum(const float* s_g, int e, int copyStride)
+{
+    const double* t = reinterpret_cast<const double*>(s_g) + e;
+    double v = t[0];
+    if (copyStride > 0) {
+#pragma unroll
+        for (int k = 1; k < kTfCopies; ++k) v += t[k * copyStride];
+    }
+    return float(v);
+}
 
 // ---------------------------------------------------------------------------
 // Reverse-walk cell state of the volume and position adjoints.  Consecutive
@@ -296,10 +308,11 @@ struct BrickLayout {
     __device__ __forceinline__ unsigned point(int x, int y, int z) const { return xp(x) + yp(y) + zp(z); }
 };
 
-struct VolDirect {
+template <class Layout>
+struct VolDirectT {
     static constexpr bool kAgg = false;
     float* p;
-    LinearLayout L;
+    Layout L;
     __device__ __forceinline__ void add(unsigned off, float v)
     {
         if (v != 0.f) gatomic_add(p, off, v);
@@ -317,20 +330,42 @@ struct VolDirect {
     }
     __device__ __forceinline__ void maybe_flush() {}
 };
+using VolDirect = VolDirectT<LinearLayout>;
 
-template <class Layout>
+// The corner gradients of one sample, straight to device memory: the samples past the capacity of a
+// density-adjoint store (rays whose direction is shorter than 1 have more than the box bounds).
+template <int FILTER, class VS>
+__device__ __forceinline__ void add_sample(VS& vs, const Vol& V, const f3& p, float v)
+{
+    if constexpr (FILTER == 0) {
+        int x, y, z;
+        nearest_index(p, V.X, V.Y, V.Z, x, y, z);
+        vs.add(vs.L.point(x, y, z), v);
+    } else {
+        const int ix = int(p.x), iy = int(p.y), iz = int(p.z);
+        const CornerIdx o = vs.L.cell(ix, iy, iz);
+        const float fx = p.x - float(ix), fy = p.y - float(iy), fz = p.z - float(iz);
+#pragma unroll 1
+        for (int k = 0; k < 8; ++k) {
+            const unsigned off = ((k & 4) ? o.x[1] : o.x[0]) + ((k & 2) ? o.y[1] : o.y[0]) + ((k & 1) ? o.z[1] : o.z[0]);
+            vs.add(off, v * ((k & 4) ? fx : 1.f - fx) * ((k & 2) ? fy : 1.f - fy) * ((k & 1) ? fz : 1.f - fz));
+        }
+    }
+}
+
+template <class Layout, class Sum>
 struct VolAgg {
     static constexpr bool kAgg = true;
     unsigned lg;      // log2 of the slot count (uniform)
     Layout L;         // element offsets of the gradient the table adds into
     unsigned* tags;   // [slots] chunk index, kAggEmpty = free
     unsigned* list;   // [slots] occupied slots, listed by the flush
-    float* vals;      // [slots][16]
+    Sum* vals;        // [slots][16]
     float* abase;     // gradient base rounded down to 64 bytes (never dereferenced below the base)
     unsigned boff;    // floats from abase to the gradient base
 
     __device__ __forceinline__ unsigned slots() const { return 1u << lg; }
-    // every lane of the wave that owns the table; lds is 16-byte aligned, agg_bytes(log2) long
+    // every lane of the wave that owns the table; lds is 16-byte aligned, agg_bytes(log2, sizeof(Sum)) long
     __device__ __forceinline__ void init(void* lds, int log2)
     {
         const unsigned lane = threadIdx.x & 63u;
@@ -338,9 +373,9 @@ struct VolAgg {
         const unsigned kSlots = slots();
         tags = (unsigned*)lds;
         list = tags + kSlots;
-        vals = (float*)(list + kSlots + 4);  // 16 bytes of padding after the list
+        vals = (Sum*)(list + kSlots + 4);  // 16 bytes of padding after the list
         for (unsigned e = lane; e < kSlots; e += 64u) tags[e] = kAggEmpty;
-        for (unsigned e = lane; e < kSlots * 16; e += 64u) vals[e] = 0.f;
+        for (unsigned e = lane; e < kSlots * 16; e += 64u) vals[e] = Sum(0);
     }
     // the table must be empty (flushed) when the base changes
     __device__ __forceinline__ void bind(float* g)
@@ -375,7 +410,7 @@ struct VolAgg {
     }
     __device__ __forceinline__ void put(unsigned s, unsigned e, float v)
     {
-        if (s != kAggEmpty) atomicAdd(&vals[s * 16 + (e & 15)], v);
+        if (s != kAggEmpty) atomicAdd(&vals[s * 16 + (e & 15)], Sum(v));
         else gatomic_add(abase, e, v);
     }
     __device__ __forceinline__ void add(unsigned off, float v)
@@ -433,9 +468,9 @@ struct VolAgg {
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
         for (unsigned e = rank; e < n * 16u; e += cnt) {
             const unsigned s = list[e >> 4], j = e & 15u;
-            const float v = vals[s * 16 + j];
-            if (v != 0.f) gatomic_add(abase, tags[s] * 16u + j, v);
-            vals[s * 16 + j] = 0.f;
+            const Sum v = vals[s * 16 + j];
+            if (v != Sum(0)) gatomic_add(abase, tags[s] * 16u + j, float(v));
+            vals[s * 16 + j] = Sum(0);
         }
         for (unsigned e = rank; e < n; e += cnt) tags[list[e]] = kAggEmpty;
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
@@ -556,20 +591,45 @@ __device__ __forceinline__ void corner_move(CornerCache& c, const Vol& V, VS& vs
     c.cx = ix; c.cy = iy; c.cz = iz;
 }
 
+// The ray of a tile's lane `slot` for k_scatter_volume (n = 0 outside the image).
+__device__ __forceinline__ void store_ray(const AdjStore& S, int storeTile, int slot, const Ray& r, int n)
+{
+    float* o = S.rays + size_t(storeTile) * (kRayRecord * kBlock) + slot;
+    o[0] = r.p0.x; o[kBlock] = r.p0.y; o[2 * kBlock] = r.p0.z;
+    o[3 * kBlock] = r.dp.x; o[4 * kBlock] = r.dp.y; o[5 * kBlock] = r.dp.z;
+    o[6 * kBlock] = r.t0; o[7 * kBlock] = r.step; o[8 * kBlock] = __int_as_float(n);
+}
+// The density adjoints of that lane: sample i at [i * kBlock] for i < cap.  A walk of whole rays puts a
+// segment past cap (a multiple of every segment length) into the rows behind and adds its corner
+// gradients to device memory after it; the lanes of a row, which share the ray's rows, add each sample.
+template <bool SHARED>
+struct AdjLane {
+    static constexpr bool kShared = SHARED;
+    float* p = nullptr;
+    int cap = 0;
+};
+template <bool SHARED>
+__device__ __forceinline__ AdjLane<SHARED> adj_store(const AdjStore& S, int storeTile, int slot)
+{
+    return {S.adj + size_t(storeTile) * (size_t(S.cap + kAdjSpill) * kBlock) + slot, S.cap};
+}
+
 // ---------------------------------------------------------------------------
 // Reverse march of one ray with transmittance checkpoints every 2^ckShift
 // samples, walked back in register segments of K samples, from the one that
 // holds sample n - 1 down to segment segLo.  GM is the set of gradient
-// kinds compiled in: bit0 TF, bit1 volume, bit2 position (camera / step);
-// the runtime flags select among them.
+// kinds compiled in: bit0 TF, bit1 volume, bit2 position (camera / step), bit3
+// density adjoints stored for k_scatter_volume; the runtime flags select among them.
 // ---------------------------------------------------------------------------
-template <int FILTER, int TFM, int BLEND, int K, int GM, class Sink, bool SPLIT = false, class VS = VolDirect>
+template <int FILTER, int TFM, int BLEND, int K, int GM, class Sink, bool SPLIT = false, class VS = VolDirect,
+          class AL = AdjLane<false>>
 __device__ __forceinline__ void march_reverse(const Vol& V, const Tf& T, const Ray& r, int n, f4 adj_acc,
                                               const float* ck, int ckS, int cap, int ckShift, Sink& sink,
                                               bool wantTf,
                                               bool wantVol, bool wantPos, VS& vs,
                                               f3& adj_start, f3& adj_dir, float& adj_step,
-                                              const float* dsr = nullptr, int dsS = 0, int segLo = 0)
+                                              const float* dsr = nullptr, int dsS = 0, int segLo = 0,
+                                              AL as = {})
 {
     constexpr bool CT_TF = (GM & 1) != 0, CT_VOL = (GM & 2) != 0, CT_POS = (GM & 4) != 0;
     wantTf = CT_TF && wantTf;
@@ -601,6 +661,7 @@ __device__ __forceinline__ void march_reverse(const Vol& V, const Tf& T, const R
     for (int seg = nseg - 1; seg >= segLo; --seg) {
         const int i0 = seg * K;
         const int cnt = min(K, n - i0);
+        gfloat* const adjRow = (gfloat*)(as.p + (AL::kShared ? i0 : min(i0, as.cap)) * kBlock);
         // transmittance before sample i0
         float Tr = 1.0f;
         {
@@ -691,6 +752,12 @@ __device__ __forceinline__ void march_reverse(const Vol& V, const Tf& T, const R
                 SinkNone none;
                 adj_d = tf_adjoint<TFM, false, SinkNone, true>(T, dv[j], adj_s, none, &pre);
             }
+            if constexpr ((GM & 8) != 0) {
+                if (as.p) {
+                    if (!AL::kShared || i < as.cap) adjRow[j * kBlock] = adj_d;
+                    else add_sample<FILTER>(vs, V, sample_pos(r, t), adj_d);
+                }
+            }
             if constexpr (CT_VOL || CT_POS) {
                 if (wantVol || wantPos) {
                     const f3 p = sample_pos(r, t);
@@ -756,6 +823,14 @@ __device__ __forceinline__ void march_reverse(const Vol& V, const Tf& T, const R
                     if (j < cnt) walk(j);
             }
         }
+        if constexpr ((GM & 8) != 0 && !AL::kShared) {
+            if (as.p && i0 >= as.cap) {
+#pragma unroll 1
+                for (int j = 0; j < cnt; ++j)
+                    add_sample<FILTER>(vs, V, sample_pos(r, r.t0 + float(i0 + j) * r.step),
+                                       adjRow[j * kBlock]);
+            }
+        }
     }
     if constexpr (CT_VOL) {
         if (wantVol) {
@@ -806,28 +881,29 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(GM == 3 
     extern __shared__ float lds[];
     const int RC = P.R * P.C;
     float* s_tf = lds;
-    float* s_g = lds + RC;
-    const TileXY tc = tile_xy(tilesX, tilesPerView, nTiles);
+    float* s_g = lds + tf_grad_offset(RC);
+    const int copyStride = tf_grad_copy_stride(RC);
+    const TileXY tc = tile_xy(tilesX, tilesPerView, nTiles, CK.tile0);
     const bool wantTf = A.atf != nullptr;
-    const int ng = wantTf ? (usePriv ? RC * kBlock : RC) : 0;
+    const int ng = wantTf ? tf_grad_floats(RC, usePriv != 0, kBlock, copyStride) : 0;
     stage_tf(P, tc.b, s_tf);
     for (int e = threadIdx.x; e < ng; e += kBlock) s_g[e] = 0.0f;
     // volume gradient: the wave's corner values are summed per 64-byte chunk in LDS
     constexpr bool kVolInst = (GM & 2) != 0;
-    using VS = std::conditional_t<kVolInst, VolAgg<LinearLayout>, VolDirect>;
+    using VS = std::conditional_t<kVolInst, VolAgg<LinearLayout, float>, VolDirect>;
     VS vs;
     vs.L = LinearLayout{P.X, P.Y, P.Z, A.avSx, A.avSy, A.avSz};
     const bool aggOn = kVolInst && A.avol != nullptr;
     if constexpr (kVolInst) {
         if (aggOn) {
-            vs.init(lds + agg_offset(RC, ng), aggLog2);
+            vs.init(lds + agg_offset(tf_grad_offset(RC), ng), aggLog2);
             vs.bind(A.avol + tc.b * A.avSb);
         }
     }
     __syncthreads();
 
     SinkTiled<TFM> sink;
-    sink.init(s_g, tf_cols<TFM>(), usePriv != 0);
+    sink.init(s_g, tf_cols<TFM>(), usePriv != 0, kBlock, usePriv ? 0 : copyStride);
     float lossLocal = 0.0f;
     const bool valid = tc.x < P.W && tc.y < P.H;
     if (valid) {
@@ -874,15 +950,21 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(GM == 3 
         f3 adj_start = mk3(0.f, 0.f, 0.f), adj_dir = mk3(0.f, 0.f, 0.f);
         float adj_step = 0.0f;
         const bool wantVol = A.avol != nullptr;
+        AdjLane<false> as;
+        if constexpr ((GM & 8) != 0) {
+            vs.p = A.avol + tc.b * A.avSb;
+            as = adj_store<false>(CK.as, tc.tile - CK.tile0, threadIdx.x);
+            store_ray(CK.as, tc.tile - CK.tile0, threadIdx.x, r, n);
+        }
         const bool wantPos = A.ars != nullptr || A.ast != nullptr;
         const bool stored = ds != nullptr && __all(n <= CK.dsCap);  // uniform over the wave
         // the split walk (a second, predicate-free copy for segments full on every lane) pays off
         // except for the arithmetic-bound Gaussian TF
-        if constexpr (!kVolInst) vs.p = nullptr;
+        if constexpr (!kVolInst && (GM & 8) == 0) vs.p = nullptr;
         march_reverse<FILTER, TFM, BLEND, K, GM, SinkTiled<TFM>, TFM != 3, VS>(V, T, r, n, adj_acc, ck, kBlock, CK.cap,
                                                                                __builtin_ctz(K * CK.every), sink, wantTf, wantVol,
                                                  wantPos, vs, adj_start, adj_dir, adj_step, stored ? ds : nullptr,
-                                                 kBlock);
+                                                 kBlock, 0, as);
         if (A.ast) {
             float* o = A.ast + b * A.astSb + y * A.astSy + x * A.astSx;
             if (A.stepBroadcast) atomicAdd(o, adj_step);
@@ -899,6 +981,9 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(GM == 3 
                 od[0] = adj_dir.x; od[A.ardSc] = adj_dir.y; od[2 * A.ardSc] = adj_dir.z;
             }
         }
+    }
+    if constexpr ((GM & 8) != 0) {
+        if (!valid) store_ray(CK.as, tc.tile - CK.tile0, threadIdx.x, Ray{}, 0);
     }
     if constexpr (kVolInst) {
         if (aggOn) vs.flush();
@@ -917,7 +1002,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(GM == 3 
                 v = 0.0f;
                 for (int t = 0; t < kBlock; ++t) v += s_g[e * kBlock + t];
             } else {
-                v = s_g[e];
+                v = tf_grad_sum(s_g, e, copyStride);
             }
             const int rr = e / P.C, cc = e - rr * P.C;
             if (v != 0.0f) atomicAdd(g + rr * A.atfSr + cc * A.atfSc, v);
@@ -933,26 +1018,26 @@ static hipError_t adj_tiled_k(const RenderParams& P, const AdjointParams& A, con
                               bool fused, bool ckFromFwd, hipStream_t s)
 {
     const int tilesX = (P.W + kTileW - 1) / kTileW, tilesY = (P.H + kTileH - 1) / kTileH;
-    const int nTiles = tilesX * tilesY * P.B;
+    const int nTiles = CK.tileN > 0 ? CK.tileN : tilesX * tilesY * P.B;
     if (nTiles == 0) return hipSuccess;
     const int RC = P.R * P.C;
     const bool usePriv = (TFM == 3) && A.atf && RC <= 48;  // private slices <= 48 KiB of LDS
-    const int ng = A.atf ? (usePriv ? RC * kBlock : RC) : 0;
+    const int ng = A.atf ? tf_grad_floats(RC, usePriv, kBlock, tf_grad_copy_stride(RC)) : 0;
     int aggLog2 = kAggLog2;
     size_t lds;
     if ((GM & 2) && A.avol) {
-        const size_t base = sizeof(float) * size_t(agg_offset(RC, ng));
+        const size_t base = sizeof(float) * size_t(agg_offset(tf_grad_offset(RC), ng));
         if (GM == 3) {
             // the largest chunk table beside the TF tables that leaves room for sixteen one-wave
             // workgroups per CU (the four waves per SIMD the instance's registers allow)
-            while (aggLog2 > kAggMinLog2 && base + agg_bytes(aggLog2) > size_t(kLdsPerCu) / kTiledVolWgPerCu)
+            while (aggLog2 > kAggMinLog2 && base + agg_bytes(aggLog2, sizeof(float)) > size_t(kLdsPerCu) / kTiledVolWgPerCu)
                 --aggLog2;
-            lds = base + agg_bytes(aggLog2);
+            lds = base + agg_bytes(aggLog2, sizeof(float));
         } else {
-            lds = occupancy_lds(base + agg_bytes(aggLog2), tiled_wg_per_cu(TFM));
+            lds = occupancy_lds(base + agg_bytes(aggLog2, sizeof(float)), tiled_wg_per_cu(TFM));
         }
     } else {
-        lds = occupancy_lds(sizeof(float) * (size_t(RC) + size_t(ng)), tiled_wg_per_cu(TFM));
+        lds = occupancy_lds(sizeof(float) * size_t(tf_grad_offset(RC) + ng), tiled_wg_per_cu(TFM));
     }
     hipLaunchKernelGGL((k_adjoint_tiled<FILTER, TFM, BLEND, K, GM>), dim3(nTiles), dim3(kBlock), lds, s, P, A, CK, L,
                        fused ? 1 : 0, ckFromFwd ? 1 : 0, usePriv ? 1 : 0, tilesX, tilesX * tilesY, nTiles, aggLog2);
@@ -962,9 +1047,10 @@ static hipError_t adj_tiled_k(const RenderParams& P, const AdjointParams& A, con
 // gradient kinds compiled into the instance: TF only, volume (+TF), position (+TF), or everything
 // (camera / step gradients without volume gradients run an instance compiled
 // without the volume-gradient code: fewer registers)
-inline int tiled_grad_mask(const AdjointParams& A)
+inline int tiled_grad_mask(const AdjointParams& A, const CkptParams& CK)
 {
     const bool pos = A.ars || A.ast;
+    if (A.avol && CK.as.adj) return pos ? 13 : 9;  // volume gradients in two passes
     return pos ? (A.avol ? 7 : 5) : (A.avol ? 3 : 1);
 }
 
@@ -972,11 +1058,13 @@ template <int FILTER, int BLEND, int K>
 static hipError_t adj_tiled_fbk(const RenderParams& P, const AdjointParams& A, const CkptParams& CK,
                                 const LossParams& L, bool fused, bool ckFromFwd, int tfm, hipStream_t s)
 {
-    const int gm = tiled_grad_mask(A);
+    const int gm = tiled_grad_mask(A, CK);
 #define DVR_GM_CASES(TV)                                                                              \
     if (gm == 1) return adj_tiled_k<FILTER, TV, BLEND, K, 1>(P, A, CK, L, fused, ckFromFwd, s);      \
     if (gm == 3) return adj_tiled_k<FILTER, TV, BLEND, K, 3>(P, A, CK, L, fused, ckFromFwd, s);      \
     if (gm == 5) return adj_tiled_k<FILTER, TV, BLEND, K, 5>(P, A, CK, L, fused, ckFromFwd, s);      \
+    if (gm == 9) return adj_tiled_k<FILTER, TV, BLEND, K, 9>(P, A, CK, L, fused, ckFromFwd, s);      \
+    if (gm == 13) return adj_tiled_k<FILTER, TV, BLEND, K, 13>(P, A, CK, L, fused, ckFromFwd, s);    \
     return adj_tiled_k<FILTER, TV, BLEND, K, 7>(P, A, CK, L, fused, ckFromFwd, s);
     switch (tfm) {
     case 0: { DVR_GM_CASES(0) }

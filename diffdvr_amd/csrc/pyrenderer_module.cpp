@@ -85,6 +85,7 @@ struct ForwardDifferencesSettings {
 // ---------------------------------------------------------------------------
 struct TorchInfo {
     py::object torch, cuda_current_stream, cuda_current_device, float32, int32, float64, bool_;
+    py::object empty, uint8, out_of_memory;
 };
 TorchInfo& torch_info()
 {
@@ -98,6 +99,9 @@ TorchInfo& torch_info()
         t->int32 = t->torch.attr("int32");
         t->float64 = t->torch.attr("float64");
         t->bool_ = t->torch.attr("bool");
+        t->empty = t->torch.attr("empty");
+        t->uint8 = t->torch.attr("uint8");
+        t->out_of_memory = t->torch.attr("OutOfMemoryError");
     }
     return *t;
 }
@@ -135,6 +139,28 @@ dvr_tensor to_tensor(const py::handle& h)
     }
     return t;
 }
+
+// Scratch of one call on the current stream from torch's caching allocator, given back when the call's
+// work is enqueued (the allocator reuses it in stream order).  None where memory is short: the call
+// then runs the kernels that need no scratch.
+struct CallScratch {
+    py::object tensor = py::none();
+    void* data = nullptr;
+    int64_t bytes = 0;
+    CallScratch(int64_t want, const py::object& like)
+    {
+        if (want <= 0) return;
+        TorchInfo& ti = torch_info();
+        try {
+            tensor = ti.empty(want, py::arg("dtype") = ti.uint8, py::arg("device") = like.attr("device"));
+        } catch (py::error_already_set& e) {
+            if (!e.matches(ti.out_of_memory)) throw;
+            return;
+        }
+        data = reinterpret_cast<void*>(tensor.attr("data_ptr")().cast<uintptr_t>());
+        bytes = want;
+    }
+};
 
 void* current_stream(int device)
 {
@@ -559,7 +585,9 @@ PYBIND11_MODULE(_pyrenderer, m)
               opt.checkpoint_interval = checkpoint_interval;
               opt.checkpoints = to_tensor(checkpoints);
               opt.densities = to_tensor(densities);
-              check(dvr_render_adjoint_ex(&p.in, &o, &ac, &ao, &opt, current_stream(p.in.volume.device)));
+              const CallScratch scr(dvr_adjoint_scratch_bytes(&p.in, &o, &ac, &ao, &opt), inputs.volume);
+              check(dvr_render_adjoint_scratch(&p.in, &o, &ac, &ao, &opt, scr.data, scr.bytes,
+                                               current_stream(p.in.volume.device)));
           },
           py::arg("inputs"), py::arg("outputs_from_forward"), py::arg("adj_color"), py::arg("adj_outputs"),
           py::arg("method") = "auto", py::arg("path") = "auto", py::arg("checkpoint_interval") = 0,

@@ -188,6 +188,18 @@ dvr_status dvr_render_adjoint_ex(const dvr_inputs* inputs, const dvr_outputs* ou
                                  const dvr_tensor* adj_color, dvr_adjoint_outputs* adj_outputs,
                                  const dvr_adjoint_options* options, void* stream);
 
+/* dvr_render_adjoint_ex with device scratch of the caller's (256-byte aligned, used on `stream` until the
+ * call's work is done, contents undefined before and after).  dvr_adjoint_scratch_bytes says how much a call
+ * would use (0: none; -1: the arguments are invalid).  Results are the same up to the order of float sums;
+ * with less scratch, or NULL, the call runs the kernels that need none. */
+int64_t dvr_adjoint_scratch_bytes(const dvr_inputs* inputs, const dvr_outputs* outputs_from_forward,
+                                  const dvr_tensor* adj_color, const dvr_adjoint_outputs* adj_outputs,
+                                  const dvr_adjoint_options* options);
+dvr_status dvr_render_adjoint_scratch(const dvr_inputs* inputs, const dvr_outputs* outputs_from_forward,
+                                      const dvr_tensor* adj_color, dvr_adjoint_outputs* adj_outputs,
+                                      const dvr_adjoint_options* options, void* scratch, int64_t scratch_bytes,
+                                      void* stream);
+
 /* Per-pixel image loss whose gradient the fused kernels form in registers. */
 #define DVR_LOSS_L1 1 /* mean |color - target|   (torch.nn.L1Loss)  */
 #define DVR_LOSS_L2 2 /* mean (color - target)^2 (torch.nn.MSELoss) */
