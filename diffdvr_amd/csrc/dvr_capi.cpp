@@ -562,64 +562,23 @@ void check_stamp(const void* ck, int K, const Checked& c, const void* densities)
         fail(DVR_ERR_INVALID_ARGUMENT, "densities were not written by the forward that wrote these checkpoints");
 }
 
-void do_forward(const dvr_inputs* inputs, dvr_outputs* outputs, const dvr_forward_options* opt, void* stream)
-{
-    Checked c = check_inputs(inputs);
-    check_outputs(outputs, c);
-    int path = opt ? opt->path : DVR_PATH_AUTO;
-    const int K = opt ? opt->checkpoint_interval : 0;
-    if (path == DVR_PATH_AUTO) path = tiled_ok(c) ? DVR_PATH_TILED : DVR_PATH_PLAIN;
-    if (c.preshaded && (path != DVR_PATH_PLAIN || K > 0))
-        fail(DVR_ERR_UNSUPPORTED, "pre-shaded volumes render on the plain path only");
-    DeviceGuard g(c.device);
-    hipStream_t s = (hipStream_t)stream;
-    if (path == DVR_PATH_TILED && !tiled_ok(c))
-        fail(DVR_ERR_UNSUPPORTED, "tiled path needs R*C <= %d transfer-function entries", dvr::kMaxTfLds);
-    if (K > 0) {
-        if (path != DVR_PATH_TILED) fail(DVR_ERR_UNSUPPORTED, "checkpoints are written by the tiled forward only");
-        make_ckpt(c, K);  // validates K
-        const dvr_tensor& ck = opt->checkpoints;
-        const int64_t need = (int64_t)dvr::tiled_num_tiles(c.P) * checkpoint_cap(c, K) * dvr::kBlock;
-        if (!given(ck) || ck.dtype != DVR_FLOAT32 || ck.device != c.device)
-            fail(DVR_ERR_INVALID_ARGUMENT, "checkpoints must be a float32 tensor on the render device");
-        int64_t numel = 1;
-        for (int d = 0; d < ck.ndim; ++d) numel *= ck.sizes[d];
-        if (numel < need) fail(DVR_ERR_INVALID_ARGUMENT, "checkpoints needs %lld elements, has %lld", (long long)need, (long long)numel);
-        if (ck.ndim > 0 && ck.strides[ck.ndim - 1] != 1 && numel > 1)
-            fail(DVR_ERR_INVALID_ARGUMENT, "checkpoints must be contiguous");
-        if (given(opt->densities)) density_buffer(opt->densities, c);
-    } else if (opt && given(opt->densities)) {
-        fail(DVR_ERR_INVALID_ARGUMENT, "densities are written together with checkpoints (checkpoint_interval > 0)");
-    }
-    if (c.preshaded) {
-        check_hip(dvr::launch_forward_preshaded(c.P, c.blend, s), "forward (pre-shaded) launch");
-    } else if (path == DVR_PATH_PLAIN) {
-        check_hip(dvr::launch_forward_plain(c.P, c.filter, c.tfm, c.blend, s), "forward (plain) launch");
-    } else {
-        dvr::CkptParams CK{nullptr, 16, 0, 1};
-        if (K > 0) {
-            CK = make_ckpt(c, K);
-            CK.buf = (float*)opt->checkpoints.data;
-            if (given(opt->densities)) {
-                CK.ds = density_buffer(opt->densities, c);
-                CK.dsCap = density_cap(c);
-            }
-        }
-        check_hip(dvr::launch_forward_tiled(c.P, CK, c.filter, c.tfm, c.blend, s), "forward (tiled) launch");
-        if (K > 0) stamp_checkpoints(CK.buf, CkptStamp{K, c.B, c.H, c.W, CK.ds});
-    }
-}
-
 // Device scratch of one call.
 struct Scratch {
     void* data = nullptr;
     size_t bytes = 0;
 };
 
-// no two indices of the X x Y x Z (x B) gradient share an element (an expanded tensor takes atomics)
-bool distinct_elements(const Checked& c, const dvr::AdjointParams& A)
+Scratch call_scratch(void* data, int64_t bytes)
 {
-    std::pair<int64_t, int64_t> d[4] = {{A.avSx, c.X}, {A.avSy, c.Y}, {A.avSz, c.Z}, {A.avSb, A.avSb != 0 ? c.B : 1}};
+    if (bytes > 0 && (reinterpret_cast<uintptr_t>(data) & 255u) != 0)
+        fail(DVR_ERR_INVALID_ARGUMENT, "scratch must be 256-byte aligned");
+    return {data, data ? size_t(std::max<int64_t>(bytes, 0)) : 0};
+}
+
+// no two indices of the X x Y x Z (x B) gradient share an element (an expanded tensor takes atomics)
+bool distinct_elements(const Checked& c, const dvr::AdjointParams& A, int volumes)
+{
+    std::pair<int64_t, int64_t> d[4] = {{A.avSx, c.X}, {A.avSy, c.Y}, {A.avSz, c.Z}, {A.avSb, volumes}};
     std::sort(d, d + 4);
     int64_t reach = 0;  // largest offset of the dimensions so far
     for (const auto& [stride, n] : d) {
@@ -634,14 +593,17 @@ bool distinct_elements(const Checked& c, const dvr::AdjointParams& A)
 // the density adjoints of a group of tiles and their rays, k_scatter_volume adds them into bricked
 // scratch, and after the last group k_debrick adds that into the caller's gradient.  Scratch layout:
 // [bricks][rays][density adjoints], each 64-byte aligned.
+constexpr size_t kMaxStore = size_t(2) << 30;  // bytes of a group's store
+
 class TwoPassGradient {
 public:
     TwoPassGradient(const Checked& c, const dvr::AdjointParams& A) : c_(c), A_(A)
     {
         // the store holds the longest ray of a uniform box and step; clearing and adding the bricks
         // (16 bytes a voxel) pays from a few samples per ten voxels on
-        if (!A.avol || c.preshaded || c.P.st || c.P.bsize || !distinct_elements(c, A)) return;
+        if (!A.avol || c.preshaded || c.P.st || c.P.bsize) return;
         volumes_ = A.avSb != 0 ? c.B : 1;
+        if (!distinct_elements(c, A, volumes_)) return;
         const double voxels = double(c.X) * c.Y * c.Z * volumes_;
         tiles_ = dvr::tiled_num_tiles(c.P);
         cap_ = dvr::adj_store_cap(density_cap(c));
@@ -687,12 +649,138 @@ public:
     }
 
 private:
-    static constexpr size_t kMaxStore = size_t(2) << 30;
     const Checked& c_;
     const dvr::AdjointParams& A_;
     int volumes_ = 1, tiles_ = 0, cap_ = 0, group_ = 0;
     size_t brickFloats_ = 0, bytes_ = 0;
 };
+
+// The packed kernels of pre-shaded volumes (A NULL: the forward).  Scratch layout: [RGBA volume], and for
+// volume gradients [four bricked gradients][rays][colour adjoints, a plane per channel] of a group of tiles.
+class PackedPreshaded {
+public:
+    PackedPreshaded(const Checked& c, const dvr::AdjointParams* A) : c_(c), A_(A)
+    {
+        // packing moves 32 bytes a voxel: the rule of TwoPassGradient
+        const double voxels = double(c.X) * c.Y * c.Z;
+        cap_ = dvr::adj_store_cap(density_cap(c));
+        tiles_ = group_ = dvr::tiled_num_tiles(c.P);
+        if (tiles_ == 0 || double(c.B) * c.W * c.H * cap_ * 0.5 < 0.25 * voxels || voxels >= double(1 << 28)) return;
+        packed_ = size_t(c.X) * c.Y * c.Z * 4;
+        size_t perTile = 0;
+        if (A && A->avol) {
+            if (!distinct_elements(c, *A, 4)) return;
+            perTile = size_t(dvr::kRayRecord + 4 * (cap_ + dvr::kAdjSpill)) * dvr::kBlock;
+            group_ = int(std::min<size_t>(size_t(tiles_), kMaxStore / (perTile * sizeof(float))));
+            brickFloats_ = dvr::brick_floats(c.X, c.Y, c.Z);
+            if (group_ < std::min(tiles_, 4096) || brickFloats_ >= (size_t(1) << 30)) return;
+        }
+        bytes_ = sizeof(float) * (packed_ + 4 * brickFloats_ + size_t(group_) * perTile);
+    }
+    size_t bytes() const { return bytes_; }
+    bool fits(const Scratch& scr) const { return bytes_ > 0 && scr.bytes >= bytes_; }
+
+    void forward(const Scratch& scr, hipStream_t s) const
+    {
+        float* packed = fits(scr) ? (float*)scr.data : nullptr;
+        if (packed) check_hip(dvr::launch_pack_preshaded(c_.P, packed, s), "pack launch");
+        check_hip(dvr::launch_forward_preshaded(c_.P, c_.blend, packed, s), "forward (pre-shaded) launch");
+    }
+    void adjoint(const Scratch& scr, hipStream_t s) const
+    {
+        if (!fits(scr)) {
+            check_hip(dvr::launch_adjoint_preshaded(c_.P, *A_, c_.blend, s), "adjoint (pre-shaded) launch");
+            return;
+        }
+        float* packed = (float*)scr.data;
+        float* brick = packed + packed_;
+        check_hip(dvr::launch_pack_preshaded(c_.P, packed, s), "pack launch");
+        dvr::CkptParams CK{};
+        const size_t plane = size_t(group_) * size_t(cap_ + dvr::kAdjSpill) * dvr::kBlock;
+        if (A_->avol) {
+            CK.as.rays = brick + 4 * brickFloats_;
+            CK.as.adj = CK.as.rays + size_t(group_) * dvr::kRayRecord * dvr::kBlock;
+            CK.as.cap = cap_;
+            check_hip(dvr::launch_clear(brick, 4 * brickFloats_, s), "clear launch");
+        }
+        for (int t0 = 0; t0 < tiles_; t0 += group_) {
+            CK.tile0 = t0;
+            CK.tileN = std::min(group_, tiles_ - t0);
+            check_hip(dvr::launch_adjoint_preshaded_packed(c_.P, *A_, CK, plane, packed, c_.blend, s),
+                      "adjoint (pre-shaded) launch");
+            if (!A_->avol) continue;
+            dvr::ScatterParams S;
+            std::memset(&S, 0, sizeof(S));
+            S.S = CK.as;
+            S.nTiles = CK.tileN;
+            S.tile0 = t0;
+            S.brick = brick;
+            S.brickFloats = brickFloats_;
+            S.tilesPerVolume = tiles_;
+            S.X = c_.X; S.Y = c_.Y; S.Z = c_.Z;
+            S.adjPlane = plane;
+            check_hip(dvr::launch_scatter_volume(S, 1, s, 4), "scatter launch");
+        }
+        if (!A_->avol) return;
+        const dvr::DebrickSeg D{brick, A_->avol, c_.X, c_.Y, c_.Z, 0, A_->avSx, A_->avSy, A_->avSz};
+        check_hip(dvr::launch_debrick_call(D, 4, A_->avSb, s), "debrick launch");
+    }
+
+private:
+    const Checked& c_;
+    const dvr::AdjointParams* A_;
+    int tiles_ = 0, cap_ = 0, group_ = 0;
+    size_t packed_ = 0, brickFloats_ = 0, bytes_ = 0;
+};
+
+void do_forward(const dvr_inputs* inputs, dvr_outputs* outputs, const dvr_forward_options* opt, void* stream,
+                const Scratch& scr = {})
+{
+    Checked c = check_inputs(inputs);
+    check_outputs(outputs, c);
+    int path = opt ? opt->path : DVR_PATH_AUTO;
+    const int K = opt ? opt->checkpoint_interval : 0;
+    if (path == DVR_PATH_AUTO) path = tiled_ok(c) ? DVR_PATH_TILED : DVR_PATH_PLAIN;
+    if (c.preshaded && (path != DVR_PATH_PLAIN || K > 0))
+        fail(DVR_ERR_UNSUPPORTED, "pre-shaded volumes render on the plain path only");
+    DeviceGuard g(c.device);
+    hipStream_t s = (hipStream_t)stream;
+    if (path == DVR_PATH_TILED && !tiled_ok(c))
+        fail(DVR_ERR_UNSUPPORTED, "tiled path needs R*C <= %d transfer-function entries", dvr::kMaxTfLds);
+    if (K > 0) {
+        if (path != DVR_PATH_TILED) fail(DVR_ERR_UNSUPPORTED, "checkpoints are written by the tiled forward only");
+        make_ckpt(c, K);  // validates K
+        const dvr_tensor& ck = opt->checkpoints;
+        const int64_t need = (int64_t)dvr::tiled_num_tiles(c.P) * checkpoint_cap(c, K) * dvr::kBlock;
+        if (!given(ck) || ck.dtype != DVR_FLOAT32 || ck.device != c.device)
+            fail(DVR_ERR_INVALID_ARGUMENT, "checkpoints must be a float32 tensor on the render device");
+        int64_t numel = 1;
+        for (int d = 0; d < ck.ndim; ++d) numel *= ck.sizes[d];
+        if (numel < need) fail(DVR_ERR_INVALID_ARGUMENT, "checkpoints needs %lld elements, has %lld", (long long)need, (long long)numel);
+        if (ck.ndim > 0 && ck.strides[ck.ndim - 1] != 1 && numel > 1)
+            fail(DVR_ERR_INVALID_ARGUMENT, "checkpoints must be contiguous");
+        if (given(opt->densities)) density_buffer(opt->densities, c);
+    } else if (opt && given(opt->densities)) {
+        fail(DVR_ERR_INVALID_ARGUMENT, "densities are written together with checkpoints (checkpoint_interval > 0)");
+    }
+    if (c.preshaded) {
+        PackedPreshaded(c, nullptr).forward(scr, s);
+    } else if (path == DVR_PATH_PLAIN) {
+        check_hip(dvr::launch_forward_plain(c.P, c.filter, c.tfm, c.blend, s), "forward (plain) launch");
+    } else {
+        dvr::CkptParams CK{nullptr, 16, 0, 1};
+        if (K > 0) {
+            CK = make_ckpt(c, K);
+            CK.buf = (float*)opt->checkpoints.data;
+            if (given(opt->densities)) {
+                CK.ds = density_buffer(opt->densities, c);
+                CK.dsCap = density_cap(c);
+            }
+        }
+        check_hip(dvr::launch_forward_tiled(c.P, CK, c.filter, c.tfm, c.blend, s), "forward (tiled) launch");
+        if (K > 0) stamp_checkpoints(CK.buf, CkptStamp{K, c.B, c.H, c.W, CK.ds});
+    }
+}
 
 int adjoint_method(const Checked& c, const dvr_adjoint_options* opt)
 {
@@ -713,7 +801,7 @@ void do_adjoint(const dvr_inputs* inputs, const dvr_outputs* fwd, const dvr_tens
     if (c.preshaded) {
         if (method != DVR_ADJOINT_INVERSION || path == DVR_PATH_TILED)
             fail(DVR_ERR_UNSUPPORTED, "pre-shaded volumes use the inversion adjoint on the plain path");
-        check_hip(dvr::launch_adjoint_preshaded(c.P, A, c.blend, s), "adjoint (pre-shaded) launch");
+        PackedPreshaded(c, &A).adjoint(scr, s);
         return;
     }
     if (method == DVR_ADJOINT_INVERSION) {
@@ -1168,6 +1256,22 @@ dvr_status dvr_compare_to_image(const dvr_tensor* color, const dvr_tensor* gradi
     return guarded([&] { do_compare(color, gradients, reference, difference_out, gradients_out, reduce, stream); });
 }
 
+int64_t dvr_forward_scratch_bytes(const dvr_inputs* inputs)
+{
+    int64_t r = -1;
+    guarded([&] {
+        Checked c = check_inputs(inputs);
+        r = c.preshaded ? int64_t(PackedPreshaded(c, nullptr).bytes()) : 0;
+    });
+    return r;
+}
+
+dvr_status dvr_render_forward_scratch(const dvr_inputs* inputs, dvr_outputs* outputs, const dvr_forward_options* options,
+                                      void* scratch, int64_t scratch_bytes, void* stream)
+{
+    return guarded([&] { do_forward(inputs, outputs, options, stream, call_scratch(scratch, scratch_bytes)); });
+}
+
 int64_t dvr_adjoint_scratch_bytes(const dvr_inputs* inputs, const dvr_outputs* outputs_from_forward,
                                   const dvr_tensor* adj_color, const dvr_adjoint_outputs* adj_outputs,
                                   const dvr_adjoint_options* options)
@@ -1176,7 +1280,8 @@ int64_t dvr_adjoint_scratch_bytes(const dvr_inputs* inputs, const dvr_outputs* o
     guarded([&] {
         Checked c = check_inputs(inputs);
         const dvr::AdjointParams A = check_adjoint(c, outputs_from_forward, adj_color, adj_outputs);
-        r = adjoint_method(c, options) == DVR_ADJOINT_CHECKPOINT ? int64_t(TwoPassGradient(c, A).bytes()) : 0;
+        if (c.preshaded) r = int64_t(PackedPreshaded(c, &A).bytes());
+        else r = adjoint_method(c, options) == DVR_ADJOINT_CHECKPOINT ? int64_t(TwoPassGradient(c, A).bytes()) : 0;
     });
     return r;
 }
@@ -1187,10 +1292,8 @@ dvr_status dvr_render_adjoint_scratch(const dvr_inputs* inputs, const dvr_output
                                       void* stream)
 {
     return guarded([&] {
-        if (scratch_bytes > 0 && (reinterpret_cast<uintptr_t>(scratch) & 255u) != 0)
-            fail(DVR_ERR_INVALID_ARGUMENT, "scratch must be 256-byte aligned");
         do_adjoint(inputs, outputs_from_forward, adj_color, adj_outputs, options, stream,
-                   Scratch{scratch, scratch ? size_t(std::max<int64_t>(scratch_bytes, 0)) : 0});
+                   call_scratch(scratch, scratch_bytes));
     });
 }
 

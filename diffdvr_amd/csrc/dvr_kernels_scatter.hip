@@ -152,7 +152,7 @@ __global__ __launch_bounds__(kScatterBlock) void k_scatter_volume(ScatterParams 
         V.brick = vol.brick;
     } else {
         V.X = P.X; V.Y = P.Y; V.Z = P.Z;
-        V.brick = P.brick + size_t((P.tile0 + tile) / P.tilesPerVolume) * P.brickFloats;
+        V.brick = P.brick + size_t((P.tile0 + tile) / P.tilesPerVolume + int(blockIdx.y)) * P.brickFloats;
     }
     V.BY = unsigned(V.Y + 1) >> 1;
     V.BZ = unsigned(V.Z + 3) >> 2;
@@ -172,7 +172,7 @@ __global__ __launch_bounds__(kScatterBlock) void k_scatter_volume(ScatterParams 
     const f3 p0 = mk3(rec[0], rec[kBlock], rec[2 * kBlock]);
     const f3 dp = mk3(rec[3 * kBlock], rec[4 * kBlock], rec[5 * kBlock]);
     const float t0 = rec[6 * kBlock], step = rec[7 * kBlock];
-    const float* adj = P.S.adj + size_t(tile) * (size_t(P.S.cap + kAdjSpill) * kBlock) + ray;
+    const float* adj = P.S.adj + blockIdx.y * P.adjPlane + size_t(tile) * (size_t(P.S.cap + kAdjSpill) * kBlock) + ray;
 
     for (int e = threadIdx.x; e < kSlots; e += kScatterBlock) L.tags[e] = kFree;
     for (int e = threadIdx.x; e < kSlots * 16; e += kScatterBlock) L.vals[e] = 0.0;
@@ -243,14 +243,14 @@ __global__ __launch_bounds__(kScatterBlock) void k_scatter_volume(ScatterParams 
     }
 }
 
-hipError_t launch_scatter_volume(const ScatterParams& P, int filter, hipStream_t s)
+hipError_t launch_scatter_volume(const ScatterParams& P, int filter, hipStream_t s, int channels)
 {
     if (P.nTiles <= 0) return hipSuccess;
     ScatterParams Q = P;
     // few tiles: several workgroups share a tile's samples
     Q.parts = 1;
     while (Q.parts < 16 && Q.nTiles * Q.parts < 2048) Q.parts *= 2;
-    const dim3 grid(unsigned(Q.nTiles) * unsigned(Q.parts));
+    const dim3 grid(unsigned(Q.nTiles) * unsigned(Q.parts), unsigned(channels));
     if (filter == 0) hipLaunchKernelGGL(k_scatter_volume<0>, grid, dim3(kScatterBlock), 0, s, Q);
     else hipLaunchKernelGGL(k_scatter_volume<1>, grid, dim3(kScatterBlock), 0, s, Q);
     return hipGetLastError();

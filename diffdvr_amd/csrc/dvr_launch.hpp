@@ -93,12 +93,16 @@ hipError_t launch_debrick(const DebrickSeg* dSegs, int nSegs, long long maxBrick
 // the same for one call's gradient: `batches` scratch volumes of brick_floats() each, batch stride sb of the gradient
 hipError_t launch_debrick_call(const DebrickSeg& S, int batches, long long sb, hipStream_t s);
 // dvr_kernels_scatter.hip: the second pass of the volume gradients (P.parts is chosen here)
-hipError_t launch_scatter_volume(const ScatterParams& P, int filter, hipStream_t s);
+hipError_t launch_scatter_volume(const ScatterParams& P, int filter, hipStream_t s, int channels = 1);
 // clears n floats (a multiple of 4, 16-byte aligned) with a kernel
 hipError_t launch_clear(float* p, size_t n, hipStream_t s);
 
-// pre-shaded volumes (dvr_kernels_preshaded.hip): plain structure, inversion adjoint
-hipError_t launch_forward_preshaded(const RenderParams& P, int blend, hipStream_t s);
+// pre-shaded volumes (dvr_kernels_preshaded.hip): inversion adjoint; plain structure where packed is NULL
+hipError_t launch_forward_preshaded(const RenderParams& P, int blend, const float* packed, hipStream_t s);
+// packed: the four slices as one RGBA volume, [X][Y][Z][4]
+hipError_t launch_pack_preshaded(const RenderParams& P, float* packed, hipStream_t s);
+hipError_t launch_adjoint_preshaded_packed(const RenderParams& P, const AdjointParams& A, const CkptParams& CK,
+                                           size_t plane, const float* packed, int blend, hipStream_t s);
 hipError_t launch_adjoint_preshaded(const RenderParams& P, const AdjointParams& A, int blend, hipStream_t s);
 
 // forward-mode derivatives (dvr_kernels_fwdgrad.hip)

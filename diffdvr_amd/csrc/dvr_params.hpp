@@ -181,6 +181,7 @@ struct ScatterParams {
     const struct BView* views; int nViews, tile0;
     const struct BVol* vols;
     float* brick; size_t brickFloats; int tilesPerVolume, X, Y, Z;
+    size_t adjPlane;            // floats between the channels' stores (several channels of one volume)
 };
 
 struct BTf {

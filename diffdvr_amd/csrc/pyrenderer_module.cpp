@@ -566,7 +566,10 @@ PYBIND11_MODULE(_pyrenderer, m)
               opt.checkpoint_interval = checkpoint_interval;
               opt.checkpoints = to_tensor(checkpoints);
               opt.densities = to_tensor(densities);
-              check(dvr_render_forward_ex(&p.in, &o, &opt, current_stream(p.in.volume.device)));
+              const bool preshaded = p.in.volume_filter_mode == DVR_FILTER_PRESHADED;
+              const CallScratch scr(preshaded ? dvr_forward_scratch_bytes(&p.in) : 0, inputs.volume);
+              check(dvr_render_forward_scratch(&p.in, &o, &opt, scr.data, scr.bytes,
+                                               current_stream(p.in.volume.device)));
           },
           py::arg("inputs"), py::arg("outputs"), py::arg("path") = "auto", py::arg("checkpoint_interval") = 0,
           py::arg("checkpoints") = py::none(), py::arg("densities") = py::none());

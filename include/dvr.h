@@ -188,10 +188,13 @@ dvr_status dvr_render_adjoint_ex(const dvr_inputs* inputs, const dvr_outputs* ou
                                  const dvr_tensor* adj_color, dvr_adjoint_outputs* adj_outputs,
                                  const dvr_adjoint_options* options, void* stream);
 
-/* dvr_render_adjoint_ex with device scratch of the caller's (256-byte aligned, used on `stream` until the
- * call's work is done, contents undefined before and after).  dvr_adjoint_scratch_bytes says how much a call
+/* dvr_render_forward_ex and dvr_render_adjoint_ex with device scratch of the caller's (256-byte aligned, used on `stream` until the
+ * call's work is done, contents undefined before and after).  The _bytes functions say how much a call
  * would use (0: none; -1: the arguments are invalid).  Results are the same up to the order of float sums;
  * with less scratch, or NULL, the call runs the kernels that need none. */
+int64_t dvr_forward_scratch_bytes(const dvr_inputs* inputs);
+dvr_status dvr_render_forward_scratch(const dvr_inputs* inputs, dvr_outputs* outputs, const dvr_forward_options* options,
+                                      void* scratch, int64_t scratch_bytes, void* stream);
 int64_t dvr_adjoint_scratch_bytes(const dvr_inputs* inputs, const dvr_outputs* outputs_from_forward,
                                   const dvr_tensor* adj_color, const dvr_adjoint_outputs* adj_outputs,
                                   const dvr_adjoint_options* options);

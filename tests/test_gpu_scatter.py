@@ -154,3 +154,38 @@ def test_plan_matches_per_call(size, filter, tf_mode, grads):
     torch.cuda.synchronize()
     for ref, got in [(a.adj_volume[0], gv)] + ([(a.adj_tf[0], gt)] if "tf" in grads else []):
         assert float((ref - got).abs().max() / ref.abs().max()) <= 1e-4
+
+
+@pytest.mark.parametrize("W,H,B", [(13, 11, 2), (203, 97, 1)])
+@pytest.mark.parametrize("layout,blend,grads", [("contiguous", 0, ("volume",)), ("xfast", 1, ("volume",)),
+                                                ("padded", 0, ("volume", "camera")), ("contiguous", 1, ("camera",))])
+def test_packed_preshaded(W, H, B, layout, blend, grads):
+    """Pre-shaded volumes packed into RGBA against the kernels that gather from the four slices (which a
+    gradient shared over x makes the call run)."""
+    d = dev()
+    rng = np.random.default_rng(W + blend)
+    s = camera_scene(rng, W, H, B=B, X=7, Y=6, Z=9, step=0.03)
+    s["volume"] = to_f32(rng.uniform(0.1, 0.9, (4, 7, 6, 9)) * np.array([1, 1, 1, 4.0 if blend == 0 else 0.3])[:, None, None, None])
+    inp = gpu_inputs(s)
+    inp.volume_filter_mode = pr.VolumeFilterMode.Preshaded
+    inp.tf_mode = pr.TFMode.Preshaded
+    inp.blend_mode = pr.BlendMode(blend)
+    adj = torch.randn(B, H, W, 4, generator=torch.Generator().manual_seed(8)).to(d)
+    o = pr.RendererOutputs(torch.empty(B, H, W, 4, device=d), torch.empty(B, H, W, dtype=torch.int32, device=d))
+    pr.Renderer.render_forward(inp, o)
+    res = []
+    for lay in ("expanded", layout):
+        a = pr.AdjointOutputs()
+        a.has_volume_derivatives = "volume" in grads or lay == "expanded"
+        a.adj_volume = gradient((4, 7, 6, 9), lay)
+        a.has_camera_derivatives = True
+        a.adj_camera_ray_start = torch.zeros(B, H, W, 3, device=d)
+        a.adj_camera_ray_dir = torch.zeros(B, H, W, 3, device=d)
+        pr.Renderer.render_adjoint(inp, o, adj, a)
+        torch.cuda.synchronize()
+        res.append((a.adj_camera_ray_start, a.adj_camera_ray_dir, a.adj_volume))
+    for k in range(2):
+        assert float((res[0][k] - res[1][k]).abs().max() / res[0][k].abs().max()) <= 1e-4
+    if "volume" in grads:  # the shared gradient is the sum over x
+        one, two = res[0][2][:, 0], res[1][2].sum(1)
+        assert float((one - two).abs().max() / one.abs().max()) <= 1e-4
