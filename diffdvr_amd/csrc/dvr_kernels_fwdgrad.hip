@@ -11,6 +11,8 @@
 // ray of the pixel after camera evaluation, renderer_camera.cuh:64-130), and
 // TF entries through the index table d_tf.  tmin is not traced (the
 // reference casts it to real).
+#include <algorithm>
+
 #include "dvr_tiled_impl.hpp"
 
 namespace dvr {
@@ -234,6 +236,113 @@ __global__ __launch_bounds__(kBlock) void k_forward_gradients(RenderParams P, Fw
     }
 }
 
+// Slices that trace entries of a Gaussian TF only (no step size, no ray).  An
+// entry's derivative of the TF output is then a scalar of the sample times a
+// vector of the launch: rgba entries n times a unit vector, the mean's
+// n (d - mu) / s^2 and the deviation's n (d - mu)^2 / s^3 times the row's
+// colour.  The scalar is n (fa + dd (fb + dd fc)) with coefficients per slot
+// (in LDS, read as broadcasts: kept in scalar registers they spilled and ran
+// 16 us longer), without branches over rows and columns, and the colour
+// derivative through the TF needs one sum per slot, sum T alpha f, times the
+// vector's channels at the end.  Two views of 160 x 160, 24 entries: 1061 us
+// with k_forward_gradients (186 registers, two waves a SIMD), 270 us here; the
+// longest rays' chain bounds it.  Four entries a slice took 90 us more (the value
+// part is marched by every slice), twelve as long.
+template <int FILTER, int BLEND>
+__global__ __launch_bounds__(kBlock) void k_forward_gradients_gauss(RenderParams P, FwdGradParams G, int vecStore,
+                                                                    int tilesX, int tilesPerView, int nTiles)
+{
+    extern __shared__ float lds[];
+    constexpr int kC = tf_cols<3>();
+    const TileXY tc = tile_xy(tilesX, tilesPerView, nTiles);
+    const int b = tc.b, x = tc.x, y = tc.y;
+    const int d0 = blockIdx.y * kFwdChunk;
+    const int nSlots = min(kFwdChunk, G.D - d0);
+    const float* tf = P.tf + b * P.tfSb;
+    __shared__ float4 s_c[kFwdChunk][2];  // (mean, exponent scale, fa, fb), (fc, va) of a slot
+    if (threadIdx.x < kFwdChunk) {
+        const int k = threadIdx.x, e = k < nSlots ? G.tfEntry[b * G.tfEntrySb + d0 + k] : -1;
+        const int row = max(e, 0) / kC, col = max(e, 0) - row * kC;
+        const float* r = tf + row * P.tfSr;
+        const float sg = r[5 * P.tfSc];
+        s_c[k][0] = make_float4(r[4 * P.tfSc], -1.44269504088896341f / (2.0f * sg * sg), e >= 0 && col < 4 ? 1.0f : 0.0f,
+                                e >= 0 && col == 4 ? 1.0f / (sg * sg) : 0.0f);
+        s_c[k][1] = make_float4(e >= 0 && col == 5 ? 1.0f / (sg * sg * sg) : 0.0f,
+                                col < 4 ? (col == 3 ? 1.0f : 0.0f) : r[3 * P.tfSc], 0.0f, 0.0f);
+    }
+    stage_tf(P, b, lds);
+    __syncthreads();
+    if (x >= P.W || y >= P.H) return;
+
+    const Ray r = setup_ray(P, x, y, b);
+    const Vol V = make_vol(P, b);
+    const Tf T{lds, P.R, kC, kC, 1};
+    Acc acc{0.f, 0.f, 0.f, 0.f, 1.f};
+    float dr[kFwdChunk], dg[kFwdChunk], db[kFwdChunk], dA[kFwdChunk], dT[kFwdChunk], sf[kFwdChunk];
+#pragma unroll
+    for (int k = 0; k < kFwdChunk; ++k) { dr[k] = 0.f; dg[k] = 0.f; db[k] = 0.f; dA[k] = 0.f; dT[k] = 0.f; sf[k] = 0.f; }
+    const float tEarly = 1.0f - P.earlyOut;
+    FetchPipe<FILTER> pipe;
+    float t = r.t0;
+    f3 p = sample_pos(r, t);
+    if (!(t > r.t1)) pipe.start(V, p);
+    int i = 0;
+    for (; i < kMaxSamples; ++i) {
+        if (t > r.t1) break;
+        if (acc.T < tEarly) break;
+        const float dens = pipe.value(p);
+        t = r.t0 + float(i + 1) * r.step;
+        p = sample_pos(r, t);
+        if (!(t > r.t1)) pipe.request(V, p);
+        const f4 s = tf_eval<3, true>(T, dens);
+        float alpha, keep;
+        alpha_keep<BLEND>(s.w, r.step, alpha, keep);
+        const float w = acc.T * alpha;
+        const float slope = acc.T * r.step * (BLEND == 0 ? keep : (s.w * r.step < 1.0f ? 1.0f : 0.0f));
+#pragma unroll
+        for (int k = 0; k < kFwdChunk; ++k) {
+            const float4 c = s_c[k][0];
+            const float2 v = *reinterpret_cast<const float2*>(&s_c[k][1]);
+            const float dd = dens - c.x;
+            const float f = __builtin_amdgcn_exp2f(dd * dd * c.y) * (c.z + dd * (c.w + dd * v.x));
+            const float da = slope * v.y * f;  // T dalpha = -T dkeep
+            const float dw = dT[k] * alpha + da;
+            dr[k] += dw * s.x;
+            dg[k] += dw * s.y;
+            db[k] += dw * s.z;
+            dA[k] += dw;
+            dT[k] = dT[k] * keep - da;
+            sf[k] += w * f;
+        }
+        pipe.advance();
+        acc.r += w * s.x;
+        acc.g += w * s.y;
+        acc.b += w * s.z;
+        acc.A += w;
+        acc.T *= keep;
+    }
+    if (blockIdx.y == 0) {
+        float* o = P.color + b * P.colSb + y * P.colSy + x * P.colSx;
+        o[0] = acc.r; o[P.colSc] = acc.g; o[2 * P.colSc] = acc.b; o[3 * P.colSc] = acc.A;
+        P.term[b * P.termSb + y * P.termSy + x * P.termSx] = i;
+    }
+    float* g = G.grad + b * G.gSb + y * G.gSy + x * G.gSx + d0 * G.gSd;
+#pragma unroll
+    for (int k = 0; k < kFwdChunk; ++k) {
+        if (k < nSlots) {
+            const int e = max(G.tfEntry[b * G.tfEntrySb + d0 + k], 0), row = e / kC, col = e - row * kC;
+            const float* c = tf + row * P.tfSr;
+            const float vx = col < 4 ? (col == 0 ? 1.0f : 0.0f) : c[0];
+            const float vy = col < 4 ? (col == 1 ? 1.0f : 0.0f) : c[P.tfSc];
+            const float vz = col < 4 ? (col == 2 ? 1.0f : 0.0f) : c[2 * P.tfSc];
+            const float4 v = make_float4(dr[k] + sf[k] * vx, dg[k] + sf[k] * vy, db[k] + sf[k] * vz, dA[k]);
+            float* q = g + k * G.gSd;
+            if (vecStore) *reinterpret_cast<float4*>(q) = v;
+            else { q[0] = v.x; q[G.gSc] = v.y; q[2 * G.gSc] = v.z; q[3 * G.gSc] = v.w; }
+        }
+    }
+}
+
 template <int FILTER, int TFM, int BLEND>
 static hipError_t fwdgrad_t(const RenderParams& P, const FwdGradParams& G, hipStream_t s)
 {
@@ -242,6 +351,17 @@ static hipError_t fwdgrad_t(const RenderParams& P, const FwdGradParams& G, hipSt
     if (nTiles == 0 || G.D == 0) return hipSuccess;
     const int chunks = (G.D + kFwdChunk - 1) / kFwdChunk;
     const size_t lds = sizeof(float) * size_t(P.R) * P.C;
+    if constexpr (TFM == 3) {
+        const bool rays = G.dStep >= 0 || std::max({G.dStart[0], G.dStart[1], G.dStart[2]}) >= 0 ||
+                          std::max({G.dDir[0], G.dDir[1], G.dDir[2]}) >= 0;
+        if (!rays && G.tfEntry) {
+            const int vec = G.gSc == 1 && ((G.gSb | G.gSy | G.gSx | G.gSd) & 3) == 0 &&
+                            (reinterpret_cast<uintptr_t>(G.grad) & 15u) == 0;
+            hipLaunchKernelGGL((k_forward_gradients_gauss<FILTER, BLEND>), dim3(nTiles, (G.D + kFwdChunk - 1) / kFwdChunk), dim3(kBlock), lds, s, P,
+                               G, vec, tilesX, tilesX * tilesY, nTiles);
+            return hipGetLastError();
+        }
+    }
     hipLaunchKernelGGL((k_forward_gradients<FILTER, TFM, BLEND>), dim3(nTiles, chunks), dim3(kBlock), lds, s, P, G,
                        tilesX, tilesX * tilesY, nTiles);
     return hipGetLastError();
