@@ -111,6 +111,9 @@ struct dvr_batch_plan {
     dvr::DebrickSeg* dDebrick = nullptr;
     int nDebrick = 0;
     long long maxBricks = 0;
+    double* dSums = nullptr;            // sums of a run: loss, TF gradients (added into the caller's after it)
+    dvr::SumSeg* dSumSegs = nullptr;
+    int nSums = 0, maxSum = 0;
     float* dCk = nullptr;
     size_t ckFloats = 0;
     float* dDs = nullptr;   // density store of the forward march (adjoint plans), or NULL
@@ -126,15 +129,15 @@ struct dvr_batch_plan {
     ~dvr_batch_plan()
     {
         dev_free(dViews); dev_free(dVols); dev_free(dTfs); dev_free(dQueues); dev_free(dSegsAll); dev_free(dCk);
-        dev_free(dDs); dev_free(dAs); dev_free(dBricks); dev_free(dDebrick);
+        dev_free(dDs); dev_free(dAs); dev_free(dBricks); dev_free(dDebrick); dev_free(dSums); dev_free(dSumSegs);
     }
 
     // doubles between the TF-gradient table copies; 0 (one table) when the copies would take more than
     // 16 KiB of LDS per workgroup, which keeps eight one-wave workgroups resident per CU
     int copy_stride() const { return dvr::tf_grad_copy_stride(maxRC); }
 
-    // floats of the LDS TF table (the kernel pads linear-TF rows to 8 floats, dvr::tf_lds_stride), even
-    int tf_lds() const { return dvr::tf_grad_offset(tfm == 2 ? (maxRC / 5) * 8 : maxRC); }
+    // floats of the LDS TF table (linear and Gaussian rows take 8 floats, dvr::tf_lds_stride), even
+    int tf_lds() const { return dvr::tf_grad_offset(tfm >= 2 ? (maxRC / tf_cols(tfm)) * 8 : maxRC); }
 
     // register segment length of checkpoint interval K (64 = two 32-sample segments)
     int segK() const { return K > 32 ? 32 : K; }
@@ -146,7 +149,7 @@ struct dvr_batch_plan {
     dvr::BatchParams params(int group = 0) const
     {
         dvr::BatchParams P{};
-        P.views = dViews; P.vols = dVols; P.tfs = dTfs; P.ck = dCk; P.lossOut = lossOut;
+        P.views = dViews; P.vols = dVols; P.tfs = dTfs; P.ck = dCk; P.lossOut = lossOut ? dSums : nullptr;
         P.ds = dsCap > 0 ? dDs : nullptr; P.dsCap = dsCap;
         P.nViews = (int)views.size(); P.nTiles = nTiles; P.ckCap = cap;
         P.ckEvery = K > 32 ? K / 32 : 1;
@@ -309,6 +312,7 @@ struct dvr_batch_plan {
         }
         if (evEnd) check_hip(hipEventRecord(evEnd, s), "hipEventRecord");
         if (nDebrick > 0) check_hip(dvr::launch_debrick(dDebrick, nDebrick, maxBricks, s), "debrick launch");
+        if (nTiles > 0) check_hip(dvr::launch_add_sums(dSumSegs, nSums, maxSum, s), "sum launch");
     }
 };
 
@@ -571,6 +575,33 @@ dvr_batch_plan* create(const dvr_batch* b, const dvr_batch_options* o)
             p->nDebrick = (int)db.size();
             p->dDebrick = dev_alloc<dvr::DebrickSeg>(db.size());
             check_hip(hipMemcpy(p->dDebrick, db.data(), db.size() * sizeof(dvr::DebrickSeg), hipMemcpyHostToDevice),
+                      "hipMemcpy");
+        }
+    }
+    // sums in doubles: the loss first, then every TF gradient
+    if (p->gm) {
+        size_t n = 1;
+        std::vector<size_t> off;
+        for (auto& t : p->tfs) {
+            off.push_back(n);
+            if (t.adj) n += size_t(t.R) * t.C;
+        }
+        p->dSums = dev_alloc<double>(n);
+        segs.push_back({reinterpret_cast<float*>(p->dSums), (long long)n * 2});
+        p->maxSegAlways = std::max(p->maxSegAlways, (long long)n * 2);
+        std::vector<dvr::SumSeg> sums;
+        if (p->lossOut) sums.push_back({p->dSums, p->lossOut, 1, 0});
+        for (size_t k = 0; k < p->tfs.size(); ++k) {
+            dvr::BTf& t = p->tfs[k];
+            if (!t.adj) continue;
+            t.sum = p->dSums + off[k];
+            sums.push_back({t.sum, t.adj, t.R * t.C, 0});
+        }
+        for (auto& q : sums) p->maxSum = std::max(p->maxSum, q.n);
+        p->nSums = (int)sums.size();
+        if (p->nSums > 0) {
+            p->dSumSegs = dev_alloc<dvr::SumSeg>(sums.size());
+            check_hip(hipMemcpy(p->dSumSegs, sums.data(), sums.size() * sizeof(dvr::SumSeg), hipMemcpyHostToDevice),
                       "hipMemcpy");
         }
     }

@@ -26,16 +26,16 @@ namespace dvr {
 template <int TFM>
 __device__ __forceinline__ void batched_flush_tf(const BatchParams& B, int tfi, const float* s_g, int RC, bool priv)
 {
-    float* g = B.tfs[tfi].adj;
+    double* g = B.tfs[tfi].sum;
     for (int e = threadIdx.x; e < RC; e += kBatchBlock) {
-        float v;
+        double v;
         if (priv) {
-            v = 0.0f;
-            for (int t = 0; t < kBatchBlock; ++t) v += s_g[e * kBatchBlock + t];
+            v = 0.0;
+            for (int t = 0; t < kBatchBlock; ++t) v += double(s_g[e * kBatchBlock + t]);
         } else {
             v = tf_grad_sum(s_g, e, B.tfCopyStride);
         }
-        if (v != 0.0f) gatomic_add(g, unsigned(e), v);
+        if (v != 0.0) atomicAdd(g + e, v);
     }
 }
 
@@ -116,7 +116,7 @@ __global__ __launch_bounds__(kBatchBlock) __attribute__((amdgpu_waves_per_eu(
             curWantTf = ADJ && B.wantTf && tf.adj != nullptr;
             // rows at a stride of tf_lds_stride<TFM>() floats (16-byte aligned RGBA for the linear TF)
             for (int e = threadIdx.x; e < curRC; e += kBatchBlock)
-                s_tf[(e / tf_cols<TFM>()) * tf_lds_stride<TFM>() + (e % tf_cols<TFM>())] = gld(tf.p, unsigned(e));
+                tf_stage_entry<TFM>(s_tf, e / tf_cols<TFM>(), e % tf_cols<TFM>(), gld(tf.p, unsigned(e)));
             if (curWantTf) {
                 const int ng = tf_grad_floats(curRC, priv, kBatchBlock, B.tfCopyStride);
                 for (int e = threadIdx.x; e < ng; e += kBatchBlock) s_g[e] = 0.0f;
@@ -260,7 +260,7 @@ __global__ __launch_bounds__(kBatchBlock) __attribute__((amdgpu_waves_per_eu(
         }
         if (B.lossOut) {
             const float s = wave_sum(lossLocal);
-            if (lane == 0 && s != 0.0f) atomicAdd(B.lossOut, s);
+            if (lane == 0 && s != 0.0f) atomicAdd(B.lossOut, double(s));
         }
     }
 }

@@ -568,6 +568,8 @@ struct Scratch {
     size_t bytes = 0;
 };
 
+constexpr size_t kMaxStore = size_t(2) << 30;  // bytes of the density adjoints a call may store at a time
+
 Scratch call_scratch(void* data, int64_t bytes)
 {
     if (bytes > 0 && (reinterpret_cast<uintptr_t>(data) & 255u) != 0)
@@ -589,50 +591,42 @@ bool distinct_elements(const Checked& c, const dvr::AdjointParams& A, int volume
     return true;
 }
 
-// Volume gradients of the checkpointed adjoint in two passes (dvr_kernels_scatter.hip): the walk stores
-// the density adjoints of a group of tiles and their rays, k_scatter_volume adds them into bricked
-// scratch, and after the last group k_debrick adds that into the caller's gradient.  Scratch layout:
-// [bricks][rays][density adjoints], each 64-byte aligned.
-constexpr size_t kMaxStore = size_t(2) << 30;  // bytes of a group's store
-
-class TwoPassGradient {
+// Call scratch of the checkpointed adjoint.  TF gradients that thousands of workgroups add to are summed in
+// doubles and added into the caller's tensor after the last launch.  Volume gradients take two passes
+// (dvr_kernels_scatter.hip): the walk stores the density adjoints of a group of tiles and their rays,
+// k_scatter_volume adds them into bricked scratch, and after the last group k_debrick adds that into the
+// caller's gradient.  Scratch layout: [TF sums][bricks][rays][density adjoints], each 16-byte aligned.
+class AdjointScratch {
 public:
-    TwoPassGradient(const Checked& c, const dvr::AdjointParams& A) : c_(c), A_(A)
+    AdjointScratch(const Checked& c, const dvr::AdjointParams& A) : c_(c), A_(A), tiles_(dvr::tiled_num_tiles(c.P))
     {
-        // the store holds the longest ray of a uniform box and step; clearing and adding the bricks
-        // (16 bytes a voxel) pays from a few samples per ten voxels on
-        if (!A.avol || c.preshaded || c.P.st || c.P.bsize) return;
-        volumes_ = A.avSb != 0 ? c.B : 1;
-        if (!distinct_elements(c, A, volumes_)) return;
-        const double voxels = double(c.X) * c.Y * c.Z * volumes_;
-        tiles_ = dvr::tiled_num_tiles(c.P);
-        cap_ = dvr::adj_store_cap(density_cap(c));
-        const double samples = double(c.B) * c.W * c.H * cap_ * 0.5;
-        if (tiles_ == 0 || samples < 0.25 * voxels) return;
-        const size_t perTile = dvr::adj_store_floats(cap_) * sizeof(float);
-        group_ = int(std::min<size_t>(size_t(tiles_), kMaxStore / perTile));
-        if (group_ < std::min(tiles_, 4096)) return;  // groups too small to fill the chip
-        brickFloats_ = dvr::brick_floats(c.X, c.Y, c.Z);
-        if (brickFloats_ >= (size_t(1) << 30)) return;  // 32-bit byte offsets
-        bytes_ = sizeof(float) * brickFloats_ * volumes_ + size_t(group_) * perTile;
+        if (c.preshaded || tiles_ == 0) return;
+        if (A.atf && tiles_ >= kSumTiles) sums_ = (size_t(A.atfSb != 0 ? c.B : 1) * c.P.R * c.P.C + 1) / 2 * 4;
+        plan_volume();
+        bytes_ = sizeof(float) * (sums_ + brickFloats_ * volumes_ + size_t(group_) * perTile_);
     }
     size_t bytes() const { return bytes_; }
 
-    // Runs the adjoint: launch(CK) must launch the tiles CK.tile0 .. tile0 + tileN - 1.
+    // Runs the adjoint: launch(A, CK) must launch the tiles CK.tile0 .. tile0 + tileN - 1 (0: all).
     template <class Launch>
     void run(dvr::CkptParams CK, const Scratch& scr, hipStream_t s, Launch launch) const
     {
-        if (bytes_ == 0 || scr.bytes < bytes_) return launch(CK);
-        float* brick = (float*)scr.data;
-        const size_t brickAll = brickFloats_ * volumes_;
-        CK.as.rays = brick + brickAll;
-        CK.as.adj = CK.as.rays + size_t(group_) * dvr::kRayRecord * dvr::kBlock;
-        CK.as.cap = cap_;
-        check_hip(dvr::launch_clear(brick, brickAll, s), "clear launch");
-        for (int t0 = 0; t0 < tiles_; t0 += group_) {
+        if (bytes_ == 0 || scr.bytes < bytes_) return launch(A_, CK);
+        float* base = (float*)scr.data;
+        float* brick = base + sums_;
+        dvr::AdjointParams A = A_;
+        if (sums_ > 0) A.atfSum = (double*)base;
+        check_hip(dvr::launch_clear(base, sums_ + brickFloats_ * volumes_, s), "clear launch");
+        if (group_ == 0) launch(A, CK);
+        else {
+            CK.as.rays = brick + brickFloats_ * volumes_;
+            CK.as.adj = CK.as.rays + size_t(group_) * dvr::kRayRecord * dvr::kBlock;
+            CK.as.cap = cap_;
+        }
+        for (int t0 = 0; group_ > 0 && t0 < tiles_; t0 += group_) {
             CK.tile0 = t0;
             CK.tileN = std::min(group_, tiles_ - t0);
-            launch(CK);
+            launch(A, CK);
             dvr::ScatterParams S;
             std::memset(&S, 0, sizeof(S));
             S.S = CK.as;
@@ -644,15 +638,39 @@ public:
             S.X = c_.X; S.Y = c_.Y; S.Z = c_.Z;
             check_hip(dvr::launch_scatter_volume(S, c_.filter, s), "scatter launch");
         }
-        const dvr::DebrickSeg D{brick, A_.avol, c_.X, c_.Y, c_.Z, 0, A_.avSx, A_.avSy, A_.avSz};
-        check_hip(dvr::launch_debrick_call(D, volumes_, A_.avSb, s), "debrick launch");
+        if (group_ > 0) {
+            const dvr::DebrickSeg D{brick, A.avol, c_.X, c_.Y, c_.Z, 0, A.avSx, A.avSy, A.avSz};
+            check_hip(dvr::launch_debrick_call(D, volumes_, A.avSb, s), "debrick launch");
+        }
+        if (sums_ > 0)
+            check_hip(dvr::launch_add_tf_sums(A.atfSum, A, c_.B, c_.P.R, c_.P.C, s), "TF gradient launch");
     }
 
 private:
+    // sums pay two small launches from as many tiles on
+    static constexpr int kSumTiles = 1024;
+
+    void plan_volume()
+    {
+        // the store holds the longest ray of a uniform box and step; clearing and adding the bricks
+        // (16 bytes a voxel) pays from a few samples per ten voxels on
+        if (!A_.avol || c_.P.st || c_.P.bsize) return;
+        const int volumes = A_.avSb != 0 ? c_.B : 1;
+        if (!distinct_elements(c_, A_, volumes)) return;
+        const double voxels = double(c_.X) * c_.Y * c_.Z * volumes;
+        const int cap = dvr::adj_store_cap(density_cap(c_));
+        if (double(c_.B) * c_.W * c_.H * cap * 0.5 < 0.25 * voxels) return;
+        const size_t perTile = dvr::adj_store_floats(cap), brick = dvr::brick_floats(c_.X, c_.Y, c_.Z);
+        const int group = int(std::min<size_t>(size_t(tiles_), kMaxStore / (perTile * sizeof(float))));
+        // groups too small to fill the chip; 32-bit byte offsets
+        if (group < std::min(tiles_, 4096) || brick >= (size_t(1) << 30)) return;
+        volumes_ = volumes; cap_ = cap; perTile_ = perTile; brickFloats_ = brick; group_ = group;
+    }
+
     const Checked& c_;
     const dvr::AdjointParams& A_;
-    int volumes_ = 1, tiles_ = 0, cap_ = 0, group_ = 0;
-    size_t brickFloats_ = 0, bytes_ = 0;
+    int tiles_ = 0, volumes_ = 1, cap_ = 0, group_ = 0;  // group_ 0: no second pass
+    size_t sums_ = 0, perTile_ = 0, brickFloats_ = 0, bytes_ = 0;
 };
 
 // The packed kernels of pre-shaded volumes (A NULL: the forward).  Scratch layout: [RGBA volume], and for
@@ -661,7 +679,7 @@ class PackedPreshaded {
 public:
     PackedPreshaded(const Checked& c, const dvr::AdjointParams* A) : c_(c), A_(A)
     {
-        // packing moves 32 bytes a voxel: the rule of TwoPassGradient
+        // packing moves 32 bytes a voxel: the rule of AdjointScratch
         const double voxels = double(c.X) * c.Y * c.Z;
         cap_ = dvr::adj_store_cap(density_cap(c));
         tiles_ = group_ = dvr::tiled_num_tiles(c.P);
@@ -845,9 +863,8 @@ void do_adjoint(const dvr_inputs* inputs, const dvr_outputs* fwd, const dvr_tens
     }
     dvr::LossParams L;
     std::memset(&L, 0, sizeof(L));
-    const TwoPassGradient vol(c, A);
-    vol.run(CK, scr, s, [&](const dvr::CkptParams& ck) {
-        check_hip(dvr::launch_adjoint_tiled(c.P, A, ck, L, false, fromFwd, c.filter, c.tfm, c.blend, s),
+    AdjointScratch(c, A).run(CK, scr, s, [&](const dvr::AdjointParams& a, const dvr::CkptParams& ck) {
+        check_hip(dvr::launch_adjoint_tiled(c.P, a, ck, L, false, fromFwd, c.filter, c.tfm, c.blend, s),
                   "adjoint (tiled) launch");
     });
 }
@@ -1281,7 +1298,7 @@ int64_t dvr_adjoint_scratch_bytes(const dvr_inputs* inputs, const dvr_outputs* o
         Checked c = check_inputs(inputs);
         const dvr::AdjointParams A = check_adjoint(c, outputs_from_forward, adj_color, adj_outputs);
         if (c.preshaded) r = int64_t(PackedPreshaded(c, &A).bytes());
-        else r = adjoint_method(c, options) == DVR_ADJOINT_CHECKPOINT ? int64_t(TwoPassGradient(c, A).bytes()) : 0;
+        else r = adjoint_method(c, options) == DVR_ADJOINT_CHECKPOINT ? int64_t(AdjointScratch(c, A).bytes()) : 0;
     });
     return r;
 }

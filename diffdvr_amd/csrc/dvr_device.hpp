@@ -422,20 +422,34 @@ struct Tf {
     int R, C, sr, sc;
 };
 
-// Columns of a TF table per mode (identity, texture, linear, Gaussian); LDS
-// copies are staged densely, so kernels that read them pass this constant as
-// row stride and the row addressing needs no multiply.
+// Columns of a TF table per mode (identity, texture, linear, Gaussian)
 template <int TFM>
 constexpr int tf_cols()
 {
     return TFM == 0 ? 2 : (TFM == 1 ? 4 : (TFM == 2 ? 5 : 6));
 }
-// Row stride of a TF staged in LDS by the batched kernel: the linear TF's rows
-// are padded to 8 floats so a row's RGBA is one 16-byte LDS read.
+// Row stride of a TF staged in LDS (a constant: the row addressing needs no
+// multiply).  Linear and Gaussian rows take 8 floats, so a row's RGBA is one
+// 16-byte read.  A Gaussian row holds red, green, blue, absorption, the mean mu
+// and, instead of the deviation s, what the FAST instances form from it for every
+// sample and row otherwise: log2 e / (2 s^2), 1 / s^2 and 1 / s.
 template <int TFM>
 constexpr int tf_lds_stride()
 {
-    return TFM == 2 ? 8 : tf_cols<TFM>();
+    return tf_lds_row_floats(TFM, tf_cols<TFM>());
+}
+// entry (r, c) of a TF into its staged table
+template <int TFM>
+__device__ __forceinline__ void tf_stage_entry(float* s_tf, int r, int c, float v)
+{
+    float* row = s_tf + r * tf_lds_stride<TFM>();
+    if (TFM == 3 && c == 5) {
+        row[5] = 1.44269504088896341f * __builtin_amdgcn_rcpf(2.0f * v * v);
+        row[6] = 1.0f / (v * v);
+        row[7] = 1.0f / v;
+    } else {
+        row[c] = v;
+    }
 }
 
 // Interval of a piecewise-linear TF that holds a density: rows i and i+1, their
@@ -468,8 +482,8 @@ __device__ __forceinline__ TfLoc tf_linear_locate(const Tf& T, float density)
     return tf_linear_row<FAST>(T, i);
 }
 
-// One Gaussian component's weight exp(-(d - mu)^2 / (2 s^2)); FAST multiplies by
-// v_rcp_f32's reciprocal instead of dividing and evaluates 2^(-z log2 e) on the
+// One Gaussian component's weight exp(-(d - mu)^2 / (2 s^2)); FAST takes the staged
+// scale log2 e / (2 s^2) in place of s and evaluates 2^(-z log2 e) on the
 // hardware base-2 exponential, z = (d - mu)^2 / (2 s^2) (relative error about
 // z * 1e-7, below 2e-6 for the weights above 1e-8), in one expression for the
 // value, the absorption and the adjoint, so the three agree bitwise.
@@ -477,8 +491,7 @@ template <bool FAST>
 __device__ __forceinline__ float gauss_n(float density, float mu, float s)
 {
     if constexpr (FAST)
-        return __builtin_amdgcn_exp2f(-(density - mu) * (density - mu) *
-                                      (1.44269504088896341f * __builtin_amdgcn_rcpf(2.0f * s * s)));
+        return __builtin_amdgcn_exp2f(-(density - mu) * (density - mu) * s);
     else return expf(-(density - mu) * (density - mu) / (2.0f * s * s));
 }
 
@@ -818,12 +831,11 @@ __device__ __forceinline__ float tf_adjoint(const Tf& T, float density, const f4
             const float* r = T.p + i * T.sr;
             const float c0 = r[0], c1 = r[T.sc], c2 = r[2 * T.sc], c3 = r[3 * T.sc];
             const float mu = r[4 * T.sc], s = r[5 * T.sc];
-            const float s2 = s * s;
-            const float f1 = FAST ? (mu - density) * __builtin_amdgcn_rcpf(s2) * n : (mu - density) / s2 * n;
+            const float f1 = FAST ? (mu - density) * r[6 * T.sc] * n : (mu - density) / (s * s) * n;
             const float g = adj.x * (c0 * f1) + adj.y * (c1 * f1) + adj.z * (c2 * f1) + adj.w * (c3 * f1);
             adj_d += g;
             if constexpr (WANT_TF) {
-                const float f2 = FAST ? f1 * (mu - density) * __builtin_amdgcn_rcpf(s) : f1 * (mu - density) / s;
+                const float f2 = FAST ? f1 * (mu - density) * r[7 * T.sc] : f1 * (mu - density) / s;
                 sink.add(i, 0, adj.x * n);
                 sink.add(i, 1, adj.y * n);
                 sink.add(i, 2, adj.z * n);

@@ -106,6 +106,39 @@ hipError_t launch_debrick_call(const DebrickSeg& S, int batches, long long sb, h
     return hipGetLastError();
 }
 
+// blockIdx.y = segment
+__global__ __launch_bounds__(256) void k_add_sums(const SumSeg* segs)
+{
+    const SumSeg S = segs[blockIdx.y];
+    for (int i = blockIdx.x * 256 + threadIdx.x; i < S.n; i += gridDim.x * 256)
+        atomicAdd(S.dst + i, float(S.sum[i]));  // tables may share a gradient
+}
+// the TF gradients of one call: batch, row and column strides of its tensor
+__global__ __launch_bounds__(256) void k_add_tf_sums(const double* sum, float* dst, int n, int RC, int C, int sb, int sr,
+                                                     int sc)
+{
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= n) return;
+    const int b = i / RC, e = i - b * RC, r = e / C, c = e - r * C;
+    atomicAdd(dst + b * sb + r * sr + c * sc, float(sum[i]));  // an expanded gradient shares elements
+}
+
+hipError_t launch_add_sums(const SumSeg* dSegs, int nSegs, int maxN, hipStream_t s)
+{
+    if (nSegs == 0) return hipSuccess;
+    hipLaunchKernelGGL(k_add_sums, dim3(unsigned((maxN + 255) / 256), unsigned(nSegs)), dim3(256), 0, s, dSegs);
+    return hipGetLastError();
+}
+
+hipError_t launch_add_tf_sums(const double* sum, const AdjointParams& A, int B, int R, int C, hipStream_t s)
+{
+    const int n = (A.atfSb != 0 ? B : 1) * R * C;
+    if (n == 0) return hipSuccess;
+    hipLaunchKernelGGL(k_add_tf_sums, dim3(unsigned((n + 255) / 256)), dim3(256), 0, s, sum, A.atf, n, R * C, C, A.atfSb,
+                       A.atfSr, A.atfSc);
+    return hipGetLastError();
+}
+
 hipError_t launch_debrick(const DebrickSeg* dSegs, int nSegs, long long maxBricks, hipStream_t s)
 {
     if (nSegs <= 0) return hipSuccess;

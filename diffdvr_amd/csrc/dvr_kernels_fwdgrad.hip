@@ -73,8 +73,8 @@ __device__ __forceinline__ void tf_deriv(const Tf& T, float density, f4& ds, con
         const int di = int(floorf(d));
         const float df = d - float(di);
         const int i0 = iclamp(di, 0, T.R - 1), i1 = iclamp(di + 1, 0, T.R - 1);
-        const float* a = T.p + i0 * C;
-        const float* c = T.p + i1 * C;
+        const float* a = T.p + i0 * T.sr;
+        const float* c = T.p + i1 * T.sr;
         const float R = float(T.R);
         ds = mk4((c[0] - a[0]) * R, (c[1] - a[1]) * R, (c[2] - a[2]) * R, (c[3] - a[3]) * R);
 #pragma unroll
@@ -87,9 +87,9 @@ __device__ __forceinline__ void tf_deriv(const Tf& T, float density, f4& ds, con
     } else if constexpr (TFM == 2) {
         int i;
         for (i = 0; i < T.R - 2; ++i)
-            if (T.p[(i + 1) * C + 4] > density) break;
-        const float* a = T.p + i * C;
-        const float* c = a + C;
+            if (T.p[(i + 1) * T.sr + 4] > density) break;
+        const float* a = T.p + i * T.sr;
+        const float* c = a + T.sr;
         const float p0 = a[4], p1 = c[4];
         const float d2 = fclamp(density, p0, p1);
         const float f = (d2 - p0) / (p1 - p0);
@@ -112,10 +112,10 @@ __device__ __forceinline__ void tf_deriv(const Tf& T, float density, f4& ds, con
     } else {
         ds = mk4(0.f, 0.f, 0.f, 0.f);
         for (int i = 0; i < T.R; ++i) {
-            const float* r = T.p + i * C;
-            const float mu = r[4], sg = r[5];
-            const float n = gauss_n<true>(density, mu, sg);  // as the colour (tf_eval<3, true>)
-            const float dn = n * (mu - density) / (sg * sg);
+            const float* r = T.p + i * T.sr;
+            const float mu = r[4];
+            const float n = gauss_n<true>(density, mu, r[5]);  // as the colour (tf_eval<3, true>)
+            const float dn = n * (mu - density) * r[6];
             ds.x += r[0] * dn; ds.y += r[1] * dn; ds.z += r[2] * dn; ds.w += r[3] * dn;
 #pragma unroll
             for (int k = 0; k < NE; ++k) {
@@ -127,7 +127,7 @@ __device__ __forceinline__ void tf_deriv(const Tf& T, float density, f4& ds, con
                 else if (col == 3) de[k].w = n;
                 else {
                     const float dd = density - mu;
-                    const float q = col == 4 ? n * dd / (sg * sg) : n * dd * dd / (sg * sg * sg);
+                    const float q = col == 4 ? n * dd * r[6] : n * dd * dd * r[6] * r[7];
                     de[k] = mk4(r[0] * q, r[1] * q, r[2] * q, r[3] * q);
                 }
             }
@@ -141,7 +141,7 @@ __global__ __launch_bounds__(kBlock) void k_forward_gradients(RenderParams P, Fw
 {
     extern __shared__ float lds[];
     const TileXY tc = tile_xy(tilesX, tilesPerView, nTiles);
-    stage_tf(P, tc.b, lds);
+    stage_tf<TFM>(P, tc.b, lds);
     __syncthreads();
     if (tc.x >= P.W || tc.y >= P.H) return;
     const int b = tc.b, x = tc.x, y = tc.y;
@@ -156,7 +156,7 @@ __global__ __launch_bounds__(kBlock) void k_forward_gradients(RenderParams P, Fw
     const Ray r = setup_ray(P, x, y, b);
     const Vol V = make_vol(P, b);
     constexpr int kC = tf_cols<TFM>();
-    const Tf T{lds, P.R, kC, kC, 1};
+    const Tf T{lds, P.R, kC, tf_lds_stride<TFM>(), 1};
     // derivative seeds of slot k (uniform): step, start (3), direction (3)
     float sStep[kFwdChunk];
     f3 sStart[kFwdChunk], sDir[kFwdChunk];
@@ -270,13 +270,13 @@ __global__ __launch_bounds__(kBlock) void k_forward_gradients_gauss(RenderParams
         s_c[k][1] = make_float4(e >= 0 && col == 5 ? 1.0f / (sg * sg * sg) : 0.0f,
                                 col < 4 ? (col == 3 ? 1.0f : 0.0f) : r[3 * P.tfSc], 0.0f, 0.0f);
     }
-    stage_tf(P, b, lds);
+    stage_tf<3>(P, b, lds);
     __syncthreads();
     if (x >= P.W || y >= P.H) return;
 
     const Ray r = setup_ray(P, x, y, b);
     const Vol V = make_vol(P, b);
-    const Tf T{lds, P.R, kC, kC, 1};
+    const Tf T{lds, P.R, kC, tf_lds_stride<3>(), 1};
     Acc acc{0.f, 0.f, 0.f, 0.f, 1.f};
     float dr[kFwdChunk], dg[kFwdChunk], db[kFwdChunk], dA[kFwdChunk], dT[kFwdChunk], sf[kFwdChunk];
 #pragma unroll
@@ -350,7 +350,7 @@ static hipError_t fwdgrad_t(const RenderParams& P, const FwdGradParams& G, hipSt
     const int nTiles = tilesX * tilesY * P.B;
     if (nTiles == 0 || G.D == 0) return hipSuccess;
     const int chunks = (G.D + kFwdChunk - 1) / kFwdChunk;
-    const size_t lds = sizeof(float) * size_t(P.R) * P.C;
+    const size_t lds = sizeof(float) * size_t(P.R) * tf_lds_stride<TFM>();
     if constexpr (TFM == 3) {
         const bool rays = G.dStep >= 0 || std::max({G.dStart[0], G.dStart[1], G.dStart[2]}) >= 0 ||
                           std::max({G.dDir[0], G.dDir[1], G.dDir[2]}) >= 0;

@@ -61,7 +61,7 @@ static hipError_t fwd_row_t(const RenderParams& P, const CkptParams& CK, hipStre
     const int tilesX = (P.W + kTileW - 1) / kTileW, tilesY = (P.H + kTileH - 1) / kTileH;
     const int nTiles = tilesX * tilesY * P.B;
     if (nTiles == 0) return hipSuccess;
-    const size_t lds = sizeof(float) * size_t(P.R) * P.C;
+    const size_t lds = sizeof(float) * size_t(P.R) * tf_lds_stride<TFM>();
     hipLaunchKernelGGL((k_forward_row<FILTER, TFM, BLEND>), dim3(nTiles * row_blocks_per_tile(kRowBlock)),
                        dim3(kRowBlock), lds, s, P, CK, tilesX, tilesX * tilesY, nTiles);
     return hipGetLastError();
@@ -86,10 +86,11 @@ static hipError_t adj_row_g(const RenderParams& P, const AdjointParams& A, const
     const int copyStride = tf_grad_copy_stride(RC);
     const int ng = A.atf ? tf_grad_floats(RC, usePriv, kThreads, copyStride) : 0;
     int aggLog2 = kAggLog2;
-    size_t lds = sizeof(float) * size_t(tf_grad_offset(RC) + ng);
+    const int tfFloats = tf_grad_offset(P.R * tf_lds_stride<TFM>());
+    size_t lds = sizeof(float) * size_t(tfFloats + ng);
     if ((GM & 2) && A.avol) {
         // the largest chunk table per wave beside the TF tables that leaves room for sixteen waves per CU
-        const size_t base = sizeof(float) * size_t(agg_offset(tf_grad_offset(RC), ng));
+        const size_t base = sizeof(float) * size_t(agg_offset(tfFloats, ng));
         constexpr size_t kWaves = kThreads / 64;
         while (aggLog2 > kAggMinLog2 && base + kWaves * agg_bytes(aggLog2, sizeof(float)) > size_t(kLdsPerCu) * kWaves / kTiledVolWgPerCu)
             --aggLog2;

@@ -94,6 +94,9 @@ hipError_t launch_debrick(const DebrickSeg* dSegs, int nSegs, long long maxBrick
 hipError_t launch_debrick_call(const DebrickSeg& S, int batches, long long sb, hipStream_t s);
 // dvr_kernels_scatter.hip: the second pass of the volume gradients (P.parts is chosen here)
 hipError_t launch_scatter_volume(const ScatterParams& P, int filter, hipStream_t s, int channels = 1);
+// sums of doubles added into the caller's gradients: a plan's segments, one call's TF gradient
+hipError_t launch_add_sums(const SumSeg* dSegs, int nSegs, int maxN, hipStream_t s);
+hipError_t launch_add_tf_sums(const double* sum, const AdjointParams& A, int B, int R, int C, hipStream_t s);
 // clears n floats (a multiple of 4, 16-byte aligned) with a kernel
 hipError_t launch_clear(float* p, size_t n, hipStream_t s);
 

@@ -17,6 +17,8 @@ constexpr int kTfCopies = 4;      // copies of the LDS TF-gradient table, lane &
 // 3 to 4 clocks each either way).
 // TF gradients: doubles between the copies (odd: the copies start in different banks), 0 = one table (copies
 // would take more than 16 KiB); 8-byte aligned offset behind the TF table; floats in all
+// floats of a staged row of a TF of that mode with `cols` columns (see tf_lds_stride)
+constexpr int tf_lds_row_floats(int tfm, int cols) { return tfm >= 2 ? 8 : cols; }
 constexpr int tf_grad_copy_stride(int RC) { return kTfCopies * (RC | 1) * 8 <= 16384 ? (RC | 1) : 0; }
 constexpr int tf_grad_offset(int tfFloats) { return (tfFloats + 1) & ~1; }
 constexpr int tf_grad_floats(int RC, bool priv, int threads, int stride)
@@ -85,6 +87,7 @@ struct AdjointParams {
     float* ars; int arsSb, arsSy, arsSx, arsSc;
     float* ard; int ardSb, ardSy, ardSx, ardSc; int camBroadcast;
     float* atf; int atfSb, atfSr, atfSc;
+    double* atfSum;             // [batch][R*C] sums of the call, added into atf after it, or NULL
     int tfDelayed;
 };
 
@@ -187,7 +190,14 @@ struct ScatterParams {
 struct BTf {
     const float* p;
     float* adj;                 // gradient (accumulated) or NULL
+    double* sum;                // the plan's sums of a run, added into adj after it
     int R, C;
+};
+// Sums of doubles added into a caller's floats
+struct SumSeg {
+    const double* sum;
+    float* dst;
+    int n, pad0;
 };
 
 struct BatchParams {
@@ -200,7 +210,7 @@ struct BatchParams {
     int dsCap;                  // samples per ray the density store holds
     AdjStore as;                // density adjoints of the launch's tiles (volume gradients), or NULL
     int tile0;                  // first tile of the launch
-    float* lossOut;             // scalar loss accumulator or NULL
+    double* lossOut;            // the plan's sum of the loss, or NULL
     int nViews, nTiles, ckCap;
     int ckEvery;                // checkpoint interval = K * ckEvery samples
     int qBegin[kNumXcd + 1];    // tile range of each XCD's queue

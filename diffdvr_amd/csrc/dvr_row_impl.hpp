@@ -338,13 +338,13 @@ __global__ __launch_bounds__(kRowBlock) void k_forward_row(RenderParams P, CkptP
     extern __shared__ float lds[];
     __shared__ __attribute__((aligned(16))) float s_x[kRowXchgFloats];
     const RowXY tc = row_xy<kRowBlock>(tilesX, tilesPerView, nTiles);
-    stage_tf(P, tc.b, lds);
+    stage_tf<TFM>(P, tc.b, lds);
     __syncthreads();
     const bool valid = tc.x < P.W && tc.y < P.H;
     const Ray r = setup_ray(P, min(tc.x, P.W - 1), min(tc.y, P.H - 1), tc.b);
     const Vol V = make_vol(P, tc.b);
     constexpr int kC = tf_cols<TFM>();
-    const Tf T{lds, P.R, kC, kC, 1};
+    const Tf T{lds, P.R, kC, tf_lds_stride<TFM>(), 1};
     float* ck = CK.buf ? CK.buf + (size_t(tc.tile) * CK.cap) * kBlock + tc.slot : nullptr;
     float* ds = CK.ds ? CK.ds + (size_t(tc.tile) * CK.dsCap) * kBlock + tc.slot : nullptr;
     float channel;
@@ -371,11 +371,12 @@ __global__ __launch_bounds__(kRowAdjBlock) __attribute__((amdgpu_waves_per_eu(GM
     float* xc = s_x + (threadIdx.x / kRow) * kRowXchg;
     const int RC = P.R * P.C;
     float* s_tf = lds;
-    float* s_g = lds + tf_grad_offset(RC);
+    const int tfFloats = tf_grad_offset(P.R * tf_lds_stride<TFM>());
+    float* s_g = lds + tfFloats;
     const RowXY tc = row_xy<kThreads>(tilesX, tilesPerView, nTiles);
     const bool wantTf = (GM & 1) && A.atf != nullptr;
     const int ng = wantTf ? tf_grad_floats(RC, usePriv != 0, kThreads, copyStride) : 0;
-    stage_tf(P, tc.b, s_tf);
+    stage_tf<TFM>(P, tc.b, s_tf);
     for (int e = threadIdx.x; e < ng; e += kThreads) s_g[e] = 0.0f;
     constexpr bool kVolInst = (GM & 2) != 0;
     using VS = std::conditional_t<kVolInst, VolAgg<LinearLayout, float>, VolDirect>;
@@ -384,7 +385,7 @@ __global__ __launch_bounds__(kRowAdjBlock) __attribute__((amdgpu_waves_per_eu(GM
     const bool aggOn = kVolInst && A.avol != nullptr;
     if constexpr (kVolInst) {
         if (aggOn) {
-            char* table = reinterpret_cast<char*>(lds + agg_offset(tf_grad_offset(RC), ng));
+            char* table = reinterpret_cast<char*>(lds + agg_offset(tfFloats, ng));
             vs.init(table + (threadIdx.x >> 6) * agg_bytes(aggLog2, sizeof(float)), aggLog2);
             vs.bind(A.avol + tc.b * A.avSb);
         }
@@ -398,7 +399,7 @@ __global__ __launch_bounds__(kRowAdjBlock) __attribute__((amdgpu_waves_per_eu(GM
     const Ray r = setup_ray(P, x, y, b);
     const Vol V = make_vol(P, b);
     constexpr int kC = tf_cols<TFM>();
-    const Tf T{s_tf, P.R, kC, kC, 1};
+    const Tf T{s_tf, P.R, kC, tf_lds_stride<TFM>(), 1};
     const int ckShift = __builtin_ctz(CK.K * CK.every);
     float* ck = CK.buf + (size_t(tc.tile) * CK.cap) * kBlock + tc.slot;
     float* ds = CK.ds ? CK.ds + (size_t(tc.tile) * CK.dsCap) * kBlock + tc.slot : nullptr;
@@ -498,7 +499,6 @@ __global__ __launch_bounds__(kRowAdjBlock) __attribute__((amdgpu_waves_per_eu(GM
     }
     if (wantTf) {
         __syncthreads();
-        float* g = A.atf + b * A.atfSb;
         if (usePriv) {  // a wave sums the threads' slices of an entry
             const int lane = threadIdx.x & 63;
             for (int e = threadIdx.x >> 6; e < RC; e += kThreads / 64) {
@@ -506,14 +506,11 @@ __global__ __launch_bounds__(kRowAdjBlock) __attribute__((amdgpu_waves_per_eu(GM
 #pragma unroll
                 for (int k = 0; k < kThreads / 64; ++k) v += s_g[e * kThreads + k * 64 + lane];
                 v = wave_sum(v);
-                const int rr = e / P.C, cc = e - rr * P.C;
-                if (lane == 0 && v != 0.0f) atomicAdd(g + rr * A.atfSr + cc * A.atfSc, v);
+                if (lane == 0) tf_grad_add(P, A, b, e, v);
             }
         } else {
             for (int e = threadIdx.x; e < RC; e += kThreads) {
-                const float v = tf_grad_sum(s_g, e, copyStride);
-                const int rr = e / P.C, cc = e - rr * P.C;
-                if (v != 0.0f) atomicAdd(g + rr * A.atfSr + cc * A.atfSc, v);
+                tf_grad_add(P, A, b, e, tf_grad_sum(s_g, e, copyStride));
             }
         }
     }

@@ -37,13 +37,14 @@ __device__ __forceinline__ TileXY tile_xy(int tilesX, int tilesPerView, int nTil
     return t;
 }
 
+template <int TFM>
 __device__ __forceinline__ void stage_tf(const RenderParams& P, int b, float* s_tf)
 {
     const float* g = P.tf + b * P.tfSb;
-    const int RC = P.R * P.C;
-    for (int e = threadIdx.x; e < RC; e += blockDim.x) {
-        const int r = e / P.C, c = e - r * P.C;
-        s_tf[e] = g[r * P.tfSr + c * P.tfSc];
+    constexpr int kC = tf_cols<TFM>();
+    for (int e = threadIdx.x; e < P.R * kC; e += blockDim.x) {
+        const int r = e / kC, c = e - r * kC;
+        tf_stage_entry<TFM>(s_tf, r, c, g[r * P.tfSr + c * P.tfSc]);
     }
 }
 
@@ -193,7 +194,7 @@ struct SinkTiled {
 };
 
 // sum of entry e over the copies of the workgroup's table
-__device__ __forceinline__ float tf_grad_sum(const float* s_g, int e, int copyStride)
+__device__ __forceinline__ double tf_grad_sum(const float* s_g, int e, int copyStride)
 {
     const double* t = reinterpret_cast<const double*>(s_g) + e;
     double v = t[0];
@@ -201,7 +202,20 @@ __device__ __forceinline__ float tf_grad_sum(const float* s_g, int e, int copySt
 #pragma unroll
         for (int k = 1; k < kTfCopies; ++k) v += t[k * copyStride];
     }
-    return float(v);
+    return v;
+}
+// Adds a workgroup's sum of entry e of batch b: into the call's doubles, or (without call scratch) the
+// gradient.  Thousands of workgroups add to one entry: the order of float additions there gave errors of
+// 2e-6 of the gradient.
+__device__ __forceinline__ void tf_grad_add(const RenderParams& P, const AdjointParams& A, int b, int e, double v)
+{
+    if (v == 0.0) return;
+    if (A.atfSum) {
+        atomicAdd(A.atfSum + (A.atfSb != 0 ? b * P.R * P.C : 0) + e, v);
+    } else {
+        const int rr = e / P.C, cc = e - rr * P.C;
+        atomicAdd(A.atf + b * A.atfSb + rr * A.atfSr + cc * A.atfSc, float(v));
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -852,13 +866,13 @@ __global__ __launch_bounds__(kBlock) void k_forward_tiled(RenderParams P, CkptPa
 {
     extern __shared__ float lds[];
     const TileXY tc = tile_xy(tilesX, tilesPerView, nTiles);
-    stage_tf(P, tc.b, lds);
+    stage_tf<TFM>(P, tc.b, lds);
     __syncthreads();
     if (tc.x >= P.W || tc.y >= P.H) return;
     const Ray r = setup_ray(P, tc.x, tc.y, tc.b);
     const Vol V = make_vol(P, tc.b);
     constexpr int kC = tf_cols<TFM>();
-    const Tf T{lds, P.R, kC, kC, 1};
+    const Tf T{lds, P.R, kC, tf_lds_stride<TFM>(), 1};
     float* ck = CK.buf ? CK.buf + (size_t(tc.tile) * CK.cap) * kBlock + threadIdx.x : nullptr;
     float* ds = CK.ds ? CK.ds + (size_t(tc.tile) * CK.dsCap) * kBlock + threadIdx.x : nullptr;
     Acc acc;
@@ -881,12 +895,13 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(GM == 3 
     extern __shared__ float lds[];
     const int RC = P.R * P.C;
     float* s_tf = lds;
-    float* s_g = lds + tf_grad_offset(RC);
+    const int tfFloats = tf_grad_offset(P.R * tf_lds_stride<TFM>());
+    float* s_g = lds + tfFloats;
     const int copyStride = tf_grad_copy_stride(RC);
     const TileXY tc = tile_xy(tilesX, tilesPerView, nTiles, CK.tile0);
     const bool wantTf = A.atf != nullptr;
     const int ng = wantTf ? tf_grad_floats(RC, usePriv != 0, kBlock, copyStride) : 0;
-    stage_tf(P, tc.b, s_tf);
+    stage_tf<TFM>(P, tc.b, s_tf);
     for (int e = threadIdx.x; e < ng; e += kBlock) s_g[e] = 0.0f;
     // volume gradient: the wave's corner values are summed per 64-byte chunk in LDS
     constexpr bool kVolInst = (GM & 2) != 0;
@@ -896,7 +911,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(GM == 3 
     const bool aggOn = kVolInst && A.avol != nullptr;
     if constexpr (kVolInst) {
         if (aggOn) {
-            vs.init(lds + agg_offset(tf_grad_offset(RC), ng), aggLog2);
+            vs.init(lds + agg_offset(tfFloats, ng), aggLog2);
             vs.bind(A.avol + tc.b * A.avSb);
         }
     }
@@ -911,7 +926,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(GM == 3 
         const Ray r = setup_ray(P, x, y, b);
         const Vol V = make_vol(P, b);
         constexpr int kC = tf_cols<TFM>();
-        const Tf T{s_tf, P.R, kC, kC, 1};
+        const Tf T{s_tf, P.R, kC, tf_lds_stride<TFM>(), 1};
         float* ck = CK.buf + (size_t(tc.tile) * CK.cap) * kBlock + threadIdx.x;
         // density store: written by this kernel's forward march (fused, or replayed without
         // checkpoints) or by the forward launch that wrote the checkpoints
@@ -995,17 +1010,15 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(GM == 3 
     }
     if (wantTf) {
         __syncthreads();
-        float* g = A.atf + tc.b * A.atfSb;
         for (int e = threadIdx.x; e < RC; e += kBlock) {
-            float v;
+            double v;
             if (usePriv) {
-                v = 0.0f;
-                for (int t = 0; t < kBlock; ++t) v += s_g[e * kBlock + t];
+                v = 0.0;
+                for (int t = 0; t < kBlock; ++t) v += double(s_g[e * kBlock + t]);
             } else {
                 v = tf_grad_sum(s_g, e, copyStride);
             }
-            const int rr = e / P.C, cc = e - rr * P.C;
-            if (v != 0.0f) atomicAdd(g + rr * A.atfSr + cc * A.atfSc, v);
+            tf_grad_add(P, A, tc.b, e, v);
         }
     }
 }
@@ -1023,10 +1036,11 @@ static hipError_t adj_tiled_k(const RenderParams& P, const AdjointParams& A, con
     const int RC = P.R * P.C;
     const bool usePriv = (TFM == 3) && A.atf && RC <= 48;  // private slices <= 48 KiB of LDS
     const int ng = A.atf ? tf_grad_floats(RC, usePriv, kBlock, tf_grad_copy_stride(RC)) : 0;
+    const int tfFloats = tf_grad_offset(P.R * tf_lds_stride<TFM>());
     int aggLog2 = kAggLog2;
     size_t lds;
     if ((GM & 2) && A.avol) {
-        const size_t base = sizeof(float) * size_t(agg_offset(tf_grad_offset(RC), ng));
+        const size_t base = sizeof(float) * size_t(agg_offset(tfFloats, ng));
         if (GM == 3) {
             // the largest chunk table beside the TF tables that leaves room for sixteen one-wave
             // workgroups per CU (the four waves per SIMD the instance's registers allow)
@@ -1037,7 +1051,7 @@ static hipError_t adj_tiled_k(const RenderParams& P, const AdjointParams& A, con
             lds = occupancy_lds(base + agg_bytes(aggLog2, sizeof(float)), tiled_wg_per_cu(TFM));
         }
     } else {
-        lds = occupancy_lds(sizeof(float) * size_t(tf_grad_offset(RC) + ng), tiled_wg_per_cu(TFM));
+        lds = occupancy_lds(sizeof(float) * size_t(tfFloats + ng), tiled_wg_per_cu(TFM));
     }
     hipLaunchKernelGGL((k_adjoint_tiled<FILTER, TFM, BLEND, K, GM>), dim3(nTiles), dim3(kBlock), lds, s, P, A, CK, L,
                        fused ? 1 : 0, ckFromFwd ? 1 : 0, usePriv ? 1 : 0, tilesX, tilesX * tilesY, nTiles, aggLog2);
