@@ -793,7 +793,12 @@ __device__ __forceinline__ void march_reverse(const Vol& V, const Tf& T, const R
                         if (ix != cc.cx || iy != cc.cy || iz != cc.cz) {
                             if (wantVol && wantPos) corner_move<true, true>(cc, V, vs, ix, iy, iz);
                             else if (wantVol) corner_move<true, false>(cc, V, vs, ix, iy, iz);
-                            else corner_move<false, true>(cc, V, vs, ix, iy, iz);
+                            else if (V.sz == 1) {
+                                // four 8-byte loads beat the face cases' divergent gathers (96 camera views
+                                // 12.6 -> 9.6 ms, with the forward march's pair loads)
+                                cell_load(V, ix, iy, iz, cc.d);
+                                cc.cx = ix; cc.cy = iy; cc.cz = iz;
+                            } else corner_move<false, true>(cc, V, vs, ix, iy, iz);
                         }
                         const float fx = p.x - float(ix), fy = p.y - float(iy), fz = p.z - float(iz);
                         float w[8];
