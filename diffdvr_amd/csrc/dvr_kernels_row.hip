@@ -21,36 +21,39 @@ static float pixel_voxels(const RenderParams& P)
     return float(P.X + P.Y + P.Z) / (3.0f * float(P.W < P.H ? P.W : P.H));
 }
 
-// Few rays leave the tiled kernel's chain of samples exposed: up to 768 tiles the row kernel wins
-// at every size measured (576 tiles: 35 against 84 us through 64^3, 142 against 221 us through
-// 128^3 at quarter-voxel steps).  Beyond, it pays by what the gathers touch: with
-// g = (voxels per pixel) x (voxels per step), 64 neighbouring rays reach further apart than 16
-// consecutive samples where g is large.  Measured, row against tiled, in us: g = 0.125, 64^3,
-// 2048 tiles 101 / 127, 4096 tiles 136 / 124; g = 0.25, 128^3, 4096 tiles 218 / 270, 8192 tiles
-// 411 / 307; g = 0.5, 256^3, 8192 tiles 785 / 1313, 32768 tiles 2824 / 3341; g = 0.44 and 0.6
-// with 160^3 (nearer the 4 MiB L2s), 16384 and 32768 tiles 715 / 669, 1031 / 940; g = 0.35,
-// 256^3, 32768 tiles 2150 / 1896.  A nearest-neighbour sample gathers one voxel, not eight, and
-// has nothing to gain from the last two rules.
+// Few rays leave the tiled kernel's chain of samples exposed: up to 2048 tiles the row kernel wins
+// at every size measured (1024 tiles: 45 against 102 us through 64^3, 122 / 275 through 256^3; 2048
+// tiles 75 / 125 and 214 / 693).  Beyond, it pays by what the gathers touch: with g = (voxels per
+// pixel) x (voxels per step), 64 neighbouring rays reach further apart than 16 consecutive samples
+// where g is large, and more so where the volume exceeds the 4 MiB L2s; short steps leave more
+// samples to overlap.  Measured, row against tiled, in us: g = 0.5, 256^3, 8192 tiles 507 / 1387,
+// 16384 tiles 988 / 2149, 128^3 534 / 640; g = 0.375, 192^3, 691 / 943; g = 0.31, 160^3, 594 / 609;
+// g = 0.25, 256^3, 16384 tiles 892 / 922, 32768 tiles 1742 / 1617, 128^3, 8192 tiles 257 / 243;
+// g = 0.125, 4096 tiles 203 / 221, 8192 tiles 384 / 359; g = 0.06, 4096 tiles 136 / 120; quarter-voxel
+// steps, 8192 tiles 391 / 475, 343 / 350, 16384 tiles 745 / 776, 2385 / 2389.  A nearest-neighbour
+// sample gathers one voxel, not eight, and gains up to 768 tiles.
 bool use_row_forward(const RenderParams& P, int filter)
 {
     const int tiles = tiled_num_tiles(P);
     if (tiles <= 768) return true;
     if (filter != 1 || tiles > kMaxRowTiles) return false;
-    const float g = step_voxels(P) * pixel_voxels(P);
-    if (g >= 0.45f && size_t(P.X) * P.Y * P.Z >= (size_t(6) << 20)) return true;
-    return tiles <= (g >= 0.22f ? 4096 : (g >= 0.11f ? 2048 : 0));
+    const float step = step_voxels(P), g = step * pixel_voxels(P);
+    if (tiles <= 2048 || g >= 0.3f) return true;
+    if (step < 0.4f) return tiles <= 16384;
+    if (g >= 0.24f && size_t(P.X) * P.Y * P.Z >= (size_t(4) << 20)) return tiles <= 16384;
+    return tiles <= (g >= 0.1f ? 4096 : 2048);
 }
 
-// Position gradients alone (row_reverse): 583 against 931 us at 8192 tiles (Gaussian TF, 4 rows),
-// 903 / 925 at 16384 (identity TF), 1899 / 1594 at 32768; with steps below 0.4 voxel 4290 / 5011 at
-// 32768.  Volume gradients (split_reverse): 347 / 917 us at 1024 tiles, 634 / 1038 at 2048,
-// 2707 / 2684 at 4096.  TF gradients: 161 / 279 and 141 / 199 us at 1024 tiles, 265 / 247 at 2048;
-// the identity TF's walk is short, 53 / 65 at 576 and 83 / 67 at 1024.
-bool use_row_adjoint(const RenderParams& P, const AdjointParams& A, int tfm)
+// Position gradients alone (row_reverse): 220 against 636 us at 2048 tiles, 486 / 786 at 8192, 947 /
+// 1295 at 16384 (Gaussian TF, 4 rows); with steps below 0.4 voxel 4290 / 5011 at 32768.  Volume
+// gradients (split_reverse) in two passes: 185 / 262 and 273 / 277 us at 1024 tiles, 415 / 350 at
+// 2048; in one pass 634 / 1038 at 2048, 2707 / 2684 at 4096.  TF gradients: 137 / 160 us at 1024
+// tiles, 238 / 184 at 2048; the identity TF's walk is short, 53 / 65 at 576 and 83 / 67 at 1024.
+bool use_row_adjoint(const RenderParams& P, const AdjointParams& A, const CkptParams& CK, int tfm)
 {
     const int tiles = tiled_num_tiles(P);
     if (tiles > kMaxRowTiles) return false;
-    if (A.avol) return tiles <= 2048;
+    if (A.avol) return tiles <= (CK.as.adj ? 1024 : 2048);
     if (A.atf) return tiles <= (tfm == 0 && !A.ars && !A.ast ? 768 : 1024);
     return tiles <= 16384 || step_voxels(P) < 0.4f;
 }

@@ -64,7 +64,7 @@ hipError_t launch_adjoint_tiled(const RenderParams& P, const AdjointParams& A, c
 
 // dvr_kernels_row.hip: the same, 16 lanes a ray, and the sizes at which they are faster
 bool use_row_forward(const RenderParams& P, int filter);
-bool use_row_adjoint(const RenderParams& P, const AdjointParams& A, int tfm);
+bool use_row_adjoint(const RenderParams& P, const AdjointParams& A, const CkptParams& CK, int tfm);
 hipError_t launch_forward_row(const RenderParams& P, const CkptParams& CK, int filter, int tfm, int blend,
                               hipStream_t s);
 hipError_t launch_adjoint_row(const RenderParams& P, const AdjointParams& A, const CkptParams& CK, const LossParams& L,
