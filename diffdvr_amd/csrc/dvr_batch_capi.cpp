@@ -61,7 +61,7 @@ int wave_shift_of(int ww)
 // 900-sample rays then run in groups of 37 000), and groups a run may be cut into.
 constexpr long long kMaxAdjointStore = 8LL << 30;
 constexpr int kMaxGroups = 64;
-constexpr double kMaxSampleDensity = 16.0;
+constexpr double kMaxRayDensity = 5.5;
 
 int tf_cols(int tfm)
 {
@@ -87,7 +87,7 @@ struct dvr_batch_plan {
     std::vector<dvr::BTf> tfs;
     int maxRC = 0;
     bool usePriv = false;
-    double sampleDensity = 0;  // samples per voxel of a view, averaged over the samples of the volume gradients
+    double rayDensity = 0;  // rays per voxel face of a view, averaged over the samples of the volume gradients
     double maxSamples = 0;  // upper bound of samples per ray over the views
     // layout
     int K = 16, waveWidth = 8, gridReq = 0, grid = 0, nTiles = 0, cap = 1;
@@ -105,13 +105,14 @@ struct dvr_batch_plan {
     int nSegsAll = 0;
     long long maxSegAll = 0;
     int nSegsAlways = 1;                // cleared by every run: queues and bricked scratch
-    long long maxSegAlways = kMaxGroups * dvr::kNumXcd;
+    long long maxSegAlways = 0;
     float* dBricks = nullptr;           // bricked volume-gradient scratch of every gradient volume
     size_t brickFloats = 0;
     dvr::DebrickSeg* dDebrick = nullptr;
     int nDebrick = 0;
     long long maxBricks = 0;
-    double* dSums = nullptr;            // sums of a run: loss, TF gradients (added into the caller's after it)
+    // behind the queue counters: sums of a run (loss, TF gradients), added into the caller's after it
+    double* dSums = nullptr;
     dvr::SumSeg* dSumSegs = nullptr;
     int nSums = 0, maxSum = 0;
     float* dCk = nullptr;
@@ -129,7 +130,7 @@ struct dvr_batch_plan {
     ~dvr_batch_plan()
     {
         dev_free(dViews); dev_free(dVols); dev_free(dTfs); dev_free(dQueues); dev_free(dSegsAll); dev_free(dCk);
-        dev_free(dDs); dev_free(dAs); dev_free(dBricks); dev_free(dDebrick); dev_free(dSums); dev_free(dSumSegs);
+        dev_free(dDs); dev_free(dAs); dev_free(dBricks); dev_free(dDebrick);
     }
 
     // doubles between the TF-gradient table copies; 0 (one table) when the copies would take more than
@@ -202,11 +203,12 @@ struct dvr_batch_plan {
                           "occupancy query");
                 if (occ >= target) break;
             }
-            // Two passes up to kMaxSampleDensity samples a voxel and view: the samples of rays close
-            // together meet in the one-pass walk's registers and small table, those of rays far apart
-            // only in the scatter kernel's.  Measured (one pass / two passes): 0.4 samples a voxel 11.4 /
-            // 5.2 ms, 1.7 12.2 / 5.9, 6.9 5.9 / 4.0, 14 4.9 / 4.4, 28 5.7 / 11.0 (256^3; 2.0 / 1.9 at 128^3).
-            if (sampleDensity <= kMaxSampleDensity && reserve_adjoints()) {
+            // Two passes up to kMaxRayDensity rays a voxel face: the samples of rays close together meet in
+            // the one-pass walk's registers and small table, those of rays far apart only in the scatter
+            // kernel's.  Measured (one pass / two passes, ms): 0.25 rays 11.4 / 5.2, 1 ray 12.2 / 5.9, 4 rays
+            // 5.9 / 4.0 (256^3) and 4.8 / 4.3 (128^3, quarter-voxel steps), 7 rays on average over 284 views
+            // of 16 volumes 83.5 / 112, 16 rays 5.7 / 11.0 (256^3) and 1.9 / 1.9 (128^3).
+            if (rayDensity <= kMaxRayDensity && reserve_adjoints()) {
                 lds = sizeof(float) * (size_t(tf_lds()) + ldsG);
                 check_hip(dvr::launch_batched(params(), filter, tfm, blend, segK(), gmRun(), 0, lds, nullptr, &occ),
                           "occupancy query");
@@ -517,7 +519,7 @@ dvr_batch_plan* create(const dvr_batch* b, const dvr_batch_options* o)
         if (vol.adj) {  // about half the longest ray on average
             const double samples = 0.5 * rayMax * v.width * v.height;
             volSamples += samples;
-            volDensity += samples * samples / (double(vol.X) * vol.Y * vol.Z);
+            volDensity += samples * v.width * v.height / std::pow(double(vol.X) * vol.Y * vol.Z, 2.0 / 3.0);
         }
         vs.push_back(d);
     }
@@ -531,7 +533,7 @@ dvr_batch_plan* create(const dvr_batch* b, const dvr_batch_options* o)
         return a.tf != c.tf ? a.tf < c.tf : a.vol < c.vol;
     });
     p->views = vs;
-    p->sampleDensity = volSamples > 0 ? volDensity / volSamples : 0.0;
+    p->rayDensity = volSamples > 0 ? volDensity / volSamples : 0.0;
     if (b->forward_only) p->gm = 0;
     else {
         if (!anyTfGrad && !anyVolGrad && !anyCamGrad && !p->lossOut)
@@ -545,8 +547,36 @@ dvr_batch_plan* create(const dvr_batch* b, const dvr_batch_options* o)
     DeviceGuard guard(b->device);
     // clear list: queue counters first, then every gradient buffer and the loss
     std::vector<dvr::ZeroSeg> segs;
-    p->dQueues = dev_alloc<unsigned>(kMaxGroups * dvr::kNumXcd);
-    segs.push_back({reinterpret_cast<float*>(p->dQueues), kMaxGroups * dvr::kNumXcd});
+    // one allocation: queue counters, the sums of a run in doubles (the loss, then every TF gradient) and
+    // where they are added
+    std::vector<dvr::SumSeg> sums;
+    std::vector<size_t> sumOff;
+    size_t nSum = 0;
+    auto add_sum = [&](float* dst, int n) {
+        sums.push_back({nullptr, dst, n, 0});
+        sumOff.push_back(nSum);
+        nSum += size_t(n);
+        p->maxSum = std::max(p->maxSum, n);
+    };
+    if (p->gm) {
+        if (p->lossOut) add_sum(p->lossOut, 1);
+        for (auto& t : p->tfs)
+            if (t.adj) add_sum(t.adj, t.R * t.C);
+    }
+    constexpr size_t kQueues = size_t(kMaxGroups) * dvr::kNumXcd;
+    p->dQueues = reinterpret_cast<unsigned*>(
+        dev_alloc<char>(kQueues * sizeof(unsigned) + nSum * sizeof(double) + sums.size() * sizeof(dvr::SumSeg)));
+    p->dSums = reinterpret_cast<double*>(p->dQueues + kQueues);
+    p->dSumSegs = reinterpret_cast<dvr::SumSeg*>(p->dSums + nSum);
+    p->nSums = (int)sums.size();
+    for (size_t k = 0; k < sums.size(); ++k) sums[k].sum = p->dSums + sumOff[k];
+    size_t at = p->lossOut ? 1 : 0;
+    for (auto& t : p->tfs)
+        if (p->gm && t.adj) t.sum = p->dSums + sumOff[at++];
+    if (!sums.empty())
+        check_hip(hipMemcpy(p->dSumSegs, sums.data(), sums.size() * sizeof(dvr::SumSeg), hipMemcpyHostToDevice), "hipMemcpy");
+    p->maxSegAlways = (long long)(kQueues + 2 * nSum);
+    segs.push_back({reinterpret_cast<float*>(p->dQueues), p->maxSegAlways});
     // bricked volume-gradient scratch (2 x 2 x 4 voxels per 64-byte chunk), one range per gradient
     // volume, each 256-byte aligned; cleared by every run, added into the gradient after the kernel
     if (p->gm & 2) {
@@ -575,33 +605,6 @@ dvr_batch_plan* create(const dvr_batch* b, const dvr_batch_options* o)
             p->nDebrick = (int)db.size();
             p->dDebrick = dev_alloc<dvr::DebrickSeg>(db.size());
             check_hip(hipMemcpy(p->dDebrick, db.data(), db.size() * sizeof(dvr::DebrickSeg), hipMemcpyHostToDevice),
-                      "hipMemcpy");
-        }
-    }
-    // sums in doubles: the loss first, then every TF gradient
-    if (p->gm) {
-        size_t n = 1;
-        std::vector<size_t> off;
-        for (auto& t : p->tfs) {
-            off.push_back(n);
-            if (t.adj) n += size_t(t.R) * t.C;
-        }
-        p->dSums = dev_alloc<double>(n);
-        segs.push_back({reinterpret_cast<float*>(p->dSums), (long long)n * 2});
-        p->maxSegAlways = std::max(p->maxSegAlways, (long long)n * 2);
-        std::vector<dvr::SumSeg> sums;
-        if (p->lossOut) sums.push_back({p->dSums, p->lossOut, 1, 0});
-        for (size_t k = 0; k < p->tfs.size(); ++k) {
-            dvr::BTf& t = p->tfs[k];
-            if (!t.adj) continue;
-            t.sum = p->dSums + off[k];
-            sums.push_back({t.sum, t.adj, t.R * t.C, 0});
-        }
-        for (auto& q : sums) p->maxSum = std::max(p->maxSum, q.n);
-        p->nSums = (int)sums.size();
-        if (p->nSums > 0) {
-            p->dSumSegs = dev_alloc<dvr::SumSeg>(sums.size());
-            check_hip(hipMemcpy(p->dSumSegs, sums.data(), sums.size() * sizeof(dvr::SumSeg), hipMemcpyHostToDevice),
                       "hipMemcpy");
         }
     }
