@@ -87,6 +87,7 @@ struct dvr_batch_plan {
     std::vector<dvr::BTf> tfs;
     int maxRC = 0;
     bool usePriv = false;
+    bool farRays = false;   // most samples: at most 1.5 rays per voxel face of a volume of at least 8 M voxels
     double rayDensity = 0;  // rays per voxel face of a view, averaged over the samples of the volume gradients
     double maxSamples = 0;  // upper bound of samples per ray over the views
     // layout
@@ -221,12 +222,16 @@ struct dvr_batch_plan {
         check_hip(hipGetDeviceProperties(&prop, device), "hipGetDeviceProperties");
         cus = prop.multiProcessorCount;
         resident = std::max(1, occ) * cus;
-        // default: two waves per SIMD (eight one-wave workgroups per CU; measured
-        // best for gather-bound tiles on MI355X: fewer concurrent rays per CU keep
-        // their cells in L1), within residency; volume-gradient instances are bound
-        // by the latency of their walk and fill the CU (four waves per SIMD) unless they leave the
-        // corner gradients to k_scatter_volume
-        int g = gridReq > 0 ? gridReq : (((gm & 2) && volGrad && !twoPass()) ? resident : std::min(resident, 8 * cus));
+        // default, within residency: two waves per SIMD (eight one-wave workgroups per CU): gather-bound
+        // tiles keep their cells in L1 with few rays in flight.  One-pass volume-gradient instances are
+        // bound by the latency of their walk and fill the CU (four waves per SIMD).  Five workgroups where
+        // most samples are of far rays through volumes larger than the L2s together (256^3, one ray a voxel
+        // face, us with 8 / 5: texture 1700 / 1350, linear 1885 / 1575, volume gradients 8140 / 7290; 192^3
+        // 1147 / 1185; four rays a face 3712 / 3826).  Twelve for Gaussian TFs, which are bound by VALU
+        // issue (8 / 12: cameras 2664 / 2052, TF 2259 / 1878; with the second pass of volume gradients
+        // 2976 / 3156).
+        const int perCu = gm && tfm == 3 && !twoPass() ? 12 : (gm && tfm != 3 && farRays ? 5 : 8);
+        int g = gridReq > 0 ? gridReq : (((gm & 2) && volGrad && !twoPass()) ? resident : std::min(resident, perCu * cus));
         g = std::max(1, std::min(g, std::max(nTiles, 1)));
         grid = g;
         cap = std::max(1, std::min((int)std::ceil(maxSamples / K), 1 << 14));
@@ -477,7 +482,7 @@ dvr_batch_plan* create(const dvr_batch* b, const dvr_batch_options* o)
         p->tfs.push_back(d);
     }
     long long totalPix = 0;
-    double volSamples = 0, volDensity = 0;
+    double volSamples = 0, volDensity = 0, allSamples = 0, farSamples = 0;
     std::vector<dvr::BView> vs;
     for (int i = 0; i < b->num_views; ++i) {
         const dvr_batch_view& v = b->views[i];
@@ -516,10 +521,13 @@ dvr_batch_plan* create(const dvr_batch* b, const dvr_batch_options* o)
                                       double(vol.bsize[2]) * vol.bsize[2]);
         const double rayMax = diag / double(v.step_size) + 2.0;
         p->maxSamples = std::max(p->maxSamples, rayMax);
-        if (vol.adj) {  // about half the longest ray on average
-            const double samples = 0.5 * rayMax * v.width * v.height;
+        const double samples = 0.5 * rayMax * v.width * v.height;  // about half the longest ray on average
+        const double voxels = double(vol.X) * vol.Y * vol.Z, density = v.width * double(v.height) / std::pow(voxels, 2.0 / 3.0);
+        allSamples += samples;
+        if (density <= 1.5 && voxels >= double(8 << 20)) farSamples += samples;
+        if (vol.adj) {
             volSamples += samples;
-            volDensity += samples * v.width * v.height / std::pow(double(vol.X) * vol.Y * vol.Z, 2.0 / 3.0);
+            volDensity += samples * density;
         }
         vs.push_back(d);
     }
@@ -533,6 +541,7 @@ dvr_batch_plan* create(const dvr_batch* b, const dvr_batch_options* o)
         return a.tf != c.tf ? a.tf < c.tf : a.vol < c.vol;
     });
     p->views = vs;
+    p->farRays = farSamples > 0.5 * allSamples;
     p->rayDensity = volSamples > 0 ? volDensity / volSamples : 0.0;
     if (b->forward_only) p->gm = 0;
     else {
