@@ -21,27 +21,30 @@ static float pixel_voxels(const RenderParams& P)
     return float(P.X + P.Y + P.Z) / (3.0f * float(P.W < P.H ? P.W : P.H));
 }
 
-// Few rays leave the tiled kernel's chain of samples exposed: up to 2048 tiles the row kernel wins
-// at every size measured (1024 tiles: 45 against 102 us through 64^3, 122 / 275 through 256^3; 2048
-// tiles 75 / 125 and 214 / 693).  Beyond, it pays by what the gathers touch: with g = (voxels per
-// pixel) x (voxels per step), 64 neighbouring rays reach further apart than 16 consecutive samples
-// where g is large, and more so where the volume exceeds the 4 MiB L2s; short steps leave more
-// samples to overlap.  Measured, row against tiled, in us: g = 0.5, 256^3, 8192 tiles 507 / 1387,
-// 16384 tiles 988 / 2149, 128^3 534 / 640; g = 0.375, 192^3, 691 / 943; g = 0.31, 160^3, 594 / 609;
-// g = 0.25, 256^3, 16384 tiles 892 / 922, 32768 tiles 1742 / 1617, 128^3, 8192 tiles 257 / 243;
-// g = 0.125, 4096 tiles 203 / 221, 8192 tiles 384 / 359; g = 0.06, 4096 tiles 136 / 120; quarter-voxel
-// steps, 8192 tiles 391 / 475, 343 / 350, 16384 tiles 745 / 776, 2385 / 2389.  A nearest-neighbour
-// sample gathers one voxel, not eight, and gains up to 768 tiles.
+// Few rays leave the tiled kernel's chain of samples exposed: up to 768 tiles the row kernel wins at
+// every size measured, up to 1024 and 2048 but for small volumes seen closely (row against tiled, us:
+// 1024 tiles 43 / 67 through 64^3, 122 / 275 through 256^3; 2048 tiles 114 / 191 through 128^3, 54 /
+// 46 through 32^3).  Beyond, it pays by what the gathers touch: 64 neighbouring rays reach further
+// apart than 16 consecutive samples where g = (voxels per pixel) x (voxels per step) is large, and
+// more so where the volume exceeds the 4 MiB L2s.  Below 0.3 voxels per pixel the tiled kernel's
+// twenty workgroups a CU win: 4096 tiles 200 / 189, 8192 tiles 598 / 538.  Others: g = 0.5, 256^3, 8192
+// tiles 507 / 1387, 16384 tiles 988 / 2149; g = 0.375, 192^3, 362 / 665, 96^3, 16384 tiles 451 / 430;
+// g = 0.25, 256^3, 8192 tiles 728 / 878, 16384 tiles 890 / 920, 32768 tiles 1742 / 1617, 128^3, 4096
+// tiles 151 / 186, 16384 tiles 514 / 480; quarter-voxel steps, 0.5 voxels per pixel, 128^3, 8192 tiles
+// 388 / 451, 16384 tiles 774 / 691, 256^3, 16384 tiles 1450 / 1494.  A nearest-neighbour sample gathers
+// one voxel, not eight, and gains up to 768 tiles.
 bool use_row_forward(const RenderParams& P, int filter)
 {
     const int tiles = tiled_num_tiles(P);
     if (tiles <= 768) return true;
     if (filter != 1 || tiles > kMaxRowTiles) return false;
-    const float step = step_voxels(P), g = step * pixel_voxels(P);
-    if (tiles <= 2048 || g >= 0.3f) return true;
-    if (step < 0.4f) return tiles <= 16384;
-    if (g >= 0.24f && size_t(P.X) * P.Y * P.Z >= (size_t(4) << 20)) return tiles <= 16384;
-    return tiles <= (g >= 0.1f ? 4096 : 2048);
+    const float step = step_voxels(P), pixel = pixel_voxels(P), g = step * pixel;
+    const size_t voxels = size_t(P.X) * P.Y * P.Z;
+    if (g >= 0.3f) return tiles <= 8192 || voxels >= (size_t(2) << 20);
+    if (pixel <= 0.3f) return tiles <= (pixel <= 0.15f ? 1024 : 2048);
+    const bool large = voxels >= 4000000;
+    if (step < 0.4f) return tiles <= (large ? 16384 : 8192);
+    return tiles <= (large && g >= 0.24f ? 16384 : 4096);
 }
 
 // Position gradients alone (row_reverse): 220 against 636 us at 2048 tiles, 486 / 786 at 8192, 947 /

@@ -28,13 +28,25 @@ int tiled_num_tiles(const RenderParams& P)
     return tx * ty * P.B;
 }
 
+// One-wave workgroups a CU of the forward march: more hide more of a sample's latency, fewer keep the
+// rays' cells in L1.  Twelve, and twenty where at most 0.3 voxels lie between pixels (the rays of a tile
+// share cells).  us with 8 / 12 / 16 / 20: 2 x 1024 x 768 rays of 256^3 1200 / 1067 / 1095 / -; 1024 x 1024
+// of 256^3 (0.25 voxels) 1074 / 936 / 804 / 777; 2 x 1024 x 1024 with quarter-voxel steps 5393 / - / 3420 /
+// 3188; 8 x 512 x 512 (0.5) 1442 / 1454 / 1601; 4 x 512 x 512 of 192^3 (0.38) 572 / 522 / 553.
+static int forward_wg_per_cu(const RenderParams& P, int tfm)
+{
+    if (tfm == 3) return 0;
+    const float voxels = float(P.X + P.Y + P.Z) / (3.0f * float(P.W < P.H ? P.W : P.H));
+    return voxels <= 0.3f ? 20 : 12;
+}
+
 template <int FILTER, int TFM, int BLEND>
 static hipError_t fwd_tiled_t(const RenderParams& P, const CkptParams& CK, hipStream_t s)
 {
     const int tilesX = (P.W + kTileW - 1) / kTileW, tilesY = (P.H + kTileH - 1) / kTileH;
     const int nTiles = tilesX * tilesY * P.B;
     if (nTiles == 0) return hipSuccess;
-    const size_t lds = occupancy_lds(sizeof(float) * size_t(P.R) * tf_lds_stride<TFM>(), tiled_wg_per_cu(TFM));
+    const size_t lds = occupancy_lds(sizeof(float) * size_t(P.R) * tf_lds_stride<TFM>(), forward_wg_per_cu(P, TFM));
     hipLaunchKernelGGL((k_forward_tiled<FILTER, TFM, BLEND>), dim3(nTiles), dim3(kBlock), lds, s, P, CK, tilesX,
                        tilesX * tilesY, nTiles);
     return hipGetLastError();
