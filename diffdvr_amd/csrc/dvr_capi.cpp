@@ -643,7 +643,7 @@ public:
             check_hip(dvr::launch_debrick_call(D, volumes_, A.avSb, s), "debrick launch");
         }
         if (sums_ > 0)
-            check_hip(dvr::launch_add_tf_sums(A.atfSum, A, c_.B, c_.P.R, c_.P.C, s), "TF gradient launch");
+            check_hip(dvr::launch_add_call_sums(nullptr, A, c_.B, c_.P.R, c_.P.C, s), "TF gradient launch");
     }
 
 private:
@@ -906,7 +906,10 @@ void do_fused(const dvr_inputs* inputs, dvr_outputs* outputs, const dvr_loss* lo
     DeviceGuard g(c.device);
     hipStream_t s = (hipStream_t)stream;
     const int64_t need = (int64_t)dvr::tiled_num_tiles(c.P) * CK.cap * dvr::kBlock;
-    ScratchLease lease(c.device, s);  // the scratch (either kind), until the launch is enqueued
+    ScratchLease lease(c.device, s);  // the scratch (either kind), until the launches are enqueued
+    // the call's sums of the loss lie behind the checkpoints; where the static scratch has no room left the
+    // workgroups add floats to the caller's scalar (the tiled kernel, once a tile)
+    const int64_t sums = L.lossOut ? 2 * dvr::kLossSlots * dvr::kLossStride : 0;
     if (fixed) {
         // checkpoints in the device's static scratch; no density store (the reverse march
         // re-interpolates: the same densities)
@@ -917,13 +920,18 @@ void do_fused(const dvr_inputs* inputs, dvr_outputs* outputs, const dvr_loss* lo
                  "per call)", (long long)need, K, (long long)fixed->floats);
         CK.buf = fixed->get(c.device);
     } else {
-        CK.buf = (float*)workspace(c.device, size_t(need) * sizeof(float), s);
+        CK.buf = (float*)workspace(c.device, size_t(need + sums) * sizeof(float), s);
         if (double(density_elements(c)) * sizeof(float) <= kMaxDensityStore) {
             CK.ds = (float*)workspace(c.device, size_t(density_elements(c)) * sizeof(float), s, 1);
             CK.dsCap = density_cap(c);
         }
     }
+    if (sums > 0 && (!fixed || need + sums <= fixed->floats)) {
+        L.lossSum = reinterpret_cast<double*>(CK.buf + need);
+        check_hip(dvr::launch_clear(CK.buf + need, size_t(sums), s), "clear launch");
+    }
     check_hip(dvr::launch_adjoint_tiled(c.P, A, CK, L, true, false, c.filter, c.tfm, c.blend, s), "fused launch");
+    check_hip(dvr::launch_add_call_sums(&L, A, c.B, c.P.R, c.P.C, s), "loss launch");
 }
 
 // ---------------------------------------------------------------------------

@@ -113,10 +113,16 @@ __global__ __launch_bounds__(256) void k_add_sums(const SumSeg* segs)
     for (int i = blockIdx.x * 256 + threadIdx.x; i < S.n; i += gridDim.x * 256)
         atomicAdd(S.dst + i, float(S.sum[i]));  // tables may share a gradient
 }
-// the TF gradients of one call: batch, row and column strides of its tensor
-__global__ __launch_bounds__(256) void k_add_tf_sums(const double* sum, float* dst, int n, int RC, int C, int sb, int sr,
-                                                     int sc)
+// the loss and the TF gradients of one call: batch, row and column strides of its tensor
+__global__ __launch_bounds__(256) void k_add_call_sums(const double* lossSum, float* lossOut, const double* sum, float* dst,
+                                                       int n, int RC, int C, int sb, int sr, int sc)
 {
+    if (lossSum && blockIdx.x == 0 && threadIdx.x < 64) {
+        double v = threadIdx.x < kLossSlots ? lossSum[threadIdx.x * kLossStride] : 0.0;
+#pragma unroll
+        for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o, 64);
+        if (threadIdx.x == 0) atomicAdd(lossOut, float(v));
+    }
     const int i = blockIdx.x * 256 + threadIdx.x;
     if (i >= n) return;
     const int b = i / RC, e = i - b * RC, r = e / C, c = e - r * C;
@@ -130,12 +136,13 @@ hipError_t launch_add_sums(const SumSeg* dSegs, int nSegs, int maxN, hipStream_t
     return hipGetLastError();
 }
 
-hipError_t launch_add_tf_sums(const double* sum, const AdjointParams& A, int B, int R, int C, hipStream_t s)
+hipError_t launch_add_call_sums(const LossParams* L, const AdjointParams& A, int B, int R, int C, hipStream_t s)
 {
-    const int n = (A.atfSb != 0 ? B : 1) * R * C;
-    if (n == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_add_tf_sums, dim3(unsigned((n + 255) / 256)), dim3(256), 0, s, sum, A.atf, n, R * C, C, A.atfSb,
-                       A.atfSr, A.atfSc);
+    const double* lossSum = L ? L->lossSum : nullptr;
+    const int n = A.atfSum ? (A.atfSb != 0 ? B : 1) * R * C : 0;
+    if (n == 0 && !lossSum) return hipSuccess;
+    hipLaunchKernelGGL(k_add_call_sums, dim3(unsigned(n > 0 ? (n + 255) / 256 : 1)), dim3(256), 0, s, lossSum,
+                       L ? L->lossOut : nullptr, A.atfSum, A.atf, n, R * C, C, A.atfSb, A.atfSr, A.atfSc);
     return hipGetLastError();
 }
 

@@ -65,7 +65,7 @@ hipError_t launch_adjoint_tiled(const RenderParams& P, const AdjointParams& A, c
                                 hipStream_t s)
 {
     if (filter < 0 || filter > 1 || blend < 0 || blend > 1) return hipErrorInvalidValue;
-    if (use_row_adjoint(P, A, CK, tfm))
+    if (use_row_adjoint(P, A, CK, L, tfm))
         return launch_adjoint_row(P, A, CK, L, fused, ckFromFwd, filter, tfm, blend, s);
 #define DVR_CALL(F, B, K) return adj_tiled_inst_##F##_##B##_##K(P, A, CK, L, fused, ckFromFwd, tfm, s)
 #define DVR_SEL_K(F, B)                      \

@@ -64,7 +64,7 @@ hipError_t launch_adjoint_tiled(const RenderParams& P, const AdjointParams& A, c
 
 // dvr_kernels_row.hip: the same, 16 lanes a ray, and the sizes at which they are faster
 bool use_row_forward(const RenderParams& P, int filter);
-bool use_row_adjoint(const RenderParams& P, const AdjointParams& A, const CkptParams& CK, int tfm);
+bool use_row_adjoint(const RenderParams& P, const AdjointParams& A, const CkptParams& CK, const LossParams& L, int tfm);
 hipError_t launch_forward_row(const RenderParams& P, const CkptParams& CK, int filter, int tfm, int blend,
                               hipStream_t s);
 hipError_t launch_adjoint_row(const RenderParams& P, const AdjointParams& A, const CkptParams& CK, const LossParams& L,
@@ -94,9 +94,10 @@ hipError_t launch_debrick(const DebrickSeg* dSegs, int nSegs, long long maxBrick
 hipError_t launch_debrick_call(const DebrickSeg& S, int batches, long long sb, hipStream_t s);
 // dvr_kernels_scatter.hip: the second pass of the volume gradients (P.parts is chosen here)
 hipError_t launch_scatter_volume(const ScatterParams& P, int filter, hipStream_t s, int channels = 1);
-// sums of doubles added into the caller's gradients: a plan's segments, one call's TF gradient
+// sums of doubles added into the caller's gradients and loss: a plan's segments; one call's loss (L may be NULL)
+// and TF gradient
 hipError_t launch_add_sums(const SumSeg* dSegs, int nSegs, int maxN, hipStream_t s);
-hipError_t launch_add_tf_sums(const double* sum, const AdjointParams& A, int B, int R, int C, hipStream_t s);
+hipError_t launch_add_call_sums(const LossParams* L, const AdjointParams& A, int B, int R, int C, hipStream_t s);
 // clears n floats (a multiple of 4, 16-byte aligned) with a kernel
 hipError_t launch_clear(float* p, size_t n, hipStream_t s);
 

@@ -121,11 +121,14 @@ struct CkptParams {
 #define DVR_LOSS_L1 1     // mean |color - target|   (torch.nn.L1Loss)
 #define DVR_LOSS_L2 2     // mean (color - target)^2 (torch.nn.MSELoss)
 
+// Sums of the loss of a call, each on a line of its own: thousands of workgroups add to them.
+constexpr int kLossSlots = 32, kLossStride = 8;
 struct LossParams {
     int kind;
     const float* target; int tgSb, tgSy, tgSx, tgSc;
     float scale;          // 1 / number of loss elements
     float* lossOut;       // optional scalar accumulator (atomic), may be NULL
+    double* lossSum;      // [kLossSlots][kLossStride] sums of the call, added into lossOut after it, or NULL
 };
 
 

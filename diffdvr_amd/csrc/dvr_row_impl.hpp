@@ -494,8 +494,16 @@ __global__ __launch_bounds__(kRowAdjBlock) __attribute__((amdgpu_waves_per_eu(GM
         }
     }
     if (fused && LP.lossOut) {
+        __shared__ double s_loss[kThreads / 64];
         const float v = wave_sum(lossLocal);
-        if ((threadIdx.x & 63) == 0) atomicAdd(LP.lossOut, v);
+        if ((threadIdx.x & 63) == 0) s_loss[threadIdx.x >> 6] = v;
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            double sum = 0.0;
+#pragma unroll
+            for (int k = 0; k < kThreads / 64; ++k) sum += s_loss[k];
+            loss_add(LP, sum);
+        }
     }
     if (wantTf) {
         __syncthreads();

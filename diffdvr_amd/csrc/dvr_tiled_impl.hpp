@@ -218,6 +218,13 @@ __device__ __forceinline__ void tf_grad_add(const RenderParams& P, const Adjoint
     }
 }
 
+// Adds a workgroup's share of the loss: into the call's doubles, or (without them) the caller's scalar.
+__device__ __forceinline__ void loss_add(const LossParams& L, double v)
+{
+    if (L.lossSum) atomicAdd(L.lossSum + (blockIdx.x & unsigned(kLossSlots - 1)) * kLossStride, v);
+    else atomicAdd(L.lossOut, float(v));
+}
+
 // ---------------------------------------------------------------------------
 // Reverse-walk cell state of the volume and position adjoints.  Consecutive
 // cells of a ray that differ by one step along one axis share the 4 corners
@@ -1011,7 +1018,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(GM == 3 
     if (wantTf) sink.template finish<TFM == 2 ? 5 : 4>();
     if (fused && L.lossOut) {
         const float s = wave_sum(lossLocal);
-        if ((threadIdx.x & 63) == 0) atomicAdd(L.lossOut, s);
+        if ((threadIdx.x & 63) == 0) loss_add(L, s);
     }
     if (wantTf) {
         __syncthreads();

@@ -214,7 +214,8 @@ typedef struct dvr_loss {
 } dvr_loss;
 
 /* Forward march, image loss against `target` and checkpointed adjoint in ONE
- * launch per batch: colour and termination index are written to `outputs`,
+ * launch per batch (and two small ones around it for the sums of the loss):
+ * colour and termination index are written to `outputs`,
  * the loss gradient never leaves registers, and the adjoint outputs are
  * accumulated as by dvr_render_adjoint.  checkpoint_interval K in {0,8,16,32,64}
  * (0 = default).  No reference counterpart: it fuses Renderer::renderForward,
