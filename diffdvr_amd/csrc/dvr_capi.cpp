@@ -591,7 +591,13 @@ bool distinct_elements(const Checked& c, const dvr::AdjointParams& A, int volume
     return true;
 }
 
-// Call scratch of the checkpointed adjoint.  TF gradients that thousands of workgroups add to are summed in
+// floats of the double sums of a call's TF gradient, a multiple of 4
+size_t tf_sum_floats(const Checked& c, const dvr::AdjointParams& A)
+{
+    return A.atf ? (size_t(A.atfSb != 0 ? c.B : 1) * c.P.R * c.P.C + 1) / 2 * 4 : 0;
+}
+
+// Call scratch of the checkpointed adjoint.  TF gradients, to which every workgroup adds, are summed in
 // doubles and added into the caller's tensor after the last launch.  Volume gradients take two passes
 // (dvr_kernels_scatter.hip): the walk stores the density adjoints of a group of tiles and their rays,
 // k_scatter_volume adds them into bricked scratch, and after the last group k_debrick adds that into the
@@ -601,29 +607,32 @@ public:
     AdjointScratch(const Checked& c, const dvr::AdjointParams& A) : c_(c), A_(A), tiles_(dvr::tiled_num_tiles(c.P))
     {
         if (c.preshaded || tiles_ == 0) return;
-        if (A.atf && tiles_ >= kSumTiles) sums_ = (size_t(A.atfSb != 0 ? c.B : 1) * c.P.R * c.P.C + 1) / 2 * 4;
+        sums_ = tf_sum_floats(c, A);
         plan_volume();
         bytes_ = sizeof(float) * (sums_ + brickFloats_ * volumes_ + size_t(group_) * perTile_);
     }
     size_t bytes() const { return bytes_; }
+    bool holds_sums(const Scratch& scr) const { return scr.bytes >= sums_ * sizeof(float); }
 
     // Runs the adjoint: launch(A, CK) must launch the tiles CK.tile0 .. tile0 + tileN - 1 (0: all).
+    // sums: memory for the TF sums where the scratch holds none, or NULL.
     template <class Launch>
-    void run(dvr::CkptParams CK, const Scratch& scr, hipStream_t s, Launch launch) const
+    void run(dvr::CkptParams CK, const Scratch& scr, float* sums, hipStream_t s, Launch launch) const
     {
-        if (bytes_ == 0 || scr.bytes < bytes_) return launch(A_, CK);
-        float* base = (float*)scr.data;
-        float* brick = base + sums_;
+        if (holds_sums(scr)) sums = (float*)scr.data;
+        const bool twoPass = group_ > 0 && scr.bytes >= bytes_;
         dvr::AdjointParams A = A_;
-        if (sums_ > 0) A.atfSum = (double*)base;
-        check_hip(dvr::launch_clear(base, sums_ + brickFloats_ * volumes_, s), "clear launch");
-        if (group_ == 0) launch(A, CK);
+        if (sums_ > 0) A.atfSum = (double*)sums;
+        float* brick = (float*)scr.data + sums_;
+        if (twoPass) check_hip(dvr::launch_clear(sums, sums_ + brickFloats_ * volumes_, s), "clear launch");
+        else if (A.atfSum) check_hip(dvr::launch_clear(sums, sums_, s), "clear launch");
+        if (!twoPass) launch(A, CK);
         else {
             CK.as.rays = brick + brickFloats_ * volumes_;
             CK.as.adj = CK.as.rays + size_t(group_) * dvr::kRayRecord * dvr::kBlock;
             CK.as.cap = cap_;
         }
-        for (int t0 = 0; group_ > 0 && t0 < tiles_; t0 += group_) {
+        for (int t0 = 0; twoPass && t0 < tiles_; t0 += group_) {
             CK.tile0 = t0;
             CK.tileN = std::min(group_, tiles_ - t0);
             launch(A, CK);
@@ -638,18 +647,14 @@ public:
             S.X = c_.X; S.Y = c_.Y; S.Z = c_.Z;
             check_hip(dvr::launch_scatter_volume(S, c_.filter, s), "scatter launch");
         }
-        if (group_ > 0) {
+        if (twoPass) {
             const dvr::DebrickSeg D{brick, A.avol, c_.X, c_.Y, c_.Z, 0, A.avSx, A.avSy, A.avSz};
             check_hip(dvr::launch_debrick_call(D, volumes_, A.avSb, s), "debrick launch");
         }
-        if (sums_ > 0)
-            check_hip(dvr::launch_add_call_sums(nullptr, A, c_.B, c_.P.R, c_.P.C, s), "TF gradient launch");
+        check_hip(dvr::launch_add_call_sums(nullptr, A, c_.B, c_.P.R, c_.P.C, s), "TF gradient launch");
     }
 
 private:
-    // sums pay two small launches from as many tiles on
-    static constexpr int kSumTiles = 1024;
-
     void plan_volume()
     {
         // the store holds the longest ray of a uniform box and step; clearing and adding the bricks
@@ -835,6 +840,8 @@ void do_adjoint(const dvr_inputs* inputs, const dvr_outputs* fwd, const dvr_tens
     dvr::CkptParams CK = make_ckpt(c, K);
     const int64_t need = (int64_t)dvr::tiled_num_tiles(c.P) * CK.cap * dvr::kBlock;
     bool fromFwd = false;
+    const AdjointScratch own(c, A);
+    float* sums = nullptr;  // TF sums in the library scratch
     std::optional<ScratchLease> lease;  // the library scratch, until the launch is enqueued
     if (opt && given(opt->checkpoints)) {
         const dvr_tensor& ck = opt->checkpoints;
@@ -855,7 +862,9 @@ void do_adjoint(const dvr_inputs* inputs, const dvr_outputs* fwd, const dvr_tens
         if (opt && given(opt->densities))
             fail(DVR_ERR_INVALID_ARGUMENT, "densities are read together with the checkpoints of the same forward");
         lease.emplace(c.device, s);
-        CK.buf = (float*)workspace(c.device, size_t(need) * sizeof(float), s);
+        const size_t behind = own.holds_sums(scr) ? 0 : tf_sum_floats(c, A);
+        CK.buf = (float*)workspace(c.device, (size_t(need) + behind) * sizeof(float), s);
+        if (behind > 0) sums = CK.buf + need;
         if (double(density_elements(c)) * sizeof(float) <= kMaxDensityStore) {  // the replaying forward writes them
             CK.ds = (float*)workspace(c.device, size_t(density_elements(c)) * sizeof(float), s, 1);
             CK.dsCap = density_cap(c);
@@ -863,7 +872,7 @@ void do_adjoint(const dvr_inputs* inputs, const dvr_outputs* fwd, const dvr_tens
     }
     dvr::LossParams L;
     std::memset(&L, 0, sizeof(L));
-    AdjointScratch(c, A).run(CK, scr, s, [&](const dvr::AdjointParams& a, const dvr::CkptParams& ck) {
+    own.run(CK, scr, sums, s, [&](const dvr::AdjointParams& a, const dvr::CkptParams& ck) {
         check_hip(dvr::launch_adjoint_tiled(c.P, a, ck, L, false, fromFwd, c.filter, c.tfm, c.blend, s),
                   "adjoint (tiled) launch");
     });
@@ -907,9 +916,10 @@ void do_fused(const dvr_inputs* inputs, dvr_outputs* outputs, const dvr_loss* lo
     hipStream_t s = (hipStream_t)stream;
     const int64_t need = (int64_t)dvr::tiled_num_tiles(c.P) * CK.cap * dvr::kBlock;
     ScratchLease lease(c.device, s);  // the scratch (either kind), until the launches are enqueued
-    // the call's sums of the loss lie behind the checkpoints; where the static scratch has no room left the
-    // workgroups add floats to the caller's scalar (the tiled kernel, once a tile)
-    const int64_t sums = L.lossOut ? 2 * dvr::kLossSlots * dvr::kLossStride : 0;
+    // the call's sums of the loss and the TF gradient lie behind the checkpoints; where the static scratch has
+    // no room left the workgroups add floats to the caller's (the tiled kernel, once a tile)
+    const int64_t lossFloats = L.lossOut ? 2 * dvr::kLossSlots * dvr::kLossStride : 0;
+    const int64_t sums = lossFloats + (int64_t)tf_sum_floats(c, A);
     if (fixed) {
         // checkpoints in the device's static scratch; no density store (the reverse march
         // re-interpolates: the same densities)
@@ -927,7 +937,8 @@ void do_fused(const dvr_inputs* inputs, dvr_outputs* outputs, const dvr_loss* lo
         }
     }
     if (sums > 0 && (!fixed || need + sums <= fixed->floats)) {
-        L.lossSum = reinterpret_cast<double*>(CK.buf + need);
+        if (L.lossOut) L.lossSum = reinterpret_cast<double*>(CK.buf + need);
+        if (A.atf) A.atfSum = reinterpret_cast<double*>(CK.buf + need + lossFloats);
         check_hip(dvr::launch_clear(CK.buf + need, size_t(sums), s), "clear launch");
     }
     check_hip(dvr::launch_adjoint_tiled(c.P, A, CK, L, true, false, c.filter, c.tfm, c.blend, s), "fused launch");

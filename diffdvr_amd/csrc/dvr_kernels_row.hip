@@ -52,12 +52,13 @@ bool use_row_forward(const RenderParams& P, int filter)
 // gradients (split_reverse) in two passes: 185 / 262 and 273 / 277 us at 1024 tiles, 415 / 350 at
 // 2048; in one pass 634 / 1038 at 2048, 2707 / 2684 at 4096.  TF gradients: 137 / 160 us at 1024
 // tiles, 238 / 184 at 2048; the identity TF's walk is short, 53 / 65 at 576 and 83 / 67 at 1024.
-// A loss is summed in doubles: the row kernel adds four times a tile, and 4096 or more floats added to one
-// scalar in any order are off by 1e-6 of it and more.
+// The loss and TF gradients are summed in doubles: the row kernel adds four times a tile, and 4096 or more
+// floats added to one scalar in any order are off by 1e-6 of it and more.  Without memory for these sums the
+// tiled kernel runs.
 bool use_row_adjoint(const RenderParams& P, const AdjointParams& A, const CkptParams& CK, const LossParams& L, int tfm)
 {
     const int tiles = tiled_num_tiles(P);
-    if (tiles > kMaxRowTiles || (L.lossOut && !L.lossSum)) return false;
+    if (tiles > kMaxRowTiles || (L.lossOut && !L.lossSum) || (A.atf && !A.atfSum)) return false;
     if (A.avol) return tiles <= (CK.as.adj ? 1024 : 2048);
     if (A.atf) return tiles <= (tfm == 0 && !A.ars && !A.ast ? 768 : 1024);
     return tiles <= 16384 || step_voxels(P) < 0.4f;

@@ -206,7 +206,7 @@ __device__ __forceinline__ double tf_grad_sum(const float* s_g, int e, int copyS
 }
 // Adds a workgroup's sum of entry e of batch b: into the call's doubles, or (without call scratch) the
 // gradient.  Thousands of workgroups add to one entry: the order of float additions there gave errors of
-// 2e-6 of the gradient.
+// 2e-6 of the gradient (the row kernels, which add four times as often, run with the call's doubles only).
 __device__ __forceinline__ void tf_grad_add(const RenderParams& P, const AdjointParams& A, int b, int e, double v)
 {
     if (v == 0.0) return;

@@ -588,9 +588,8 @@ PYBIND11_MODULE(_pyrenderer, m)
               opt.checkpoint_interval = checkpoint_interval;
               opt.checkpoints = to_tensor(checkpoints);
               opt.densities = to_tensor(densities);
-              // without volume gradients only large images use scratch: small calls skip the question
-              const int64_t rays = o.color.ndim == 4 ? o.color.sizes[0] * o.color.sizes[1] * o.color.sizes[2] : 0;
-              const bool ask = ao.has_volume_derivatives || rays >= 65536 ||
+              // camera and step gradients alone use no scratch
+              const bool ask = ao.has_volume_derivatives || ao.has_tf_derivatives ||
                                p.in.volume_filter_mode == DVR_FILTER_PRESHADED;
               const CallScratch scr(ask ? dvr_adjoint_scratch_bytes(&p.in, &o, &ac, &ao, &opt) : 0, inputs.volume);
               check(dvr_render_adjoint_scratch(&p.in, &o, &ac, &ao, &opt, scr.data, scr.bytes,
