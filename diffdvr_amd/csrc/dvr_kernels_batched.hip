@@ -37,35 +37,28 @@ hipError_t launch_batched(const BatchParams& P, int filter, int tfm, int blend, 
 }
 
 // Adds a volume's bricked gradient scratch (2 x 2 x 4 voxels per 64-byte chunk,
-// bricks z-fastest) into the caller's X x Y x Z gradient: a thread per brick,
-// consecutive threads on consecutive z bricks of one (x, y) brick column, so
-// reads and, with z innermost, the four 16-byte row segments it updates are
-// contiguous across the wave.
+// bricks z-fastest) into the caller's X x Y x Z gradient: a thread per 2 x 2
+// column of voxels, consecutive threads on consecutive z, so that a wave reads
+// whole chunks and, with z innermost, adds to four contiguous rows.  Other
+// streams may add to the same gradient at the same time (calls with their own
+// scratch and plans are not ordered with each other): device atomics, of the
+// voxels that have a gradient (256^3, every voxel touched: 8 us more than a read-modify-write in a
+// call of 2.4 ms).
 __device__ __forceinline__ void debrick(const DebrickSeg& S)
 {
-    const int BY = (S.Y + 1) >> 1, BZ = (S.Z + 3) >> 2;
-    const long long nb = (long long)((S.X + 1) >> 1) * BY * BZ;
-    const bool vec = S.sz == 1 && (S.Z & 3) == 0 && (S.sx & 3) == 0 && (S.sy & 3) == 0 &&
-                     (reinterpret_cast<uintptr_t>(S.adj) & 15u) == 0;
-    for (long long b = (long long)blockIdx.x * 256 + threadIdx.x; b < nb; b += (long long)gridDim.x * 256) {
-        const int zb = int(b % BZ);
-        const long long r = b / BZ;
-        const int yb = int(r % BY), xb = int(r / BY);
-        const float4* src = reinterpret_cast<const float4*>(S.brick) + b * 4;
+    // a volume of at most 2^30 voxels has fewer than 2^31 columns
+    const unsigned Z = unsigned(S.Z), BY = unsigned(S.Y + 1) >> 1, BZ = (Z + 3) >> 2;
+    const unsigned n = (unsigned(S.X + 1) >> 1) * BY * Z;
+    for (unsigned i = blockIdx.x * 256u + threadIdx.x; i < n; i += gridDim.x * 256u) {
+        const unsigned r = i / Z, z = i - r * Z, xb = r / BY, yb = r - xb * BY;
+        const float* src = S.brick + size_t(r * BZ + (z >> 2)) * 16 + (z & 3);
+        float v[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) v[q] = src[4 * q];
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-            const int x = 2 * xb + (q >> 1), y = 2 * yb + (q & 1);
-            if (x >= S.X || y >= S.Y) continue;
-            const float4 v = src[q];
-            float* g = S.adj + x * S.sx + y * S.sy + 4 * zb * S.sz;
-            if (vec) {
-                float4 o = *reinterpret_cast<float4*>(g);
-                o.x += v.x; o.y += v.y; o.z += v.z; o.w += v.w;
-                *reinterpret_cast<float4*>(g) = o;
-            } else {
-                const float vv[4] = {v.x, v.y, v.z, v.w};
-                for (int k = 0; k < 4 && 4 * zb + k < S.Z; ++k) g[k * S.sz] += vv[k];
-            }
+            const int x = int(2 * xb) + (q >> 1), y = int(2 * yb) + (q & 1);
+            if (v[q] != 0.0f && x < S.X && y < S.Y) atomicAdd(S.adj + x * S.sx + y * S.sy + int(z) * S.sz, v[q]);
         }
     }
 }
@@ -101,7 +94,7 @@ hipError_t launch_clear(float* p, size_t n, hipStream_t s)
 hipError_t launch_debrick_call(const DebrickSeg& S, int batches, long long sb, hipStream_t s)
 {
     const long long bf = (long long)brick_floats(S.X, S.Y, S.Z);
-    const long long bx = (bf / 16 + 255) / 256;
+    const long long bx = (bf / 4 + 255) / 256;
     hipLaunchKernelGGL(k_debrick_call, dim3(unsigned(bx < 8192 ? bx : 8192), unsigned(batches)), dim3(256), 0, s, S, bf, sb);
     return hipGetLastError();
 }
@@ -149,8 +142,8 @@ hipError_t launch_add_call_sums(const LossParams* L, const AdjointParams& A, int
 hipError_t launch_debrick(const DebrickSeg* dSegs, int nSegs, long long maxBricks, hipStream_t s)
 {
     if (nSegs <= 0) return hipSuccess;
-    long long bx = (maxBricks + 255) / 256;
-    if (bx > 2048) bx = 2048;
+    long long bx = (4 * maxBricks + 255) / 256;
+    if (bx > 8192) bx = 8192;
     if (bx < 1) bx = 1;
     hipLaunchKernelGGL(k_debrick, dim3(unsigned(bx), unsigned(nSegs)), dim3(256), 0, s, dSegs);
     return hipGetLastError();
