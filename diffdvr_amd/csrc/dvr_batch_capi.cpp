@@ -57,8 +57,9 @@ int wave_shift_of(int ww)
     }
 }
 
-// Volume gradients in two passes: bytes of density adjoints a plan may hold at a time (C5's tiles of
-// 900-sample rays then run in groups of 37 000), and groups a run may be cut into.
+// Volume gradients in two passes: bytes of density adjoints a plan may hold at a time (tiles of 900-sample
+// rays then run in groups of 35 000), and groups a run may be cut into.  Each group drains the chip: 24
+// views of 256^3 with 8 / 4 / 2 / 1 GiB 7.4 / 8.3 / 9.0 / 12.1 ms.
 constexpr long long kMaxAdjointStore = 8LL << 30;
 constexpr int kMaxGroups = 64;
 constexpr double kMaxRayDensity = 5.5;
@@ -145,7 +146,7 @@ struct dvr_batch_plan {
     int segK() const { return K > 32 ? 32 : K; }
 
     bool twoPass() const { return groupTiles > 0; }
-    int gmRun() const { return twoPass() ? (gm & 4 ? 13 : 9) : gm; }
+    int gm_run(bool two) const { return two ? (gm & 4 ? 13 : 9) : gm; }
     int groups() const { return twoPass() ? (nTiles + groupTiles - 1) / groupTiles : 1; }
 
     dvr::BatchParams params(int group = 0) const
@@ -185,6 +186,28 @@ struct dvr_batch_plan {
         }
         if (t >= (1LL << 31)) fail(DVR_ERR_INVALID_ARGUMENT, "batch has too many tiles");
         nTiles = (int)t;
+        hipDeviceProp_t prop;
+        check_hip(hipGetDeviceProperties(&prop, device), "hipGetDeviceProperties");
+        cus = prop.multiProcessorCount;
+        // Two passes up to kMaxRayDensity rays a voxel face: the samples of rays close together meet in
+        // the one-pass walk's registers and small table, those of rays far apart only in the scatter
+        // kernel's.  Measured (one pass / two passes, ms): 0.25 rays 11.4 / 5.2, 1 ray 12.2 / 5.9, 4 rays
+        // 5.9 / 4.0 (256^3) and 4.8 / 4.3 (128^3, quarter-voxel steps), 7 rays on average over 284 views
+        // of 16 volumes 83.5 / 112, 16 rays 5.7 / 11.0 (256^3) and 1.9 / 1.9 (128^3).  Small plans alike:
+        // 0.17 / 0.08 (four tiles, 14^3), 0.80 / 0.28 (1024 tiles, 32^3).
+        const bool two = (gm & 2) && volGrad && rayDensity <= kMaxRayDensity;
+        if (!(two && layout_scratch(true))) {
+            release_adjoints();
+            layout_scratch(false);
+        }
+        check_hip(hipMemcpy(dViews, views.data(), views.size() * sizeof(dvr::BView), hipMemcpyHostToDevice),
+                  "hipMemcpy views");
+    }
+
+    // LDS, grid and scratch of one scheme of the volume gradients.  The checkpoints and densities are
+    // allocated first; two passes: false where these or the adjoint store find no memory.
+    bool layout_scratch(bool two)
+    {
         const size_t ldsG = gm ? size_t(dvr::tf_grad_floats(maxRC, usePriv, dvr::kBatchBlock, copy_stride())) : 0;
         lds = sizeof(float) * (size_t(tf_lds()) + ldsG);
         // volume gradients: the per-wave table of 64-byte chunks follows the TF tables (not
@@ -204,23 +227,12 @@ struct dvr_batch_plan {
                           "occupancy query");
                 if (occ >= target) break;
             }
-            // Two passes up to kMaxRayDensity rays a voxel face: the samples of rays close together meet in
-            // the one-pass walk's registers and small table, those of rays far apart only in the scatter
-            // kernel's.  Measured (one pass / two passes, ms): 0.25 rays 11.4 / 5.2, 1 ray 12.2 / 5.9, 4 rays
-            // 5.9 / 4.0 (256^3) and 4.8 / 4.3 (128^3, quarter-voxel steps), 7 rays on average over 284 views
-            // of 16 volumes 83.5 / 112, 16 rays 5.7 / 11.0 (256^3) and 1.9 / 1.9 (128^3).
-            if (rayDensity <= kMaxRayDensity && reserve_adjoints()) {
-                lds = sizeof(float) * (size_t(tf_lds()) + ldsG);
-                check_hip(dvr::launch_batched(params(), filter, tfm, blend, segK(), gmRun(), 0, lds, nullptr, &occ),
-                          "occupancy query");
-            }
-        } else {
-            check_hip(dvr::launch_batched(params(), filter, tfm, blend, segK(), gm, 0, lds, nullptr, &occ),
+        }
+        if (two || occ == 0) {
+            if (two) lds = sizeof(float) * (size_t(tf_lds()) + ldsG);
+            check_hip(dvr::launch_batched(params(), filter, tfm, blend, segK(), gm_run(two), 0, lds, nullptr, &occ),
                       "occupancy query");
         }
-        hipDeviceProp_t prop;
-        check_hip(hipGetDeviceProperties(&prop, device), "hipGetDeviceProperties");
-        cus = prop.multiProcessorCount;
         resident = std::max(1, occ) * cus;
         // default, within residency: two waves per SIMD (eight one-wave workgroups per CU): gather-bound
         // tiles keep their cells in L1 with few rays in flight.  One-pass volume-gradient instances are
@@ -230,19 +242,11 @@ struct dvr_batch_plan {
         // 1147 / 1185; four rays a face 3712 / 3826).  Twelve for Gaussian TFs, which are bound by VALU
         // issue (8 / 12: cameras 2664 / 2052, TF 2259 / 1878; with the second pass of volume gradients
         // 2976 / 3156).
-        const int perCu = gm && tfm == 3 && !twoPass() ? 12 : (gm && tfm != 3 && farRays ? 5 : 8);
-        int g = gridReq > 0 ? gridReq : (((gm & 2) && volGrad && !twoPass()) ? resident : std::min(resident, perCu * cus));
+        const int perCu = gm && tfm == 3 && !two ? 12 : (gm && tfm != 3 && farRays ? 5 : 8);
+        int g = gridReq > 0 ? gridReq : (((gm & 2) && volGrad && !two) ? resident : std::min(resident, perCu * cus));
         g = std::max(1, std::min(g, std::max(nTiles, 1)));
         grid = g;
         cap = std::max(1, std::min((int)std::ceil(maxSamples / K), 1 << 14));
-        const size_t need = gm ? size_t(grid) * cap * dvr::kBatchBlock : 0;
-        if (need > ckFloats) {
-            dev_free(dCk);
-            dCk = nullptr;
-            ckFloats = 0;
-            dCk = dev_alloc<float>(need);
-            ckFloats = need;
-        }
         // Density store: the forward march keeps every sample's density, so the reverse march
         // reads each segment back (one 4-byte load per sample, all in flight) instead of
         // re-interpolating it (eight gathers per new cell).  Sized for the longest possible ray;
@@ -250,44 +254,63 @@ struct dvr_batch_plan {
         const double dsWant = std::ceil(maxSamples) + 2.0;
         const double dsBytes = double(grid) * dsWant * dvr::kBatchBlock * sizeof(float);
         dsCap = (gm && !reinterpolate && dsBytes <= double(kMaxDensityStore)) ? (int)dsWant : 0;
+        const size_t ckNeed = gm ? size_t(grid) * cap * dvr::kBatchBlock : 0;
         const size_t dsNeed = size_t(grid) * size_t(dsCap) * dvr::kBatchBlock;
-        if (dsNeed > dsFloats) {
-            dev_free(dDs);
-            dDs = nullptr;
-            dsFloats = 0;
-            dDs = dev_alloc<float>(dsNeed);
-            dsFloats = dsNeed;
+        for (int k = 0; k < 2; ++k) {
+            if (grow(dCk, ckFloats, ckNeed) && grow(dDs, dsFloats, dsNeed)) return !two || reserve_adjoints();
+            release_adjoints();  // of an earlier layout
         }
-        check_hip(hipMemcpy(dViews, views.data(), views.size() * sizeof(dvr::BView), hipMemcpyHostToDevice),
-                  "hipMemcpy views");
+        if (two) return false;
+        fail(DVR_ERR_HIP, "hipMalloc failed: no memory for %zu bytes of checkpoints and densities",
+             (ckNeed + dsNeed) * sizeof(float));
     }
 
-    // The density adjoints of as many tiles as kMaxAdjointStore bytes hold (every ray as long as the
+    // at least `need` floats in p; false: no memory (p is then NULL)
+    static bool grow(float*& p, size_t& floats, size_t need)
+    {
+        if (need <= floats) return true;
+        dev_free(p);
+        p = nullptr;
+        floats = 0;
+        if (hipMalloc((void**)&p, need * sizeof(float)) != hipSuccess) {
+            (void)hipGetLastError();
+            p = nullptr;
+            return false;
+        }
+        floats = need;
+        return true;
+    }
+
+    void release_adjoints()
+    {
+        dev_free(dAs);
+        dAs = nullptr;
+        asFloats = 0;
+    }
+
+    // The density adjoints of as many tiles as the store's bytes hold (every ray as long as the
     // longest), at least 4096 (the chip's one-wave workgroups at four waves per SIMD) or all; where
-    // memory is short, half as many and so on.  False: the one-pass instances and their chunk tables.
+    // memory is short, half as many and so on.  The store holds kMaxAdjointStore bytes, but no more than
+    // an eighth of the memory that is free: torch cannot ask a plan to give it back.  False: the one-pass
+    // instances and their chunk tables.
     bool reserve_adjoints()
     {
         const double want = std::ceil(maxSamples) + 2.0;
         if (want > double(1 << 20) || nTiles == 0) return false;
         asCap = dvr::adj_store_cap((int)want);
         const size_t perTile = dvr::adj_store_floats(asCap);
+        size_t freeBytes = 0, total = 0;
+        check_hip(hipMemGetInfo(&freeBytes, &total), "hipMemGetInfo");
+        const long long bytes = std::min(kMaxAdjointStore, (long long)((freeBytes + asFloats * sizeof(float)) / 8));
         const int least = std::max(std::min(nTiles, 4096), (nTiles + kMaxGroups - 1) / kMaxGroups);
-        long long t = std::min<long long>(nTiles, kMaxAdjointStore / (long long)(perTile * sizeof(float)));
+        long long t = std::min<long long>(nTiles, bytes / (long long)(perTile * sizeof(float)));
         for (; t >= least; t = t > least ? std::max<long long>(least, t / 2) : 0) {
             const size_t need = size_t(t) * perTile;
-            if (need > asFloats) {
-                dev_free(dAs);
-                dAs = nullptr;
-                asFloats = 0;
-                if (hipMalloc((void**)&dAs, need * sizeof(float)) != hipSuccess) {
-                    (void)hipGetLastError();
-                    dAs = nullptr;
-                    continue;
-                }
-                asFloats = need;
+            if (need < asFloats) release_adjoints();  // no more than this layout uses
+            if (grow(dAs, asFloats, need)) {
+                groupTiles = (int)t;
+                return true;
             }
-            groupTiles = (int)t;
-            return true;
         }
         return false;
     }
@@ -306,7 +329,7 @@ struct dvr_batch_plan {
         if (evBegin) check_hip(hipEventRecord(evBegin, s), "hipEventRecord");
         for (int k = 0; nTiles > 0 && k < groups(); ++k) {
             const dvr::BatchParams P = params(k);
-            check_hip(dvr::launch_batched(P, filter, tfm, blend, segK(), gmRun(), grid, lds, s, nullptr), "batched launch");
+            check_hip(dvr::launch_batched(P, filter, tfm, blend, segK(), gm_run(twoPass()), grid, lds, s, nullptr), "batched launch");
             if (!twoPass()) continue;
             dvr::ScatterParams S{};
             S.S = P.as;
