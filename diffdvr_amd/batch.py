@@ -215,8 +215,15 @@ class BatchPlan:
 
     @property
     def chunk_slots(self) -> int:
-        """Slots of the per-wave LDS chunk table of the volume gradients (0: none)."""
+        """Slots of the per-wave LDS chunk table of the one-pass volume gradients (0: no volume gradients).
+
+        A plan of two passes (:attr:`volume_passes`) runs without the table."""
         return int(self._h.chunk_slots())
+
+    @property
+    def volume_passes(self) -> int:
+        """Passes of the volume gradients in the current layout (0: none are taken)."""
+        return int(self._h.volume_passes())
 
 
 class Adam:

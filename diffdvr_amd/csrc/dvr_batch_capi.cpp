@@ -117,6 +117,7 @@ struct dvr_batch_plan {
     double* dSums = nullptr;
     dvr::SumSeg* dSumSegs = nullptr;
     int nSums = 0, maxSum = 0;
+    size_t queueBytes = 0;              // of that allocation
     float* dCk = nullptr;
     size_t ckFloats = 0;
     float* dDs = nullptr;   // density store of the forward march (adjoint plans), or NULL
@@ -596,8 +597,8 @@ dvr_batch_plan* create(const dvr_batch* b, const dvr_batch_options* o)
             if (t.adj) add_sum(t.adj, t.R * t.C);
     }
     constexpr size_t kQueues = size_t(kMaxGroups) * dvr::kNumXcd;
-    p->dQueues = reinterpret_cast<unsigned*>(
-        dev_alloc<char>(kQueues * sizeof(unsigned) + nSum * sizeof(double) + sums.size() * sizeof(dvr::SumSeg)));
+    p->queueBytes = kQueues * sizeof(unsigned) + nSum * sizeof(double) + sums.size() * sizeof(dvr::SumSeg);
+    p->dQueues = reinterpret_cast<unsigned*>(dev_alloc<char>(p->queueBytes));
     p->dSums = reinterpret_cast<double*>(p->dQueues + kQueues);
     p->dSumSegs = reinterpret_cast<dvr::SumSeg*>(p->dSums + nSum);
     p->nSums = (int)sums.size();
@@ -892,7 +893,13 @@ int64_t dvr_batch_plan_workspace_bytes(const dvr_batch_plan* plan)
     return (int64_t)((plan->ckFloats + plan->dsFloats + plan->asFloats + plan->brickFloats) * sizeof(float) +
                      plan->nDebrick * sizeof(dvr::DebrickSeg) + plan->views.size() * sizeof(dvr::BView) +
                      plan->vols.size() * sizeof(dvr::BVol) + plan->tfs.size() * sizeof(dvr::BTf) +
-                     plan->nSegsAll * sizeof(dvr::ZeroSeg) + kMaxGroups * dvr::kNumXcd * sizeof(unsigned));
+                     plan->nSegsAll * sizeof(dvr::ZeroSeg) + plan->queueBytes);
+}
+
+int32_t dvr_batch_plan_volume_passes(const dvr_batch_plan* plan)
+{
+    if (!plan) return -1;
+    return (plan->gm & 2) && plan->volGrad ? (plan->twoPass() ? 2 : 1) : 0;
 }
 
 // ---------------------------------------------------------------------------

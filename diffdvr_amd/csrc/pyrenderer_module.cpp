@@ -831,7 +831,8 @@ PYBIND11_MODULE(_pyrenderer, m)
             return py::make_tuple(o.checkpoint_interval, o.wave_width, o.grid, o.reinterpolate != 0);
         })
         .def("workspace_bytes", [](const BatchPlanHandle& h) { return dvr_batch_plan_workspace_bytes(h.plan); })
-        .def("chunk_slots", [](const BatchPlanHandle& h) { return dvr_batch_plan_chunk_slots(h.plan); });
+        .def("chunk_slots", [](const BatchPlanHandle& h) { return dvr_batch_plan_chunk_slots(h.plan); })
+        .def("volume_passes", [](const BatchPlanHandle& h) { return dvr_batch_plan_volume_passes(h.plan); });
 
     py::class_<AdamHandle>(m, "_AdamGroup")
         .def(py::init([](py::list blocks, int device) {

@@ -488,10 +488,16 @@ dvr_status dvr_batch_plan_autotune(dvr_batch_plan* plan, int32_t iterations, dvr
 /* Slots of the per-wave LDS table that sums the volume-gradient corners per 64-byte chunk
  * before the device atomics (the largest of 32..256 that keeps the volume-gradient instance at
  * four waves per SIMD beside the plan's TF tables, for the current options); 0 when the plan
- * takes no volume gradients, -1 for NULL.  No counterpart in the reference (it scatters every
+ * takes no volume gradients, -1 for NULL.  A plan of two passes (dvr_batch_plan_volume_passes) sums
+ * its corners in the second pass and runs without this table: the value is then that of its
+ * one-pass instances.  No counterpart in the reference (it scatters every
  * corner with a device atomic, renderer_interpolation.cuh:299-324). */
 int32_t dvr_batch_plan_chunk_slots(const dvr_batch_plan* plan);
-/* Bytes of device scratch the plan holds (checkpoints, tables). */
+/* How the current layout takes volume gradients: 1, summed by the reverse walk in that table; 2, the walk
+ * stores every sample's density adjoint and a second kernel adds the corners (rays far apart, and memory
+ * for the store); 0, none; -1 for NULL.  No counterpart in the reference. */
+int32_t dvr_batch_plan_volume_passes(const dvr_batch_plan* plan);
+/* Bytes of device scratch the plan holds (checkpoints, densities, density adjoints, sums, tables). */
 int64_t dvr_batch_plan_workspace_bytes(const dvr_batch_plan* plan);
 
 /* ---- optimiser step ------------------------------------------------------

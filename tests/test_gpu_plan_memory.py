@@ -62,3 +62,28 @@ def test_store_follows_the_layout():
         plan.set_options(wave_width=width, grid=1)
         fresh, _ = make_plan(12, 9, 1, grid=1, wave_width=width)
         assert plan.workspace_bytes == fresh.workspace_bytes, width
+
+
+def test_workspace_counts_the_sums_of_a_run():
+    """The double sums of the loss and the TF gradients belong to the plan."""
+    d = dev()
+    bytes_ = []
+    for grads in (False, True):
+        tf = torch.rand(1000, 4, generator=torch.Generator().manual_seed(1)).to(d)
+        view = bt.BatchView(volume=0, tf=0, width=16, height=16, camera=torch.eye(3, device=d), fov_y=0.7, step=0.1,
+                            target=torch.zeros(16, 16, 4, device=d))
+        plan = bt.BatchPlan([bt.BatchVolume(torch.rand(8, 8, 8, device=d), grad=torch.zeros(8, 8, 8, device=d))],
+                            [bt.BatchTf(tf, torch.zeros_like(tf) if grads else None)], [view], loss="l2",
+                            loss_out=torch.zeros(1, device=d) if grads else None)
+        bytes_.append(plan.workspace_bytes)
+    assert bytes_[1] - bytes_[0] >= 8 * (4000 + 1)
+
+
+def test_passes_of_the_volume_gradients():
+    """Two passes up to 5.5 rays a voxel face of the volume (12^3: 144 faces)."""
+    for size, passes in ((12, 2), (28, 2), (29, 1), (64, 1)):
+        plan, _ = make_plan(12, size, 2)
+        assert plan.volume_passes == passes and plan.chunk_slots >= 32
+    view = plan.views[0]
+    plan = bt.BatchPlan(plan.volumes, plan.tfs, [view], tf_mode=0, forward_only=True)
+    assert plan.volume_passes == 0 and plan.chunk_slots == 0
