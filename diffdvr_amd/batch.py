@@ -201,8 +201,8 @@ class BatchPlan:
 
     def autotune(self, iterations: int = 3) -> dict:
         """Time the candidates on this batch and keep the fastest: checkpoint interval K in
-        {4, 8, 16, 32, 64} jointly with the persistent workgroups (1-4 waves per SIMD and full
-        residency, per K), then the wave width (tile 4x16, 8x8, 16x4 or 32x2).  Results are cached
+        {4, 8, 16, 32, 64} jointly with the persistent workgroups (1-4 waves per SIMD, full
+        residency and the default, per K), then the wave width (tile 4x16, 8x8, 16x4 or 32x2).  Results are cached
         per device and batch signature (in the process and a file, see dvr_batch_plan_autotune).
 
         Outputs are overwritten and the gradient buffers left zeroed."""

@@ -799,7 +799,7 @@ dvr_status dvr_batch_plan_autotune(dvr_batch_plan* plan, int32_t iterations, dvr
         hipStream_t s = (hipStream_t)stream;
         const int gridReq = plan->gridReq;
         // the leading tag names the kernels' and search's revision: results of older ones are not reused
-        const std::string tuneKey = "r3|" + plan->signature + (plan->reinterpolate ? "|reinterpolate" : "");
+        const std::string tuneKey = "r4|" + plan->signature + (plan->reinterpolate ? "|reinterpolate" : "");
         Tuned best{0, 0, 0};
         {
             std::lock_guard<std::mutex> lk(g_tuneMu);
@@ -839,13 +839,15 @@ dvr_status dvr_batch_plan_autotune(dvr_batch_plan* plan, int32_t iterations, dvr
                         dvr_batch_options o{K, 8, 0, reint};
                         set_options(plan, &o);
                     }
-                    const int cus = plan->cus, resident = plan->resident;
+                    const int cus = plan->cus, resident = plan->resident, untuned = plan->grid;
                     std::vector<int> grids;
                     if (gridReq > 0) grids.push_back(gridReq);
                     else {
                         for (int k = 1; k <= 4; ++k)  // 1..4 waves per SIMD
                             if (4 * k * cus <= resident) grids.push_back(4 * k * cus);
                         if (grids.empty() || grids.back() < resident) grids.push_back(resident);
+                        // and the default, which need not be a multiple of a wave per SIMD
+                        if (std::find(grids.begin(), grids.end(), untuned) == grids.end()) grids.push_back(untuned);
                     }
                     for (int g : grids) {
                         const float ms = time_it(K, 8, g);
