@@ -612,6 +612,17 @@ public:
         bytes_ = sizeof(float) * (sums_ + brickFloats_ * volumes_ + size_t(group_) * perTile_);
     }
     size_t bytes() const { return bytes_; }
+    // the kernels of a call with (or without) all its scratch: 16 lanes a ray, or one
+    int lanes_per_ray(bool scratch) const
+    {
+        static double present[1];
+        dvr::AdjointParams A = A_;
+        dvr::CkptParams CK{};
+        dvr::LossParams L{};
+        if (scratch && A.atf) A.atfSum = present;
+        if (scratch && group_ > 0) CK.as.adj = reinterpret_cast<float*>(present);
+        return dvr::use_row_adjoint(c_.P, A, CK, L, c_.tfm) ? dvr::kRow : 1;
+    }
     bool holds_sums(const Scratch& scr) const { return scr.bytes >= sums_ * sizeof(float); }
 
     // Runs the adjoint: launch(A, CK) must launch the tiles CK.tile0 .. tile0 + tileN - 1 (0: all).
@@ -1331,6 +1342,30 @@ dvr_status dvr_render_adjoint_scratch(const dvr_inputs* inputs, const dvr_output
         do_adjoint(inputs, outputs_from_forward, adj_color, adj_outputs, options, stream,
                    call_scratch(scratch, scratch_bytes));
     });
+}
+
+int32_t dvr_forward_lanes_per_ray(const dvr_inputs* inputs)
+{
+    int32_t r = -1;
+    guarded([&] {
+        Checked c = check_inputs(inputs);
+        r = !tiled_ok(c) ? 0 : (dvr::use_row_forward(c.P, c.filter) ? dvr::kRow : 1);
+    });
+    return r;
+}
+
+int32_t dvr_adjoint_lanes_per_ray(const dvr_inputs* inputs, const dvr_outputs* outputs_from_forward,
+                                  const dvr_tensor* adj_color, const dvr_adjoint_outputs* adj_outputs,
+                                  const dvr_adjoint_options* options, int32_t with_scratch)
+{
+    int32_t r = -1;
+    guarded([&] {
+        Checked c = check_inputs(inputs);
+        const dvr::AdjointParams A = check_adjoint(c, outputs_from_forward, adj_color, adj_outputs);
+        const bool ckpt = tiled_ok(c) && adjoint_method(c, options) == DVR_ADJOINT_CHECKPOINT;
+        r = ckpt ? AdjointScratch(c, A).lanes_per_ray(with_scratch != 0) : 0;
+    });
+    return r;
 }
 
 int64_t dvr_checkpoint_buffer_elements(const dvr_inputs* inputs, int32_t checkpoint_interval)

@@ -10,6 +10,7 @@ namespace dvr {
 constexpr int kTileW = 8;         // pixels per workgroup tile (x)
 constexpr int kTileH = 8;         // pixels per workgroup tile (y)
 constexpr int kBlock = 64;        // threads per workgroup = one wave of 8x8 rays
+constexpr int kRow = 16;          // lanes (samples) of one ray in the row kernels
 constexpr int kBatchBlock = 64;   // batched persistent kernel: one wave per workgroup, one wave tile per pop
 constexpr int kTfCopies = 4;      // copies of the LDS TF-gradient table, lane & 3 selects one
 // LDS gradient sums are doubles: on MI355X a ds_add_f32 takes 3 clocks a lane (193 a full wave instruction),

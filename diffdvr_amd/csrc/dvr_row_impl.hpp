@@ -44,7 +44,6 @@
 
 namespace dvr {
 
-constexpr int kRow = 16;         // lanes (samples) of one ray
 constexpr int kRowBlock = 256;   // threads of a forward workgroup: 16 rays, 4x4 pixels (a wave: 2x2)
 // Threads of an adjoint workgroup.  The rays of a workgroup share one LDS TF-gradient table: one-wave
 // workgroups add four times as often to the caller's few entries and meet there (identity TF, 2048

@@ -598,6 +598,18 @@ PYBIND11_MODULE(_pyrenderer, m)
           py::arg("inputs"), py::arg("outputs_from_forward"), py::arg("adj_color"), py::arg("adj_outputs"),
           py::arg("method") = "auto", py::arg("path") = "auto", py::arg("checkpoint_interval") = 0,
           py::arg("checkpoints") = py::none(), py::arg("densities") = py::none());
+    m.def("forward_lanes_per_ray", [](const RendererInputs& inputs) {
+        PackedInputs p = pack_inputs(inputs);
+        return dvr_forward_lanes_per_ray(&p.in);
+    });
+    m.def("adjoint_lanes_per_ray", [](const RendererInputs& inputs, const RendererOutputs& fwd, py::object adj_color,
+                                      AdjointOutputs& adj, bool with_scratch) {
+        PackedInputs p = pack_inputs(inputs);
+        dvr_outputs o = pack_outputs(fwd);
+        dvr_tensor ac = to_tensor(adj_color);
+        dvr_adjoint_outputs ao = pack_adjoint(adj);
+        return dvr_adjoint_lanes_per_ray(&p.in, &o, &ac, &ao, nullptr, with_scratch ? 1 : 0);
+    });
     m.def("render_fused",
           [](const RendererInputs& inputs, RendererOutputs& outputs, const std::string& loss, py::object target,
              AdjointOutputs& adj, py::object loss_out, float scale, int checkpoint_interval) {

@@ -203,6 +203,15 @@ dvr_status dvr_render_adjoint_scratch(const dvr_inputs* inputs, const dvr_output
                                       const dvr_adjoint_options* options, void* scratch, int64_t scratch_bytes,
                                       void* stream);
 
+/* Lanes that march one ray in the tiled forward and in the checkpointed adjoint of these inputs: 16 (few
+ * rays, or rays far apart) or 1; 0 where the plain or pre-shaded kernels run, -1 on invalid inputs.  Sample
+ * counts, colours, checkpoints and densities are bitwise the same.  with_scratch: the call is given the
+ * scratch that dvr_adjoint_scratch_bytes asks for.  No counterpart in the reference. */
+int32_t dvr_forward_lanes_per_ray(const dvr_inputs* inputs);
+int32_t dvr_adjoint_lanes_per_ray(const dvr_inputs* inputs, const dvr_outputs* outputs_from_forward,
+                                  const dvr_tensor* adj_color, const dvr_adjoint_outputs* adj_outputs,
+                                  const dvr_adjoint_options* options, int32_t with_scratch);
+
 /* Per-pixel image loss whose gradient the fused kernels form in registers. */
 #define DVR_LOSS_L1 1 /* mean |color - target|   (torch.nn.L1Loss)  */
 #define DVR_LOSS_L2 2 /* mean (color - target)^2 (torch.nn.MSELoss) */
