@@ -22,9 +22,10 @@ W = H = 64
 MODES = [(1, 0, 0, 16), (1, 1, 1, 8), (1, 2, 0, 32), (1, 3, 0, 64), (0, 1, 0, 16), (0, 2, 1, 16), (1, 3, 1, 8), (1, 2, 1, 64)]
 
 
-def scene(filter, tf_mode, blend, step):
+def scene(filter, tf_mode, blend, step, rows=8):
     rng = np.random.default_rng(3300 + 10 * tf_mode + blend + filter)
-    s = camera_scene(rng, W, H, filter=filter, tf_mode=tf_mode, blend=blend, camera=0, smooth=True, X=9, Y=8, Z=10, step=step)
+    s = camera_scene(rng, W, H, filter=filter, tf_mode=tf_mode, blend=blend, camera=0, smooth=True, X=9, Y=8, Z=10, R=rows,
+                     step=step)
     if blend == 1:
         s["tf"][..., 0 if tf_mode == 0 else 3] *= 0.5
     return s, t32(rng.standard_normal((1, H, W, 4)))
@@ -48,10 +49,10 @@ def lanes(inp, color, term, adj, grads, scratch=True):
     return pr._n.adjoint_lanes_per_ray(inp, pr.RendererOutputs(color, term), adj, a, scratch)
 
 
-def check(mode, many_views, grads_list, step):
+def check(mode, many_views, grads_list, step, rows=8):
     filter, tf_mode, blend, K = mode
     print(f"case mode={mode} views={many_views}", flush=True)
-    s, adj = scene(filter, tf_mode, blend, step)
+    s, adj = scene(filter, tf_mode, blend, step, rows)
     few, many = render(s, 1, K), render(s, many_views, K)
     assert pr._n.forward_lanes_per_ray(few[0]) == 16 and pr._n.forward_lanes_per_ray(many[0]) == 1
     assert bool((many[2] == few[2]).all()) and bool((many[1] == few[1]).all())
@@ -88,19 +89,25 @@ def test_tf_and_volume_gradients(mode):
     check(mode, 36, [("tf",), ("volume",), ("tf", "volume"), ("tf", "camera"), ("tf", "volume", "camera", "step")], 0.02)
 
 
+@pytest.mark.parametrize("tf_mode,rows", [(1, 1024), (2, 819), (3, 682)])
+def test_largest_tables(tf_mode, rows):
+    """R * C up to 4096: the staged table, the double sums and the chunk tables take up to 100 KB of LDS."""
+    check((1, tf_mode, 0, 16), 36, [("tf",), ("tf", "volume"), ("tf", "volume", "camera", "step")], 0.04, rows)
+
+
 @pytest.mark.parametrize("mode", [m for m in MODES if m[0] == 1])
 def test_position_gradients(mode):
     """260 views: 16640 tiles, half-voxel steps."""
     check(mode, 260, [("camera", "step"), ("camera",), ("step",)], 0.07)
 
 
-@pytest.mark.parametrize("mode", MODES)
-def test_one_pass_and_fused(mode):
+@pytest.mark.parametrize("mode,rows", [(m, 8) for m in MODES] + [((1, 1, 0, 16), 1024), ((1, 2, 0, 16), 819), ((1, 3, 0, 16), 682)])
+def test_one_pass_and_fused(mode, rows):
     """Volume gradients of the one-pass instances, which fused launches run: the rule is that of a gradient whose
     elements overlap (no second pass)."""
     filter, tf_mode, blend, K = mode
     views = 36
-    s, _ = scene(filter, tf_mode, blend, 0.02)
+    s, _ = scene(filter, tf_mode, blend, 0.02, rows)
     target = torch.rand(1, H, W, 4, generator=torch.Generator().manual_seed(5)).to(dev())
     res = []
     for B in (1, views):
