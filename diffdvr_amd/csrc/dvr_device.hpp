@@ -327,31 +327,36 @@ __device__ __forceinline__ void cell_load(const Vol& V, int ix, int iy, int iz, 
 {
     // z innermost (uniform): four 8-byte loads of z-neighbours instead of eight gathers of 4 bytes.  The
     // marches are bound by the gathers' address and tag cycles: 2 x 1024 x 768 rays through 256^3 1814 ->
-    // 1177 us, 8 x 256 x 256 rays through 128^3 forward 510 -> 470 us.
-    if (V.sz == 1) {
-        const unsigned b = unsigned(iclamp(ix, 0, V.X - 1)) * unsigned(V.sx) +
-                           unsigned(iclamp(iy, 0, V.Y - 1)) * unsigned(V.sy) + unsigned(iclamp(iz, 0, V.Z - 2));
-        const unsigned dx = unsigned(ix) < unsigned(V.X - 1) ? unsigned(V.sx) : 0u;
-        const unsigned dy = unsigned(iy) < unsigned(V.Y - 1) ? unsigned(V.sy) : 0u;
-        const vfloat2 v0 = gld2(V.p, b), v1 = gld2(V.p, b + dy), v2 = gld2(V.p, b + dx), v3 = gld2(V.p, b + dx + dy);
+    // 1177 us, 8 x 256 x 256 rays through 128^3 forward 510 -> 470 us.  The addresses are formed in front of
+    // the branch: either side formed its own before, in registers of d that the other side's loads might
+    // have been filling for all the compiler knew, and waited for every access in flight, the store of the last
+    // sample's density among them.
+    const bool pair = V.sz == 1;
+    const unsigned dx = unsigned(ix) < unsigned(V.X - 1) ? unsigned(V.sx) : 0u;
+    const unsigned dy = unsigned(iy) < unsigned(V.Y - 1) ? unsigned(V.sy) : 0u;
+    const bool inside = unsigned(iz) < unsigned(V.Z - 1);
+    const unsigned dz = inside ? unsigned(V.sz) : 0u;
+    const unsigned b0 = unsigned(iclamp(ix, 0, V.X - 1)) * unsigned(V.sx) + unsigned(iclamp(iy, 0, V.Y - 1)) * unsigned(V.sy) +
+                        unsigned(iclamp(iz, 0, pair ? V.Z - 2 : V.Z - 1)) * unsigned(V.sz);
+    const unsigned b1 = b0 + dy, b2 = b0 + dx, b3 = b2 + dy;
+    if (pair) {
+        const vfloat2 v0 = gld2(V.p, b0), v1 = gld2(V.p, b1), v2 = gld2(V.p, b2), v3 = gld2(V.p, b3);
         d[0] = v0.x; d[1] = v0.y; d[2] = v1.x; d[3] = v1.y; d[4] = v2.x; d[5] = v2.y; d[6] = v3.x; d[7] = v3.y;
-        if (unsigned(iz) >= unsigned(V.Z - 1)) {  // one voxel for both corners, at either end
+        if (!inside) {  // one voxel for both corners, at either end
             const bool hi = iz > 0;
 #pragma unroll
             for (int k = 0; k < 8; k += 2) d[k] = d[k + 1] = hi ? d[k + 1] : d[k];
         }
         return;
     }
-    const CellOffsets o = cell_offsets(ix, iy, iz, V.X, V.Y, V.Z, V.sx, V.sy, V.sz);
-    const unsigned b = o.base, xy = o.dx + o.dy;
-    d[0] = gld(V.p, b);
-    d[1] = gld(V.p, b + o.dz);
-    d[2] = gld(V.p, b + o.dy);
-    d[3] = gld(V.p, b + o.dy + o.dz);
-    d[4] = gld(V.p, b + o.dx);
-    d[5] = gld(V.p, b + o.dx + o.dz);
-    d[6] = gld(V.p, b + xy);
-    d[7] = gld(V.p, b + xy + o.dz);
+    d[0] = gld(V.p, b0);
+    d[1] = gld(V.p, b0 + dz);
+    d[2] = gld(V.p, b1);
+    d[3] = gld(V.p, b1 + dz);
+    d[4] = gld(V.p, b2);
+    d[5] = gld(V.p, b2 + dz);
+    d[6] = gld(V.p, b3);
+    d[7] = gld(V.p, b3 + dz);
 }
 
 __device__ __forceinline__ float tri_lerp(const float d[8], float fx, float fy, float fz)
