@@ -896,6 +896,11 @@ __global__ __launch_bounds__(kBlock) void k_forward_tiled(RenderParams P, CkptPa
     P.term[tc.b * P.termSb + tc.y * P.termSy + tc.x * P.termSx] = n;
 }
 
+// Doubles between the copies of the TF-gradient table.  One-pass volume instances take one table: four copies of
+// a 64-row texture's left their chunk table 32 slots instead of 64 (GM 3), or five workgroups a CU instead of
+// seven beside 256 slots (GM 7): 16 views of 256 x 256, 128^3, 3065 us with one float table, 4127 with the copies.
+inline __host__ __device__ int tiled_copy_stride(int gm, int RC) { return (gm & 2) ? 0 : tf_grad_copy_stride(RC); }
+
 // Volume + TF gradient instances (GM 3) are compiled for four waves per SIMD
 // (the walk is latency-bound, as in the batched kernel); the others keep the
 // compiler's default register budget.
@@ -909,7 +914,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(GM == 3 
     float* s_tf = lds;
     const int tfFloats = tf_grad_offset(P.R * tf_lds_stride<TFM>());
     float* s_g = lds + tfFloats;
-    const int copyStride = tf_grad_copy_stride(RC);
+    const int copyStride = tiled_copy_stride(GM, RC);
     const TileXY tc = tile_xy(tilesX, tilesPerView, nTiles, CK.tile0);
     const bool wantTf = A.atf != nullptr;
     const int ng = wantTf ? tf_grad_floats(RC, usePriv != 0, kBlock, copyStride) : 0;
@@ -1047,7 +1052,7 @@ static hipError_t adj_tiled_k(const RenderParams& P, const AdjointParams& A, con
     if (nTiles == 0) return hipSuccess;
     const int RC = P.R * P.C;
     const bool usePriv = (TFM == 3) && A.atf && RC <= 48;  // private slices <= 48 KiB of LDS
-    const int ng = A.atf ? tf_grad_floats(RC, usePriv, kBlock, tf_grad_copy_stride(RC)) : 0;
+    const int ng = A.atf ? tf_grad_floats(RC, usePriv, kBlock, tiled_copy_stride(GM, RC)) : 0;
     const int tfFloats = tf_grad_offset(P.R * tf_lds_stride<TFM>());
     int aggLog2 = kAggLog2;
     size_t lds;
