@@ -902,10 +902,12 @@ __global__ __launch_bounds__(kBlock) void k_forward_tiled(RenderParams P, CkptPa
 inline __host__ __device__ int tiled_copy_stride(int gm, int RC) { return (gm & 2) ? 0 : tf_grad_copy_stride(RC); }
 
 // Volume + TF gradient instances (GM 3) are compiled for four waves per SIMD
-// (the walk is latency-bound, as in the batched kernel); the others keep the
-// compiler's default register budget.
+// (the walk is latency-bound, as in the batched kernel), the Gaussian TF +
+// position instances (GM 5) for three, which 176 registers missed by one step of
+// the allocation: 64^3, 4096 tiles 567 us before, 671 us with them.  The others keep
+// the compiler's default register budget.
 template <int FILTER, int TFM, int BLEND, int K, int GM>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(GM == 3 ? 4 : 1))) void k_adjoint_tiled(
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(GM == 3 ? 4 : (GM == 5 && TFM == 3 ? 3 : 1)))) void k_adjoint_tiled(
     RenderParams P, AdjointParams A, CkptParams CK, LossParams L, int fused, int ckFromFwd, int usePriv, int tilesX,
     int tilesPerView, int nTiles, int aggLog2)
 {
