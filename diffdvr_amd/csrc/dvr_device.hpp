@@ -323,6 +323,7 @@ __device__ __forceinline__ vfloat2 gld2(const float* base, unsigned idx)
     return *(const gfloat2*)((const gchar*)base + idx * 4u);
 }
 
+template <bool PAIRS = true>
 __device__ __forceinline__ void cell_load(const Vol& V, int ix, int iy, int iz, float d[8])
 {
     // z innermost (uniform): four 8-byte loads of z-neighbours instead of eight gathers of 4 bytes.  The
@@ -331,7 +332,7 @@ __device__ __forceinline__ void cell_load(const Vol& V, int ix, int iy, int iz, 
     // the branch: either side formed its own before, in registers of d that the other side's loads might
     // have been filling for all the compiler knew, and waited for every access in flight, the store of the last
     // sample's density among them.
-    const bool pair = V.sz == 1;
+    const bool pair = PAIRS && V.sz == 1;
     const unsigned dx = unsigned(ix) < unsigned(V.X - 1) ? unsigned(V.sx) : 0u;
     const unsigned dy = unsigned(iy) < unsigned(V.Y - 1) ? unsigned(V.sy) : 0u;
     const bool inside = unsigned(iz) < unsigned(V.Z - 1);
@@ -376,7 +377,7 @@ __device__ __forceinline__ int nearest_offset(const Vol& V, f3 p)
 }
 
 
-template <int FILTER>
+template <int FILTER, bool PAIRS = true>
 __device__ __forceinline__ float fetch(const Vol& V, f3 p, Cell& c)
 {
     if constexpr (FILTER == 0) {
@@ -384,7 +385,7 @@ __device__ __forceinline__ float fetch(const Vol& V, f3 p, Cell& c)
     } else {
         const int ix = int(p.x), iy = int(p.y), iz = int(p.z);
         if (ix != c.ix || iy != c.iy || iz != c.iz) {
-            cell_load(V, ix, iy, iz, c.d);
+            cell_load<PAIRS>(V, ix, iy, iz, c.d);
             c.ix = ix; c.iy = iy; c.iz = iz;
         }
         return tri_lerp(c.d, p.x - float(ix), p.y - float(iy), p.z - float(iz));
@@ -406,18 +407,19 @@ __device__ __forceinline__ float fetch(const Vol& V, f3 p, Cell& c)
 //   request(V, pn) issue the loads of the cell of pn if it differs; pn's cell
 //                 is current from here on (its first use waits for the loads)
 //   advance()     nothing left to do (kept for the nearest filter's pipe)
+// PAIRS: see cell_load.
 // ---------------------------------------------------------------------------
-template <int FILTER>
+template <int FILTER, bool PAIRS = true>
 struct FetchPipe;
 
-template <>
-struct FetchPipe<1> {
+template <bool PAIRS>
+struct FetchPipe<1, PAIRS> {
     int ix, iy, iz;
     float d[8];
     __device__ __forceinline__ void start(const Vol& V, f3 p)
     {
         ix = int(p.x); iy = int(p.y); iz = int(p.z);
-        cell_load(V, ix, iy, iz, d);
+        cell_load<PAIRS>(V, ix, iy, iz, d);
     }
     __device__ __forceinline__ float value(f3 p) const
     {
@@ -427,15 +429,15 @@ struct FetchPipe<1> {
     {
         const int jx = int(pn.x), jy = int(pn.y), jz = int(pn.z);
         if ((jx != ix) | (jy != iy) | (jz != iz)) {
-            cell_load(V, jx, jy, jz, d);
+            cell_load<PAIRS>(V, jx, jy, jz, d);
             ix = jx; iy = jy; iz = jz;
         }
     }
     __device__ __forceinline__ void advance() {}
 };
 
-template <>
-struct FetchPipe<0> {
+template <bool PAIRS>
+struct FetchPipe<0, PAIRS> {
     float v, nv;
     __device__ __forceinline__ void start(const Vol& V, f3 p) { v = gld(V.p, unsigned(nearest_offset(V, p))); }
     __device__ __forceinline__ float value(f3) const { return v; }

@@ -676,6 +676,10 @@ __device__ __forceinline__ void march_reverse(const Vol& V, const Tf& T, const R
 #pragma unroll
     for (int k = 0; k < 8; ++k) { cc.w[k] = 0.f; cc.d[k] = 0.f; }
     int nLast = -1;
+    // Without a density store the segments are interpolated again.  One-pass volume instances (128 registers) read single voxels
+    // there: with pairs the walk had to reload the ray from scratch memory at every sample (linear TF, 4 x 256 x
+    // 256 rays through 192^3 3792 us with single loads, 4144 with pairs).
+    constexpr bool kPairs = (GM & 2) == 0;
     float nAcc = 0.0f;
 
     const int nseg = (n + K - 1) / K;
@@ -694,7 +698,7 @@ __device__ __forceinline__ void march_reverse(const Vol& V, const Tf& T, const R
             cell_invalidate(cc);
             for (int i = c << ckShift; i < i0; ++i) {
                 const float t = r.t0 + float(i) * r.step;
-                const float d = dsr ? *(const gfloat*)(dsr + i * dsS) : fetch<FILTER>(V, sample_pos(r, t), cc);
+                const float d = dsr ? *(const gfloat*)(dsr + i * dsS) : fetch<FILTER, kPairs>(V, sample_pos(r, t), cc);
                 float alpha, keep;
                 alpha_keep<BLEND>(tf_absorption<TFM, true>(T, d), r.step, alpha, keep);
                 Tr *= keep;
@@ -725,7 +729,7 @@ __device__ __forceinline__ void march_reverse(const Vol& V, const Tf& T, const R
                 Tr *= keep;
             }
         } else {
-            FetchPipe<FILTER> pipe;
+            FetchPipe<FILTER, kPairs> pipe;
             f3 p = sample_pos(r, r.t0 + float(i0) * r.step);
             pipe.start(V, p);
 #pragma unroll
