@@ -6,9 +6,9 @@ namespace dvr {
 // At most 2^20 tiles of 1024 threads: a launch holds less than 2^32 threads.
 constexpr int kMaxRowTiles = 1 << 20;
 
-// samples per voxel edge and voxel edges per pixel, both averaged over the axes;
+// voxel edges per step and voxel edges per pixel, both averaged over the axes;
 // a per-ray step or a box in device memory counts as the usual half voxel / unit box
-static float step_voxels(const RenderParams& P)
+float step_voxels(const RenderParams& P)
 {
     if (P.st || P.bsize) return 0.5f;
     const float n[3] = {float(P.X - 1), float(P.Y - 1), float(P.Z - 1)};
@@ -16,7 +16,7 @@ static float step_voxels(const RenderParams& P)
     for (int a = 0; a < 3; ++a) v += P.stU * n[a] / (3.0f * P.bsizeU[a]);
     return v;
 }
-static float pixel_voxels(const RenderParams& P)
+float pixel_voxels(const RenderParams& P)
 {
     return float(P.X + P.Y + P.Z) / (3.0f * float(P.W < P.H ? P.W : P.H));
 }
@@ -47,11 +47,18 @@ bool use_row_forward(const RenderParams& P, int filter)
     return tiles <= (large && g >= 0.24f ? 16384 : 4096);
 }
 
-// Position gradients alone (row_reverse): 220 against 636 us at 2048 tiles, 486 / 786 at 8192, 947 /
-// 1295 at 16384 (Gaussian TF, 4 rows); with steps below 0.4 voxel 4290 / 5011 at 32768.  Volume
-// gradients (split_reverse) in two passes: 185 / 262 and 273 / 277 us at 1024 tiles, 415 / 350 at
+// Position gradients alone (row_reverse): the row kernel gains with the samples of a ray, which the tiled
+// kernel walks one after the other, with their distance (its gathers then meet in fewer lines than 64 rays')
+// and with the cost of a sample's shading, which it does once; it loses with the tiles, which fill the chip
+// without it.  Up to 1024 tiles always, then up to c x (samples per axis) x sqrt(voxels per pixel): over 570
+// launches of 1024 to 32768 tiles this is 0.3 % off the better kernel on average, 19 % at most.  Row / tiled,
+// us: identity TF, 128^3, 4096 tiles 210 / 243 at 0.5 voxels a pixel, 296 / 251 at 0.25, 64^3, 16384 tiles 534 / 257;
+// linear 418 / 494 and 652 / 748 at 128^3, 8192 tiles, 578 / 435 at 64^3, 16384; Gaussian of four rows 968 / 1358
+// at 128^3, 16384, 513 / 371 at 32^3.
+// Volume gradients (split_reverse) in two passes: 185 / 262 and 273 / 277 us at 1024 tiles, 415 / 350 at
 // 2048; in one pass 634 / 1038 at 2048, 2707 / 2684 at 4096.  TF gradients: 137 / 160 us at 1024
-// tiles, 238 / 184 at 2048; the identity TF's walk is short, 53 / 65 at 576 and 83 / 67 at 1024.
+// tiles, 238 / 184 at 2048; the identity TF's walk is short, 53 / 65 at 576 and 83 / 67 at 1024, but beside the
+// forward march of a fused launch the row kernel pays up to 1024 (90 / 91 at 64^3, 224 / 346 at 256^3).
 // The loss and TF gradients are summed in doubles: the row kernel adds four times a tile, and 4096 or more
 // floats added to one scalar in any order are off by 1e-6 of it and more.  Without memory for these sums the
 // tiled kernel runs.
@@ -60,8 +67,10 @@ bool use_row_adjoint(const RenderParams& P, const AdjointParams& A, const CkptPa
     const int tiles = tiled_num_tiles(P);
     if (tiles > kMaxRowTiles || (L.lossOut && !L.lossSum) || (A.atf && !A.atfSum)) return false;
     if (A.avol) return tiles <= (CK.as.adj ? 1024 : 2048);
-    if (A.atf) return tiles <= (tfm == 0 && !A.ars && !A.ast ? 768 : 1024);
-    return tiles <= 16384 || step_voxels(P) < 0.4f;
+    if (A.atf) return tiles <= (tfm == 0 && !A.ars && !A.ast && !L.target ? 768 : 1024);
+    const float samples = float(P.X + P.Y + P.Z) / (3.0f * step_voxels(P));
+    const float c = tfm == 3 ? 266.0f : (tfm == 2 ? 94.0f : 33.0f);
+    return tiles <= 1024 || float(tiles) <= c * samples * sqrtf(pixel_voxels(P));
 }
 
 template <int FILTER, int TFM, int BLEND>

@@ -63,6 +63,8 @@ hipError_t launch_adjoint_tiled(const RenderParams& P, const AdjointParams& A, c
                                 int blend, hipStream_t s);
 
 // dvr_kernels_row.hip: the same, 16 lanes a ray, and the sizes at which they are faster
+float step_voxels(const RenderParams& P);   // voxel edges per step and per pixel
+float pixel_voxels(const RenderParams& P);
 bool use_row_forward(const RenderParams& P, int filter);
 bool use_row_adjoint(const RenderParams& P, const AdjointParams& A, const CkptParams& CK, const LossParams& L, int tfm);
 hipError_t launch_forward_row(const RenderParams& P, const CkptParams& CK, int filter, int tfm, int blend,
