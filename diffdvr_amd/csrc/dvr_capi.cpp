@@ -607,8 +607,10 @@ public:
     AdjointScratch(const Checked& c, const dvr::AdjointParams& A) : c_(c), A_(A), tiles_(dvr::tiled_num_tiles(c.P))
     {
         if (c.preshaded || tiles_ == 0) return;
-        sums_ = tf_sum_floats(c, A);
         plan_volume();
+        // the row kernel needs the sums; for the tiled kernel's one addition a tile the two launches beside it (8 us)
+        // pay from 1024 tiles on
+        if (tiles_ >= 1024 || lanes_per_ray(true) > 1) sums_ = tf_sum_floats(c, A);
         bytes_ = sizeof(float) * (sums_ + brickFloats_ * volumes_ + size_t(group_) * perTile_);
     }
     size_t bytes() const { return bytes_; }
@@ -938,10 +940,18 @@ void do_fused(const dvr_inputs* inputs, dvr_outputs* outputs, const dvr_loss* lo
     hipStream_t s = (hipStream_t)stream;
     const int64_t need = (int64_t)dvr::tiled_num_tiles(c.P) * CK.cap * dvr::kBlock;
     ScratchLease lease(c.device, s);  // the scratch (either kind), until the launches are enqueued
-    // the call's sums of the loss and the TF gradient lie behind the checkpoints; where the static scratch has
-    // no room left the workgroups add floats to the caller's (the tiled kernel, once a tile)
+    // The call's sums of the loss and the TF gradient lie behind the checkpoints: for the row kernel, and from
+    // 2048 tiles on; below, the two launches beside it (8 us of 80 at 1024 tiles) would count.  Otherwise, and
+    // where the static scratch has no room left, the tiled kernel adds floats to the caller's, once a tile.
     const int64_t lossFloats = L.lossOut ? 2 * dvr::kLossSlots * dvr::kLossStride : 0;
-    const int64_t sums = lossFloats + (int64_t)tf_sum_floats(c, A);
+    int64_t sums = lossFloats + (int64_t)tf_sum_floats(c, A);
+    if (dvr::tiled_num_tiles(c.P) < 2048) {
+        double present[1];
+        dvr::AdjointParams rowA = A;
+        dvr::LossParams rowL = L;
+        rowA.atfSum = rowL.lossSum = present;
+        if (!dvr::use_row_adjoint(c.P, rowA, CK, rowL, c.tfm)) sums = 0;
+    }
     if (fixed) {
         // checkpoints in the device's static scratch; no density store (the reverse march
         // re-interpolates: the same densities)
