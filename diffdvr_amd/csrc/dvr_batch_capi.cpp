@@ -81,6 +81,7 @@ struct dvr_batch_plan {
     int device = 0;
     int filter = 1, tfm = 0, blend = 0, gm = 0, lossKind = 0;
     bool volGrad = false;  // some volume gradient is requested (the chunk table is needed)
+    bool tfGrad = false;   // some TF gradient is requested (the LDS gradient table is needed)
     float earlyOut = 1.0f - 1e-5f;
     float* lossOut = nullptr;
     std::vector<dvr::BView> views;  // sorted by (tf, volume); tileBegin/tilesX set by layout()
@@ -96,6 +97,7 @@ struct dvr_batch_plan {
     bool reinterpolate = false;  // no density store
     int cus = 0, resident = 0;  // compute units, resident workgroups of the current instance
     size_t lds = 0;
+    int tfCopyStride = 0;  // doubles between the copies of the LDS TF-gradient table (0: one table)
     int aggOffset = 0;  // float offset of the volume-gradient chunk table in LDS (0: none)
     int aggLog2 = dvr::kAggLog2;  // log2 of the chunk table's slots
     // device
@@ -136,15 +138,13 @@ struct dvr_batch_plan {
         dev_free(dDs); dev_free(dAs); dev_free(dBricks); dev_free(dDebrick);
     }
 
-    // doubles between the TF-gradient table copies; 0 (one table) when the copies would take more than
-    // 16 KiB of LDS per workgroup, which keeps eight one-wave workgroups resident per CU
-    int copy_stride() const { return dvr::tf_grad_copy_stride(maxRC); }
-
     // floats of the LDS TF table (linear and Gaussian rows take 8 floats, dvr::tf_lds_stride), even
     int tf_lds() const { return dvr::tf_grad_offset(tfm >= 2 ? (maxRC / tf_cols(tfm)) * 8 : maxRC); }
 
-    // register segment length of checkpoint interval K (64 = two 32-sample segments)
-    int segK() const { return K > 32 ? 32 : K; }
+    // Register segment length of checkpoint interval K: at most 32 samples, eight in the one-pass volume instances.
+    // Their 128 registers hold no longer segment: with 16 samples and double sums 407 values are spilled for a
+    // texture TF, 12 with eight (128^3, 8 views of 512 x 512, interval 16: 5554 / 3206 us, 4402 with float sums).
+    int segK(bool two) const { return std::min(K, gm == 3 && !two ? 8 : 32); }
 
     bool twoPass() const { return groupTiles > 0; }
     int gm_run(bool two) const { return two ? (gm & 4 ? 13 : 9) : gm; }
@@ -156,7 +156,7 @@ struct dvr_batch_plan {
         P.views = dViews; P.vols = dVols; P.tfs = dTfs; P.ck = dCk; P.lossOut = lossOut ? dSums : nullptr;
         P.ds = dsCap > 0 ? dDs : nullptr; P.dsCap = dsCap;
         P.nViews = (int)views.size(); P.nTiles = nTiles; P.ckCap = cap;
-        P.ckEvery = K > 32 ? K / 32 : 1;
+        P.ckEvery = K / segK(twoPass());
         // the group's tiles, one range per XCD
         const int t0 = twoPass() ? group * groupTiles : 0, t1 = twoPass() ? std::min(nTiles, t0 + groupTiles) : nTiles;
         for (int q = 0; q <= dvr::kNumXcd; ++q) P.qBegin[q] = t0 + (int)((long long)(t1 - t0) * q / dvr::kNumXcd);
@@ -168,7 +168,7 @@ struct dvr_batch_plan {
         P.waveShift = wave_shift_of(waveWidth);
         P.tileW = waveWidth; P.tileH = 64 / waveWidth;
         P.ldsTf = tf_lds(); P.usePriv = usePriv ? 1 : 0;
-        P.tfCopyStride = (gm && !usePriv) ? copy_stride() : 0;
+        P.tfCopyStride = tfCopyStride;
         P.ldsAgg = twoPass() ? 0 : aggOffset;
         P.aggLog2 = aggLog2;
         return P;
@@ -206,33 +206,48 @@ struct dvr_batch_plan {
     }
 
     // LDS, grid and scratch of one scheme of the volume gradients.  The checkpoints and densities are
-    // allocated first; two passes: false where these or the adjoint store find no memory.
+    // allocated first; two passes: false where these or the adjoint store find no memory.  The TF-gradient and chunk
+    // tables take LDS only where such gradients are wanted.
     bool layout_scratch(bool two)
     {
-        const size_t ldsG = gm ? size_t(dvr::tf_grad_floats(maxRC, usePriv, dvr::kBatchBlock, copy_stride())) : 0;
-        lds = sizeof(float) * (size_t(tf_lds()) + ldsG);
-        // volume gradients: the per-wave table of 64-byte chunks follows the TF tables (not
-        // reserved for camera-only plans, which run the same instance without it)
-        aggOffset = 0;
         int occ = 0;
         groupTiles = 0;
+        // floats of the LDS TF-gradient table with copies `stride` doubles apart
+        auto tf_floats = [&](int stride) { return tfGrad ? dvr::tf_grad_floats(maxRC, usePriv, dvr::kBatchBlock, stride) : 0; };
+        auto query = [&] {
+            check_hip(dvr::launch_batched(params(), filter, tfm, blend, segK(two), gm_run(two), 0, lds, nullptr, &occ),
+                      "occupancy query");
+        };
+        // copies of the TF-gradient table where they take at most 16 KiB of LDS per workgroup, which keeps eight
+        // one-wave workgroups resident per CU
+        tfCopyStride = tfGrad && !usePriv ? dvr::tf_grad_copy_stride(maxRC) : 0;
+        aggOffset = 0;
         if ((gm & 2) && volGrad) {
-            // the largest table that keeps the instance at the waves per SIMD its registers
-            // were fitted for (workgroups per CU from the runtime's occupancy calculator)
-            aggOffset = dvr::agg_offset(tf_lds(), (int)ldsG);
+            // one pass: the per-wave table of 64-byte chunks follows the TF tables, the largest that keeps the
+            // instance at the waves per SIMD its registers were fitted for (workgroups per CU from the runtime's
+            // occupancy calculator).  It goes before the copies: 64-row textures hold 64 slots without them, 32
+            // with them (128^3, 8 views of 512 x 512: 2846 / 3206 us).
             const int target = 4 * dvr::batched_vol_waves(gm);
-            for (int lg = dvr::kAggLog2; lg >= dvr::kAggMinLog2; --lg) {
-                aggLog2 = lg;
-                lds = sizeof(float) * size_t(aggOffset) + dvr::agg_bytes(lg, sizeof(double));
-                check_hip(dvr::launch_batched(params(), filter, tfm, blend, segK(), gm, 0, lds, nullptr, &occ),
-                          "occupancy query");
-                if (occ >= target) break;
+            auto fit = [&](int stride) {
+                aggOffset = dvr::agg_offset(tf_lds(), tf_floats(stride));
+                for (int lg = dvr::kAggLog2; lg >= dvr::kAggMinLog2; --lg) {
+                    aggLog2 = lg;
+                    lds = sizeof(float) * size_t(aggOffset) + dvr::agg_bytes(lg, sizeof(double));
+                    check_hip(dvr::launch_batched(params(), filter, tfm, blend, segK(false), gm, 0, lds, nullptr, &occ),
+                              "occupancy query");
+                    if (occ >= target) break;
+                }
+                return std::make_pair(std::min(occ, target), aggLog2);
+            };
+            const auto single = fit(0);
+            if (tfCopyStride > 0 && fit(tfCopyStride) != single) {
+                if (!two) tfCopyStride = 0;
+                fit(0);
             }
         }
-        if (two || occ == 0) {
-            if (two) lds = sizeof(float) * (size_t(tf_lds()) + ldsG);
-            check_hip(dvr::launch_batched(params(), filter, tfm, blend, segK(), gm_run(two), 0, lds, nullptr, &occ),
-                      "occupancy query");
+        if (two || !((gm & 2) && volGrad)) {
+            lds = sizeof(float) * (size_t(tf_lds()) + size_t(tf_floats(tfCopyStride)));
+            query();
         }
         resident = std::max(1, occ) * cus;
         // default, within residency: two waves per SIMD (eight one-wave workgroups per CU): gather-bound
@@ -330,7 +345,7 @@ struct dvr_batch_plan {
         if (evBegin) check_hip(hipEventRecord(evBegin, s), "hipEventRecord");
         for (int k = 0; nTiles > 0 && k < groups(); ++k) {
             const dvr::BatchParams P = params(k);
-            check_hip(dvr::launch_batched(P, filter, tfm, blend, segK(), gm_run(twoPass()), grid, lds, s, nullptr), "batched launch");
+            check_hip(dvr::launch_batched(P, filter, tfm, blend, segK(twoPass()), gm_run(twoPass()), grid, lds, s, nullptr), "batched launch");
             if (!twoPass()) continue;
             dvr::ScatterParams S{};
             S.S = P.as;
@@ -573,6 +588,7 @@ dvr_batch_plan* create(const dvr_batch* b, const dvr_batch_options* o)
             fail(DVR_ERR_NO_GRADIENT, "At least one adjoint variable must be activated!");
         p->gm = anyCamGrad ? (anyVolGrad ? 7 : 5) : (anyVolGrad ? 3 : 1);
         p->volGrad = anyVolGrad;
+        p->tfGrad = anyTfGrad;
     }
     p->usePriv = p->gm && b->tf_mode == DVR_TF_GAUSSIAN && p->maxRC <= 48;
 

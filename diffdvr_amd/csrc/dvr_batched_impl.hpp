@@ -286,7 +286,9 @@ static hipError_t batched_fbk(const BatchParams& P, int tfm, int gm, int grid, s
         if constexpr (K == 16) return batched_k<FILTER, TV, BLEND, K, 0>(P, grid, lds, s, occ); \
         else return hipErrorInvalidValue;                                          \
     case 1: return batched_k<FILTER, TV, BLEND, K, 1>(P, grid, lds, s, occ);       \
-    case 3: return batched_k<FILTER, TV, BLEND, K, 3>(P, grid, lds, s, occ);       \
+    case 3:                                                                        \
+        if constexpr (K <= 8) return batched_k<FILTER, TV, BLEND, K, 3>(P, grid, lds, s, occ); \
+        return hipErrorInvalidValue; /* segments of at most eight samples */       \
     case 5: return batched_k<FILTER, TV, BLEND, K, 5>(P, grid, lds, s, occ);       \
     case 7: return batched_k<FILTER, TV, BLEND, K, 7>(P, grid, lds, s, occ);       \
     case 9: return batched_k<FILTER, TV, BLEND, K, 9>(P, grid, lds, s, occ);       \
