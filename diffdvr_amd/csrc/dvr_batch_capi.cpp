@@ -90,6 +90,7 @@ struct dvr_batch_plan {
     int maxRC = 0;
     bool usePriv = false;
     bool farRays = false;   // most samples: at most 1.5 rays per voxel face of a volume of at least 8 M voxels
+    bool sparseRays = false;  // most samples: at most 2 rays per voxel face of a volume of at least 4 M voxels
     double rayDensity = 0;  // rays per voxel face of a view, averaged over the samples of the volume gradients
     double maxSamples = 0;  // upper bound of samples per ray over the views
     // layout
@@ -143,7 +144,7 @@ struct dvr_batch_plan {
 
     // Register segment length of checkpoint interval K: at most 32 samples, eight in the one-pass volume instances.
     // Their 128 registers hold no longer segment: with 16 samples and double sums 407 values are spilled for a
-    // texture TF, 12 with eight (128^3, 8 views of 512 x 512, interval 16: 5554 / 3206 us, 4402 with float sums).
+    // texture TF, 12 with eight (128^3, 8 views of 512 x 512, interval 16: 5554 / 2724 us).
     int segK(bool two) const { return std::min(K, gm == 3 && !two ? 8 : 32); }
 
     bool twoPass() const { return groupTiles > 0; }
@@ -257,8 +258,9 @@ struct dvr_batch_plan {
         // face, us with 8 / 5: texture 1700 / 1350, linear 1885 / 1575, volume gradients 8140 / 7290; 192^3
         // 1147 / 1185; four rays a face 3712 / 3826).  Twelve for Gaussian TFs, which are bound by VALU
         // issue (8 / 12: cameras 2664 / 2052, TF 2259 / 1878; with the second pass of volume gradients
-        // 2976 / 3156).
-        const int perCu = gm && tfm == 3 && !two ? 12 : (gm && tfm != 3 && farRays ? 5 : 8);
+        // 2976 / 3156), but not where at most two rays meet a voxel face of a large volume (TF, 256^3, one ray a face
+        // 2666 / 3208, 192^3, 1.8 rays 1577 / 1769; 128^3, four rays 1318 / 1217; 256^3, four rays 4254 / 3377).
+        const int perCu = gm && tfm == 3 && !two ? (sparseRays ? 8 : 12) : (gm && tfm != 3 && farRays ? 5 : 8);
         int g = gridReq > 0 ? gridReq : (((gm & 2) && volGrad && !two) ? resident : std::min(resident, perCu * cus));
         g = std::max(1, std::min(g, std::max(nTiles, 1)));
         grid = g;
@@ -521,7 +523,7 @@ dvr_batch_plan* create(const dvr_batch* b, const dvr_batch_options* o)
         p->tfs.push_back(d);
     }
     long long totalPix = 0;
-    double volSamples = 0, volDensity = 0, allSamples = 0, farSamples = 0;
+    double volSamples = 0, volDensity = 0, allSamples = 0, farSamples = 0, sparseSamples = 0;
     std::vector<dvr::BView> vs;
     for (int i = 0; i < b->num_views; ++i) {
         const dvr_batch_view& v = b->views[i];
@@ -564,6 +566,7 @@ dvr_batch_plan* create(const dvr_batch* b, const dvr_batch_options* o)
         const double voxels = double(vol.X) * vol.Y * vol.Z, density = v.width * double(v.height) / std::pow(voxels, 2.0 / 3.0);
         allSamples += samples;
         if (density <= 1.5 && voxels >= double(8 << 20)) farSamples += samples;
+        if (density <= 2.0 && voxels >= 4.0e6) sparseSamples += samples;
         if (vol.adj) {
             volSamples += samples;
             volDensity += samples * density;
@@ -581,6 +584,7 @@ dvr_batch_plan* create(const dvr_batch* b, const dvr_batch_options* o)
     });
     p->views = vs;
     p->farRays = farSamples > 0.5 * allSamples;
+    p->sparseRays = sparseSamples > 0.5 * allSamples;
     p->rayDensity = volSamples > 0 ? volDensity / volSamples : 0.0;
     if (b->forward_only) p->gm = 0;
     else {
