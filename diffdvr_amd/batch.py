@@ -6,7 +6,8 @@ over ``Renderer.render_forward`` / ``render_adjoint`` per view
 (pytests/diffdvr/renderer.py:127-213) and sum the gradients in torch.  Here a
 :class:`BatchPlan` binds the buffers of a heterogeneous batch once, and
 :meth:`BatchPlan.run` renders every view, forms the L1/L2 image-loss gradient
-in registers and runs the checkpointed adjoint in one persistent HIP launch.
+in registers and runs the checkpointed adjoint in one persistent HIP launch
+(volume gradients of rays far apart: a persistent and a scatter launch per group of tiles).
 
 A run allocates nothing and copies nothing from the host, so optimisation
 steps built from runs and :class:`Adam` steps can be captured into a HIP graph
@@ -174,15 +175,16 @@ class BatchPlan:
         return int(torch.cuda.current_stream(self.device).cuda_stream)
 
     def run(self, zero_gradients: bool = True) -> None:
-        """Render every view, form the loss gradient and accumulate the adjoints (one persistent launch)."""
+        """Render every view, form the loss gradient and accumulate the adjoints."""
         self._h.run(ZERO_GRADIENTS if zero_gradients else 0, self._stream())
 
     def zero_gradients(self) -> None:
         self._h.zero_gradients(self._stream())
 
     def kernel_ms(self, zero_gradients: bool = True) -> float:
-        """One run with HIP events around the persistent kernel alone (on the current stream);
-        waits for it and returns that kernel's duration in milliseconds."""
+        """One run with HIP events around the persistent kernel (on the current stream; with
+        :attr:`volume_passes` 2 around every group's persistent and scatter kernels), without the clearing
+        and adding kernels; waits for it and returns the duration in milliseconds."""
         return float(self._h.time_kernel(ZERO_GRADIENTS if zero_gradients else 0, self._stream()))
 
     def freeze(self) -> None:

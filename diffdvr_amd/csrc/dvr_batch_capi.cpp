@@ -1,8 +1,9 @@
 // C-ABI of the batched persistent launch (plans), its autotuner and the
 // multi-block Adam step.  A plan validates the batch once, lays out the tile
-// queues and uploads the descriptor tables; a run is two kernel launches
-// (clear + persistent render) with no allocation, copy or memset, so that
-// optimisation steps can be captured into HIP graphs.
+// queues and uploads the descriptor tables; a run is kernel launches alone
+// (clear, persistent render, the additions of bricks and sums; two passes of volume
+// gradients: render and scatter per group of tiles) with no allocation, copy or
+// memset, so that optimisation steps can be captured into HIP graphs.
 #include <hip/hip_runtime.h>
 
 #include <sys/stat.h>
@@ -340,7 +341,8 @@ struct dvr_batch_plan {
         check_hip(dvr::launch_zero_segments(dSegsAll, n, mx, s), "zero launch");
     }
 
-    // evBegin / evEnd (optional) are recorded around the persistent kernel alone
+    // evBegin / evEnd (optional) are recorded around the persistent kernel, with two passes around every group's
+    // persistent and scatter kernels
     void run(int flags, hipStream_t s, hipEvent_t evBegin = nullptr, hipEvent_t evEnd = nullptr) const
     {
         zero((flags & DVR_BATCH_ZERO_GRADIENTS) != 0, s);

@@ -29,11 +29,10 @@ namespace dvr {
 
 // Occupancy cap of the tiled kernels.  A workgroup asks for at least
 // kLdsPerCu / (wgPerCu + 1) + 512 bytes of dynamic LDS, so no more than
-// wgPerCu of them share a CU.  The gather-bound instances run at two 4-wave
+// wgPerCu of them share a CU.  The gather-bound adjoints run at eight one-wave
 // workgroups per CU: more rays in flight evict each other's cells from the
-// 32 KB L1 faster than they hide latency (C2, 8 views 256x256 over 128^3:
-// forward with checkpoints 0.93 -> 0.59 ms, checkpointed adjoint
-// 0.72 -> 0.65 ms against the register-limited occupancy; volume gradients
+// 32 KB L1 faster than they hide latency (TF gradients, 8 views of 256x256 over
+// 128^3: 0.72 -> 0.65 ms against the register-limited occupancy; volume gradients
 // of 256^3 -9 %).  The Gaussian TF evaluates every component per sample and
 // is arithmetic-bound: it keeps the register-limited occupancy (the cap cost
 // it 3 %).
@@ -87,7 +86,8 @@ hipError_t launch_adam(const AdamSeg* dSegs, int nSegs, long long maxN, long lon
 
 // dvr_kernels_batched.hip: launch the batched persistent kernel (occ == NULL)
 // or report resident workgroups per CU of that instance.  gm: 0 forward only,
-// 1 TF, 3 volume (+TF), 7 volume + TF + camera.
+// 1 TF, 5 camera (+TF); volume gradients in one pass 3, 7 with the camera's, in two
+// passes 9 and 13 (the walk stores density adjoints).
 hipError_t launch_batched(const BatchParams& P, int filter, int tfm, int blend, int K, int gm, int grid, size_t lds,
                           hipStream_t s, int* occ);
 // adds every volume's bricked gradient scratch into its gradient (after launch_batched)

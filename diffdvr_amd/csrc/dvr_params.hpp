@@ -16,10 +16,12 @@ constexpr int kTfCopies = 4;      // copies of the LDS TF-gradient table, lane &
 // LDS gradient sums are doubles: on MI355X a ds_add_f32 takes 3 clocks a lane (193 a full wave instruction),
 // ds_add_f64 16 to 20 a wave instruction (addresses on distinct banks or random; lanes on one address take
 // 3 to 4 clocks each either way).
-// TF gradients: doubles between the copies (odd: the copies start in different banks), 0 = one table (copies
-// would take more than 16 KiB); 8-byte aligned offset behind the TF table; floats in all
+// The per-call one-pass walk keeps float sums: without a plan's bricks its slots count (see kAggLog2).
+
 // floats of a staged row of a TF of that mode with `cols` columns (see tf_lds_stride)
 constexpr int tf_lds_row_floats(int tfm, int cols) { return tfm >= 2 ? 8 : cols; }
+// TF gradients: doubles between the copies (odd: the copies start in different banks), 0 = one table (copies
+// would take more than 16 KiB); 8-byte aligned offset behind the TF table; floats in all
 constexpr int tf_grad_copy_stride(int RC) { return kTfCopies * (RC | 1) * 8 <= 16384 ? (RC | 1) : 0; }
 constexpr int tf_grad_offset(int tfFloats) { return (tfFloats + 1) & ~1; }
 constexpr int tf_grad_floats(int RC, bool priv, int threads, int stride)

@@ -394,7 +394,8 @@ dvr_status dvr_generate_rays_adjoint(const dvr_tensor* viewport, float fov_y_rad
  *
  * Many views (cameras) of many volumes and transfer functions, of uneven image
  * size and resolution, rendered forward, compared with a target image and
- * differentiated in ONE persistent launch.  The reference renders a batch
+ * differentiated in ONE persistent launch (volume gradients of rays far apart: one
+ * per group of tiles, each followed by a scatter kernel).  The reference renders a batch
  * only when all views share one image size and volume shape
  * (renderer/renderer.cpp:48-391): a caller with uneven views loops over
  * Renderer::renderForward / renderAdjoint per view
@@ -454,7 +455,8 @@ typedef struct dvr_batch {
 typedef struct dvr_batch_options {
     int32_t checkpoint_interval; /* K in {4,8,16,32,64}; 0 = 16 */
     int32_t wave_width;          /* rays along x of a wave's tile: 4, 8, 16 or 32 (tile 4x16 .. 32x2); 0 = 8 */
-    int32_t grid;                /* persistent workgroups; 0 = 2 per compute unit (within residency) */
+    int32_t grid;                /* persistent workgroups; 0 = 5 to 16 per compute unit by TF, gradients and
+                                    the distance of the rays (within residency) */
     int32_t reinterpolate;       /* 0: the forward march stores every sample's density and the reverse march
                                     reads it back (when the store fits in 2 GiB); 1: the reverse march
                                     re-interpolates (no store) */
@@ -466,12 +468,14 @@ typedef struct dvr_batch_plan dvr_batch_plan;
 
 dvr_status dvr_batch_plan_create(const dvr_batch* batch, const dvr_batch_options* options, dvr_batch_plan** plan);
 dvr_status dvr_batch_plan_destroy(dvr_batch_plan* plan);
-/* One persistent launch (plus one clearing kernel) on `stream`. */
+/* A clearing kernel, the persistent launch (see above) and small kernels that add its sums to the
+ * gradients and the loss, on `stream`. */
 dvr_status dvr_batch_plan_run(dvr_batch_plan* plan, int32_t flags, void* stream);
 /* Clear the gradient buffers and loss_out with a kernel (no memset). */
 dvr_status dvr_batch_plan_zero_gradients(dvr_batch_plan* plan, void* stream);
 /* Measurement: one run (as dvr_batch_plan_run) with HIP events recorded on `stream` around the
- * persistent kernel alone; waits for it and writes that kernel's duration.  No counterpart in the
+ * persistent kernel (two passes: around every group's persistent and scatter kernels), without the
+ * clearing and adding kernels; waits for it and writes the duration.  No counterpart in the
  * reference (its GPUTimer, bindings/bindings.cpp:99-129, times whatever the caller brackets). */
 dvr_status dvr_batch_plan_time_kernel(dvr_batch_plan* plan, int32_t flags, void* stream, float* kernel_ms);
 /* Freeze the plan's layout: from now on set_options may only repeat the current options and
