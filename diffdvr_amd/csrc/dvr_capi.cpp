@@ -686,14 +686,22 @@ private:
     }
 
     // The walk's corner registers and chunk table already sum most of a brick where many close rays take many
-    // samples of each cell; the second pass adds every sample.  one pass / two, us: quarter-voxel steps, 4 x 512 x 512
-    // rays of 64^3 1219 / 1386, 512 x 512 of 32^3 487 / 575, of 48^3 1122 / 739; half-voxel steps, 1024 x 1024 rays of
-    // 128^3 3014 / 3205, of 96^3 2267 / 2654, 4 x 512 x 512 of 64^3 980 / 808; whole steps, 1024 x 1024 of 64^3 1592 / 1156.
+    // samples of each cell; the second pass adds every sample.  One pass gains with the tiles and the samples of a
+    // ray and with their closeness; position gradients (two waves a SIMD) and gradients of textures (their table
+    // beside the chunk table) cost it more than the second pass.  Tiles x samples per axis / (step x pixel) decides:
+    // over 1370 launches of 4096 to 98304 tiles the choice is 2.3 % off the better scheme on average, 1.6 times at
+    // most (either wins by up to 4 times; views along and across the rows differ by 1.7).  One pass / two, us, identity TF,
+    // quarter-voxel steps, 512 x 512 rays: eight views of 64^3 1945 / 4324, of 128^3 4029 / 9803, of 32^3 1064 / 1965;
+    // four of 48^3 1409 / 1209; half-voxel steps, sixteen of 48^3 3390 / 2903.
     bool dense_rays() const
     {
         const float step = dvr::step_voxels(c_.P), spacing = step * dvr::pixel_voxels(c_.P);
-        if (step > 0.75f || tiles_ < 4096) return false;
-        return spacing <= (tiles_ / c_.B >= 16384 ? 0.065f : (tiles_ >= 8192 ? 0.035f : 0.02f));
+        if (tiles_ < 4096 || step > 0.75f || spacing > 0.13f) return false;
+        const bool position = A_.ars || A_.ard || A_.ast;
+        const bool table = A_.atf && (c_.tfm == 1 || (c_.tfm == 3 && position));
+        const float samples = float(c_.X + c_.Y + c_.Z) / (3.0f * step);
+        const float least = position && table ? 2.3e8f : (position || table ? 1.4e8f : 6.3e7f);
+        return float(std::min(tiles_, 98304)) * samples > least * spacing;
     }
 
     const Checked& c_;
