@@ -64,6 +64,7 @@ int wave_shift_of(int ww)
 constexpr long long kMaxAdjointStore = 8LL << 30;
 constexpr int kMaxGroups = 64;
 constexpr double kMaxRayDensity = 5.5;
+constexpr double kMaxCloseWork = 2.5e8, kMaxCloseWorkCameras = 6e8;
 
 int tf_cols(int tfm)
 {
@@ -93,6 +94,7 @@ struct dvr_batch_plan {
     bool farRays = false;   // most samples: at most 1.5 rays per voxel face of a volume of at least 8 M voxels
     bool sparseRays = false;  // most samples: at most 2 rays per voxel face of a volume of at least 4 M voxels
     double rayDensity = 0;  // rays per voxel face of a view, averaged over the samples of the volume gradients
+    double closeWork = 0;   // tiles x samples per axis / (step x pixel in voxels) of views with volume gradients
     double maxSamples = 0;  // upper bound of samples per ray over the views
     // layout
     int K = 16, waveWidth = 8, gridReq = 0, grid = 0, nTiles = 0, cap = 1;
@@ -198,7 +200,12 @@ struct dvr_batch_plan {
         // 5.9 / 4.0 (256^3) and 4.8 / 4.3 (128^3, quarter-voxel steps), 7 rays on average over 284 views
         // of 16 volumes 83.5 / 112, 16 rays 5.7 / 11.0 (256^3) and 1.9 / 1.9 (128^3).  Small plans alike:
         // 0.17 / 0.08 (four tiles, 14^3), 0.80 / 0.28 (1024 tiles, 32^3).
-        const bool two = (gm & 2) && volGrad && rayDensity <= kMaxRayDensity;
+        // Below that density short steps of many rays decide: the second pass adds every sample, the walk what
+        // leaves a cell.  Two passes' time to one pass's at four rays a face, linear TFs, by closeWork:
+        // 3.4e7 0.59, 1.3e8 1.01 (32 views of 128^3, quarter steps), 2.7e8 1.67 (8 of 256^3), 2.1e9 2.72 (16, eighth
+        // steps); with camera gradients 0.66, 0.73, 1.13, 1.66, and 1.11 at 1.1e9.
+        const bool two = (gm & 2) && volGrad && rayDensity <= kMaxRayDensity &&
+                         closeWork <= ((gm & 4) ? kMaxCloseWorkCameras : kMaxCloseWork);
         if (!(two && layout_scratch(true))) {
             release_adjoints();
             layout_scratch(false);
@@ -525,7 +532,7 @@ dvr_batch_plan* create(const dvr_batch* b, const dvr_batch_options* o)
         p->tfs.push_back(d);
     }
     long long totalPix = 0;
-    double volSamples = 0, volDensity = 0, allSamples = 0, farSamples = 0, sparseSamples = 0;
+    double volSamples = 0, volDensity = 0, volTiles = 0, closeWork = 0, allSamples = 0, farSamples = 0, sparseSamples = 0;
     std::vector<dvr::BView> vs;
     for (int i = 0; i < b->num_views; ++i) {
         const dvr_batch_view& v = b->views[i];
@@ -572,6 +579,10 @@ dvr_batch_plan* create(const dvr_batch* b, const dvr_batch_options* o)
         if (vol.adj) {
             volSamples += samples;
             volDensity += samples * density;
+            const double tiles = v.width * double(v.height) / 64.0, axis = rayMax / std::sqrt(3.0);
+            const double step = std::cbrt(voxels) / axis, spacing = step / std::sqrt(density);
+            volTiles += tiles;
+            if (step <= 0.75 && spacing <= 0.13) closeWork += tiles * axis / spacing;
         }
         vs.push_back(d);
     }
@@ -588,6 +599,8 @@ dvr_batch_plan* create(const dvr_batch* b, const dvr_batch_options* o)
     p->farRays = farSamples > 0.5 * allSamples;
     p->sparseRays = sparseSamples > 0.5 * allSamples;
     p->rayDensity = volSamples > 0 ? volDensity / volSamples : 0.0;
+    // more tiles than 98304 change nothing any more
+    p->closeWork = closeWork * std::min(1.0, 98304.0 / std::max(volTiles, 1.0));
     if (b->forward_only) p->gm = 0;
     else {
         if (!anyTfGrad && !anyVolGrad && !anyCamGrad && !p->lossOut)
