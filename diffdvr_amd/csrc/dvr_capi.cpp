@@ -692,11 +692,12 @@ private:
     // over 1370 launches of 4096 to 98304 tiles the choice is 2.3 % off the better scheme on average, 1.6 times at
     // most (either wins by up to 4 times; views along and across the rows differ by 1.7).  One pass / two, us, identity TF,
     // quarter-voxel steps, 512 x 512 rays: eight views of 64^3 1945 / 4324, of 128^3 4029 / 9803, of 32^3 1064 / 1965;
-    // four of 48^3 1409 / 1209; half-voxel steps, sixteen of 48^3 3390 / 2903.
+    // four of 48^3 1409 / 1209; half-voxel steps, sixteen of 48^3 3390 / 2903, twelve of 256^3 11083 / 14023,
+    // six 7488 / 6827; twice that distance apart two passes are faster at every count measured.
     bool dense_rays() const
     {
         const float step = dvr::step_voxels(c_.P), spacing = step * dvr::pixel_voxels(c_.P);
-        if (tiles_ < 4096 || step > 0.75f || spacing > 0.13f) return false;
+        if (tiles_ < 4096 || step > 0.75f || spacing > 0.26f) return false;
         const bool position = A_.ars || A_.ard || A_.ast;
         const bool table = A_.atf && (c_.tfm == 1 || (c_.tfm == 3 && position));
         const float samples = float(c_.X + c_.Y + c_.Z) / (3.0f * step);
